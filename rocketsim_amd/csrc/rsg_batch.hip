@@ -65,6 +65,11 @@ struct DeviceMesh {
     QSubtree* subtrees = nullptr;
     TriInfo* tri_info = nullptr;
     uint32_t* occ = nullptr;
+    struct Lists {
+        MeshLeaf* leaves = nullptr;
+        uint32_t* items = nullptr;
+        uint32_t* offsets = nullptr;
+    } box_lists, ray_lists;
 };
 // An arena's static geometry (the Soccar arena, the Hoops arena), shared
 // read-only by every batch of the process (RocketSim keeps its arena meshes
@@ -89,6 +94,17 @@ int upload_array(T** dst, const std::vector<T>& src) {
     HIP_OK(hipMalloc((void**)dst, bytes));
     HIP_OK(hipMemcpy(*dst, src.data(), bytes, hipMemcpyHostToDevice));
     return 0;
+}
+
+int upload_lists(DeviceMesh::Lists& d, const HostMesh::Lists& l) {
+    if (l.items.empty()) return 0;  // no lists: the view's pointers stay null
+    return upload_array(&d.leaves, l.leaves) || upload_array(&d.items, l.items) || upload_array(&d.offsets, l.offsets)
+               ? -1 : 0;
+}
+void set_lists(LeafGrid& g, const DeviceMesh::Lists& d) {
+    g.leaves = d.leaves;
+    g.items = d.items;
+    g.offsets = d.offsets;
 }
 
 }  // namespace
@@ -1606,6 +1622,9 @@ int rsg_init_arena_meshes(int mode, const void* const* cmf_data, const uint64_t*
     for (DeviceMesh& m : g_mesh.meshes) {
         (void)hipFree(m.verts); (void)hipFree(m.tris); (void)hipFree(m.nodes);
         (void)hipFree(m.subtrees); (void)hipFree(m.tri_info); (void)hipFree(m.occ);
+        for (DeviceMesh::Lists* l : {&m.box_lists, &m.ray_lists}) {
+            (void)hipFree(l->leaves); (void)hipFree(l->items); (void)hipFree(l->offsets);
+        }
     }
     g_mesh.meshes.assign(H.meshes.size(), DeviceMesh());
     g_mesh.host = std::move(H);
@@ -1615,7 +1634,8 @@ int rsg_init_arena_meshes(int mode, const void* const* cmf_data, const uint64_t*
         DeviceMesh& D = g_mesh.meshes[i];
         if (upload_array(&D.verts, M.verts) || upload_array(&D.tris, M.tris) || upload_array(&D.nodes, M.nodes) ||
             upload_array(&D.subtrees, M.subtrees) || upload_array(&D.tri_info, M.tri_info) ||
-            upload_array(&D.occ, M.occ))
+            upload_array(&D.occ, M.occ) || upload_lists(D.box_lists, M.box_lists) ||
+            upload_lists(D.ray_lists, M.ray_lists))
             return -1;
         MeshView v = M.view();
         v.verts = D.verts;
@@ -1624,6 +1644,8 @@ int rsg_init_arena_meshes(int mode, const void* const* cmf_data, const uint64_t*
         v.subtrees = D.subtrees;
         v.tri_info = D.tri_info;
         v.occ = D.occ;
+        set_lists(v.box_grid, D.box_lists);
+        set_lists(v.ray_grid, D.ray_lists);
         views.push_back(v);
     }
     if (upload_array(&g_mesh.views, views) || upload_array(&g_mesh.cell_statics, g_mesh.host.cell_statics)) return -1;

@@ -32,6 +32,19 @@ struct HostMesh {
     V3 aabb_min, aabb_max;
     std::vector<uint32_t> occ;          // MeshView::occ bitmask
     int occ_dims[3] = {0, 0, 0};
+    // MeshView::box_grid and ray_grid
+    struct Lists {
+        std::vector<MeshLeaf> leaves;
+        std::vector<uint32_t> items, offsets;
+        LeafGrid grid{};   // dimensions; the pointers are the view's
+        LeafGrid view() const {
+            LeafGrid g = grid;
+            g.leaves = leaves.data();
+            g.items = items.empty() ? nullptr : items.data();
+            g.offsets = offsets.data();
+            return g;
+        }
+    } box_lists, ray_lists;
 
     MeshView view() const {
         MeshView v{};
@@ -49,6 +62,8 @@ struct HostMesh {
         v.occ_nx = occ_dims[0]; v.occ_ny = occ_dims[1]; v.occ_nz = occ_dims[2];
         v.occ_origin = bvh_min;
         v.occ_inv_cell = 1.f / MESH_OCC_CELL;
+        v.box_grid = box_lists.view();
+        v.ray_grid = ray_lists.view();
         return v;
     }
 };
@@ -485,6 +500,85 @@ inline void build_occupancy(HostMesh& M) {
     }
 }
 
+// One query kind's leaf lists (LeafGrid).  `order` holds the leaf nodes as the
+// tree walk reaches them.  A mesh whose lists would take more than
+// LEAF_LIST_MAX_ITEMS entries gets none: its queries walk the tree.
+constexpr size_t LEAF_LIST_MAX_ITEMS = (size_t)1 << 25;
+inline void build_leaf_lists(HostMesh& M, const std::vector<int32_t>& order, float cell, float reach, float grow,
+                             float grow_rel, HostMesh::Lists& L) {
+    L = HostMesh::Lists();
+    L.grid.reach = reach;
+    L.grid.inv_cell = 1.f / cell;
+    L.grid.origin = M.aabb_min - v3(1.f, 1.f, 1.f);
+    const V3 ext = M.aabb_max + v3(1.f, 1.f, 1.f) - L.grid.origin;
+    if (!(ext.x < 1e5f && ext.y < 1e5f && ext.z < 1e5f)) return;
+    const int dims[3] = {(int)(ext.x / cell) + 1, (int)(ext.y / cell) + 1, (int)(ext.z / cell) + 1};
+    if ((double)dims[0] * dims[1] * dims[2] > (double)LEAF_LIST_MAX_ITEMS) return;
+    L.grid.nx = dims[0]; L.grid.ny = dims[1]; L.grid.nz = dims[2];
+    for (int32_t node : order) {
+        const int32_t t = M.nodes[(size_t)node].esc_or_tri;
+        MeshLeaf l;
+        l.tri = t;
+        l.node = node;
+        V3 p[3];
+        for (int j = 0; j < 3; j++) {
+            const int vi = M.tris[(size_t)(3 * t + j)];
+            p[j] = v3(M.verts[(size_t)(3 * vi)], M.verts[(size_t)(3 * vi + 1)], M.verts[(size_t)(3 * vi + 2)]);
+        }
+        l.lo = v3(fminf(fminf(p[0].x, p[1].x), p[2].x), fminf(fminf(p[0].y, p[1].y), p[2].y),
+                  fminf(fminf(p[0].z, p[1].z), p[2].z));
+        l.hi = v3(fmaxf(fmaxf(p[0].x, p[1].x), p[2].x), fmaxf(fmaxf(p[0].y, p[1].y), p[2].y),
+                  fmaxf(fmaxf(p[0].z, p[1].z), p[2].z));
+        const V3 e = l.hi - l.lo;
+        const float g = grow + grow_rel * fmaxf(fmaxf(e.x, e.y), e.z);
+        l.lo = l.lo - v3(g, g, g);
+        l.hi = l.hi + v3(g, g, g);
+        L.leaves.push_back(l);
+    }
+    // cells whose extended box [cell, cell + 1 + reach] (plus a rounding
+    // slack) the leaf touches
+    const float slack = MESH_OCC_SLACK;
+    const size_t n_cells = (size_t)dims[0] * dims[1] * dims[2];
+    auto each_cell = [&](const MeshLeaf& l, auto&& f) {
+        const V3 a = (l.lo - v3(reach + slack, reach + slack, reach + slack) - L.grid.origin) * L.grid.inv_cell;
+        const V3 b = (l.hi + v3(slack, slack, slack) - L.grid.origin) * L.grid.inv_cell;
+        const int i0 = std::max(0, (int)std::floor(a.x)), j0 = std::max(0, (int)std::floor(a.y)),
+                  k0 = std::max(0, (int)std::floor(a.z));
+        const int i1 = std::min(dims[0] - 1, (int)std::floor(b.x)), j1 = std::min(dims[1] - 1, (int)std::floor(b.y)),
+                  k1 = std::min(dims[2] - 1, (int)std::floor(b.z));
+        for (int i = i0; i <= i1; i++)
+            for (int j = j0; j <= j1; j++)
+                for (int k = k0; k <= k1; k++) f(((size_t)i * dims[1] + j) * dims[2] + k);
+    };
+    std::vector<uint32_t> count(n_cells + 1, 0u);
+    size_t total = 0;
+    for (const MeshLeaf& l : L.leaves) {
+        each_cell(l, [&](size_t c) { count[c + 1]++; total++; });
+        if (total > LEAF_LIST_MAX_ITEMS) return;
+    }
+    for (size_t c = 0; c < n_cells; c++) count[c + 1] += count[c];
+    L.offsets = count;
+    L.items.resize(total + 1, 0u);  // never empty, so the view is not null
+    std::vector<uint32_t> at(count.begin(), count.end() - 1);
+    for (size_t i = 0; i < L.leaves.size(); i++)
+        each_cell(L.leaves[i], [&](size_t c) { L.items[at[c]++] = (uint32_t)i; });
+}
+
+// Box lists: reach of the ball's and the cars' boxes, in the order of the box
+// walk (subtree by subtree).  Ray lists: reach of a suspension ray, in node
+// order, with boxes grown by what ray_triangle accepts beyond a triangle's
+// edge (barycentric -1e-4 of its size) and rounding.
+inline void build_leaf_grids(HostMesh& M) {
+    std::vector<int32_t> boxes, rays;
+    for (const QSubtree& st : M.subtrees)
+        for (int c = st.root; c < st.root + st.size; c++)
+            if (M.nodes[(size_t)c].esc_or_tri >= 0) boxes.push_back(c);
+    for (size_t c = 0; c < M.nodes.size(); c++)
+        if (M.nodes[c].esc_or_tri >= 0) rays.push_back((int32_t)c);
+    if (boxes.size() == rays.size()) build_leaf_lists(M, boxes, LEAF_BOX_CELL, LEAF_BOX_REACH, 0.f, 0.f, M.box_lists);
+    build_leaf_lists(M, rays, LEAF_RAY_CELL, LEAF_RAY_REACH, MESH_OCC_SLACK, 1e-3f, M.ray_lists);
+}
+
 // Full preparation of one collision mesh from .cmf bytes (one entry of
 // RocketSim::InitFromMem's list, src/RocketSim.cpp:129-155: the mesh, its
 // BVH and its triangle info map).
@@ -495,6 +589,7 @@ inline std::string build_host_mesh(const void* data, uint64_t size, HostMesh& M)
     b.build();
     build_tri_info(M);
     build_occupancy(M);
+    build_leaf_grids(M);
     return "";
 }
 

@@ -24,6 +24,7 @@ struct ArenaLocal {
     uint32_t resets;
     uint32_t status;
     SolverInfo si;
+    float ball_damping;      // (1 - ballDrag)^dt, btRigidBody::applyDamping's factor
     // broadphase registration of the dynamic proxies (0 = ball, 1 + i = car i)
     int bp_cell[1 + MAX_CARS];
     uint32_t bp_seq[1 + MAX_CARS];
@@ -38,6 +39,11 @@ struct ArenaLocal {
     uint32_t ev_seq;
     uint32_t arena_id;
     Car cars[MAX_CARS];
+#if !defined(__HIPCC__)
+    // The cars' physics values where the batch has no table of them (host
+    // test builds; the library's batches have one).
+    CarPhys own_phys[MAX_CARS];
+#endif
 };
 
 // Appends an event to the batch's ring (dropped when the ring is full; the

@@ -32,6 +32,7 @@
 #include "../../include/rsg.h"
 #include "rsg_mesh_build.h"
 #include "rsg_tick.h"
+#include "rsg_team.h"
 #include "rsg_api_convert.h"
 #include "rsg_adjoint.h"
 #include "rsg_ball_pred.h"
@@ -82,6 +83,7 @@ struct DeviceArena {
     MeshView* views = nullptr;      // device copies of the meshes' views
     uint32_t* cell_statics = nullptr;
     ArenaGeom geom{};
+    ArenaGeom* dev_geom = nullptr;  // a copy of it in device memory
 };
 DeviceArena g_arenas[2];  // by arena_kind(mode)
 std::mutex g_mesh_mutex;
@@ -144,6 +146,7 @@ struct rsg_batch {
     std::vector<rsg_mutator_config> h_mut;  // per-arena MutatorConfig (the kernels only read it)
     std::vector<rsg_car_config> h_cfgs;     // car config table: the presets, then other configs
     rsg_car_config* d_cfgs = nullptr;
+    CarPhys* d_phys = nullptr;              // make_car_phys of each entry
     std::vector<rsg_boost_pad_config> h_custom_pads;  // ArenaConfig::customBoostPads
     rsg_boost_pad_config* d_custom_pads = nullptr;
     bool host_dirty = false;  // host mirror newer than device
@@ -175,6 +178,7 @@ BatchDev host_view(rsg_batch* b) {
     h.arena = b->h_arena.data();
     h.mut = b->h_mut.data();
     h.cfgs = b->h_cfgs.data();
+    h.phys = nullptr;
     h.custom_pads = b->h_custom_pads.empty() ? nullptr : b->h_custom_pads.data();
     return h;
 }
@@ -324,6 +328,8 @@ rsg_batch* rsg_batch_create(const rsg_batch_desc* desc) {
     b->h_arena.assign(arena_words(b), 0);
     b->h_mut.assign((size_t)b->dev.n, desc->mutators ? *desc->mutators : mutator_defaults(b->dev.mode));
     hipError_t e = hipSuccess;
+    std::vector<CarPhys> phys;
+    for (const rsg_car_config& c : b->h_cfgs) phys.push_back(make_car_phys(c));
     rsg_mutator_config* dmut = nullptr;
     if ((e = hipMalloc(&b->dev.car, car_words(b) * 4)) != hipSuccess ||
         (e = hipMalloc(&b->dev.ball, ball_words(b) * 4)) != hipSuccess ||
@@ -334,6 +340,8 @@ rsg_batch* rsg_batch_create(const rsg_batch_desc* desc) {
         (e = hipMalloc(&b->d_cfgs, b->h_cfgs.size() * sizeof(rsg_car_config))) != hipSuccess ||
         (e = hipMemcpy(b->d_cfgs, b->h_cfgs.data(), b->h_cfgs.size() * sizeof(rsg_car_config),
                        hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMalloc(&b->d_phys, phys.size() * sizeof(CarPhys))) != hipSuccess ||
+        (e = hipMemcpy(b->d_phys, phys.data(), phys.size() * sizeof(CarPhys), hipMemcpyHostToDevice)) != hipSuccess ||
         (!b->h_custom_pads.empty() &&
          ((e = hipMalloc(&b->d_custom_pads, b->h_custom_pads.size() * sizeof(rsg_boost_pad_config))) != hipSuccess ||
           (e = hipMemcpy(b->d_custom_pads, b->h_custom_pads.data(),
@@ -345,6 +353,7 @@ rsg_batch* rsg_batch_create(const rsg_batch_desc* desc) {
     }
     b->dev.mut = dmut;
     b->dev.cfgs = b->d_cfgs;
+    b->dev.phys = b->d_phys;
     b->dev.custom_pads = b->d_custom_pads;
     b->dev.n_custom_pads = (int)b->h_custom_pads.size();
     // Host-side initial state: cars with config, ball at rest, pads active.
@@ -368,6 +377,7 @@ void rsg_batch_destroy(rsg_batch* b) {
     if (b->dev.space) (void)hipFree(b->dev.space);
     if (b->dev.mut) (void)hipFree(const_cast<rsg_mutator_config*>(b->dev.mut));
     if (b->d_cfgs) (void)hipFree(b->d_cfgs);
+    if (b->d_phys) (void)hipFree(b->d_phys);
     if (b->d_custom_pads) (void)hipFree(b->d_custom_pads);
     if (b->status_partials) (void)hipFree(b->status_partials);
     if (b->dev.ev_buf) (void)hipFree(b->dev.ev_buf);
@@ -419,10 +429,10 @@ int lds_max_per_block(const rsg_batch* b) {
     return m < 1 ? 0 : (m > 64 ? 64 : m);
 }
 
-// Cooperative kernel: 4 lanes per car slot, arena + ray results + flag in LDS.
+// Cooperative kernel: 4 lanes per car slot, the arena and its team's block in LDS.
 int coop_lanes(const rsg_batch* b) { return 4 * b->dev.max_cars; }
 int coop_stride(const rsg_batch* b) {
-    size_t bytes = (size_t)lds_stride(b) + (size_t)coop_lanes(b) * sizeof(RayHit) + 2 * sizeof(int);
+    size_t bytes = (size_t)lds_stride(b) + team_local_bytes(b->dev.max_cars);
     return (int)((bytes + 15) & ~(size_t)15);
 }
 int coop_max_per_block(const rsg_batch* b) {
@@ -438,11 +448,12 @@ struct Launch {
 };
 
 // Kernel and arenas per workgroup.  The cooperative kernel is the fastest
-// wherever its per-arena block fits (2v2 at 4096 arenas: 0.48 ms per tick
-// against 0.62 for the LDS kernel; at 16384: 0.98 against 1.09 and 1.16 for
-// the plain kernel), so it is the default; arenas are spread one per
-// workgroup until every SIMD has a wave, then packed up to the most a
-// workgroup holds.
+// wherever its per-arena block fits (ms per tick, cooperative / LDS / plain:
+// one 1v1 arena 0.030 / 0.100 / 0.128, 2v2 x 4096 0.303 / 0.609 / 0.771,
+// 2v2 x 16384 0.515 / 0.953 / 1.080, 32768 arenas of 1v1 to 3v3 0.81 / 2.07 /
+// 1.48), so it is the default; arenas are spread one per workgroup until every
+// SIMD has a wave, then packed up to the most a workgroup holds (2v2 x 16384
+// at 1, 2, 3 and 4 arenas a workgroup: 0.723, 0.583, 0.533 and 0.515).
 Launch choose_launch(const rsg_batch* b) {
     const int simds = device_simds();
     int spread = (b->dev.n + simds - 1) / simds;  // arenas per wave at one wave per SIMD
@@ -497,13 +508,15 @@ int launch_step(const rsg_batch* b, const BatchDev& dev, const Launch& L, int ti
     int block = L.per_block;
     int grid = (dev.n + block - 1) / block;
     ArenaGeom mv{};
+    const ArenaGeom* dev_geom = nullptr;
     if (mode_has_arena(dev.mode)) {
         const DeviceArena& ga = g_arenas[arena_kind(dev.mode)];
         if (!ga.ready) return fail("rsg_batch_step: no arena mesh (call rsg_init_mesh first)");
         mv = ga.geom;
+        dev_geom = ga.dev_geom;
     }
     if (L.kernel == RSG_KERNEL_COOP)
-        HIP_OK(launch_step_coop(dev, mv, ticks, grid, block, coop_stride(b), lds_stride(b), coop_lanes(b), s));
+        HIP_OK(launch_step_coop(dev, dev_geom, ticks, grid, block, coop_stride(b), lds_stride(b), coop_lanes(b), s));
     else if (L.kernel == RSG_KERNEL_LDS)
         HIP_OK(launch_step_lds(dev, mv, ticks, grid, block, lds_stride(b), s));
     else
@@ -1653,6 +1666,7 @@ int rsg_init_arena_meshes(int mode, const void* const* cmf_data, const uint64_t*
     g.meshes = g_mesh.views;
     g.n_meshes = (int)views.size();
     g.cell_statics = g_mesh.cell_statics;
+    if (upload_array(&g_mesh.dev_geom, std::vector<ArenaGeom>{g})) return -1;
     g_mesh.geom = g;
     g_mesh.ready = true;
     return 0;

@@ -156,7 +156,7 @@ RSG_FN void spread_by_angle(int n, const float pts[16], int keep, int first, int
 // Box 0 (transform x0, half extents h0) against box 1.  Contacts are
 // reported as the manifold receives them: normal on box 1, point on box 1,
 // signed distance.
-RSG_FN void box_box(const Xf& x0, V3 h0, const Xf& x1, V3 h1, BoxBoxContacts& out) {
+RSG_COLD_FN void box_box(const Xf& x0, V3 h0, const Xf& x1, V3 h1, BoxBoxContacts& out) {
     out.n = 0;
     const BoxFrame b0 = box_frame(x0, h0), b1 = box_frame(x1, h1);
     const V3 d = b1.c - b0.c;

@@ -127,7 +127,9 @@ struct StepSpace {
 static_assert(sizeof(StepSpace) <= 60 * 1024, "StepSpace must fit a lane's private memory");
 // The plain kernel's lane holds a StepSpace, an ArenaLocal and about 2 KB of
 // other private data within the device's 64 KiB per lane.
+#if defined(__HIPCC__)
 static_assert(sizeof(StepSpace) + sizeof(ArenaLocal) <= 62 * 1024, "the plain kernel's lane must fit 64 KiB");
+#endif
 
 // An arena's block of a batch's global work space: the world step's work
 // space and the record of a shared narrowphase.
@@ -135,6 +137,15 @@ struct ArenaSpace {
     StepSpace step;
     PairLog log;
 };
+
+// predictUnconstraintMotion (damping on every dynamic body; the ball's linear
+// damping is the arena's ballDrag, clamped to [0, 1] by
+// btRigidBody::setDamping).
+RSG_FN void world_ball_damping(ArenaLocal& A, float dt) {
+    Body& bb = A.ball.b;
+    (void)dt;
+    bb.vel *= A.ball_damping;  // the angular damping is 0: a factor of 1
+}
 
 struct World {
     ArenaLocal& A;
@@ -144,8 +155,6 @@ struct World {
     StepSpace* ws;  // null for worlds that only cast rays
 
     WorldTables* T;  // ws->wt
-    int ray_order[MAX_BODIES];  // dynamic proxies in cell-list order as of the start of the tick (wheel rays)
-    bool ray_order_ready;
     Manifold* mf;   // ws->mf
     // Narrowphase of one planned pair: where its callbacks' effects go (null:
     // applied at once) and the penetration work space (null: a query that
@@ -155,7 +164,7 @@ struct World {
     bool aborted;
 
     RSG_FN World(ArenaLocal& a, const ArenaGeom* g, bool s, StepSpace* w = nullptr)
-        : A(a), geo(g), soccar(s), mesh(nullptr), ws(w), T(w ? &w->wt : nullptr), ray_order_ready(false), mf(w ? w->mf : nullptr),
+        : A(a), geo(g), soccar(s), mesh(nullptr), ws(w), T(w ? &w->wt : nullptr), mf(w ? w->mf : nullptr),
           rec(nullptr), epa(w ? &w->epa : nullptr), aborted(false) {}
 
     // Whether the subsimplex ray cast against a convex of bounding radius
@@ -215,7 +224,7 @@ struct World {
 
     RSG_FN float threshold_of(int code) {
         if (code == 0) return make_ball_phys(A.ball.radius_uu, A.ball.mass).angular_motion_disc * CONTACT_BREAKING_THRESHOLD;
-        if (code > 0) return A.cars[code - 1].phys.angular_motion_disc * CONTACT_BREAKING_THRESHOLD;
+        if (code > 0) return A.cars[code - 1].phys->angular_motion_disc * CONTACT_BREAKING_THRESHOLD;
         return 1e30f;  // planes and the arena meshes have huge bounding spheres
     }
 
@@ -235,7 +244,7 @@ struct World {
             mn = pos - v3(r, r, r);
             mx = pos + v3(r, r, r);
         } else {
-            const CarPhys& cp = A.cars[code - 1].phys;
+            const CarPhys& cp = *A.cars[code - 1].phys;
             M3 ab = abs_m3(rot);
             V3 c = rot * cp.local_aabb_center + pos;
             V3 e = v3(dot(ab.r[0], cp.local_aabb_half), dot(ab.r[1], cp.local_aabb_half), dot(ab.r[2], cp.local_aabb_half));
@@ -247,7 +256,7 @@ struct World {
     // Child box AABB of a car (btBoxShape::getAabb at hull transform, no threshold).
     RSG_FN void car_child_aabb(int code, V3& mn, V3& mx) {
         Car& c = A.cars[code - 1];
-        const CarPhys& cp = c.phys;
+        const CarPhys& cp = *c.phys;
         Xf x = xf_mul(xf_from(c.b.pos, c.b.rot), xf_from(cp.box_offset, m3_identity()));
         V3 he = cp.box_implicit + v3(cp.box_margin, cp.box_margin, cp.box_margin);
         M3 ab = abs_m3(x.R);
@@ -302,37 +311,35 @@ struct World {
         }
         // then the dynamic proxies registered in the cell (cell-list order),
         // except the casting car (btCollisionWorld::RayResultCallback::needsCollision)
+        // that the ray may reach; few rays have any
         const int nb = num_bodies();
-        if (!ray_order_ready) {
-            // registration order does not change before the world step
-            for (int i = 0; i < nb; i++) ray_order[i] = i;
-            for (int i = 1; i < nb; i++) {
-                int v = ray_order[i], j = i - 1;
-                while (j >= 0 && A.bp_seq[ray_order[j]] > A.bp_seq[v]) { ray_order[j + 1] = ray_order[j]; j--; }
-                ray_order[j + 1] = v;
+        uint32_t near = 0;
+        for (int q = 0; q < nb; q++) {
+            if (q == self_body || !bp_cells_adjacent(A.bp_cell[q], c)) continue;
+            V3 center;
+            float radius;
+            if (q == 0) {
+                center = A.ball.b.pos;
+                radius = make_ball_phys(A.ball.radius_uu, A.ball.mass).radius;
+            } else {
+                const CarPhys& cp = *A.cars[q - 1].phys;
+                center = car_child_xf(q).t;
+                radius = len(cp.box_implicit + v3(cp.box_margin, cp.box_margin, cp.box_margin));
             }
-            ray_order_ready = true;
+            if (ray_may_hit(from, to, center, radius)) near |= 1u << q;
         }
-        for (int r = 0; r < nb; r++) {
-            int q = ray_order[r];
-            if (!bp_cells_adjacent(A.bp_cell[q], c)) continue;
+        while (near) {
+            int q = -1;  // the one registered first
+            for (int i = 0; i < nb; i++)
+                if ((near >> i & 1u) && (q < 0 || A.bp_seq[i] < A.bp_seq[q])) q = i;
+            near &= ~(1u << q);
             if (frac == 0.f) break;
-            if (q == self_body) continue;
+            const CShape shape = q == 0 ? shape_sphere(make_ball_phys(A.ball.radius_uu, A.ball.mass).radius) : car_box_shape(q);
+            const Xf x = q == 0 ? xf_from(A.ball.b.pos, A.ball.b.rot) : car_child_xf(q);
             float f;
             V3 nn;
-            if (q == 0) {
-                CShape sph = shape_sphere(make_ball_phys(A.ball.radius_uu, A.ball.mass).radius);
-                if (!ray_may_hit(from, to, A.ball.b.pos, sph.margin)) continue;
-                if (ray_convex(from, to, sph, xf_from(A.ball.b.pos, A.ball.b.rot), f, nn)) {
-                    if (len2(nn) > 0.0001f && f < frac) { frac = f; n = normalized(nn); hit_obj = q; }
-                }
-            } else {
-                CShape box = car_box_shape(q);
-                Xf cx = car_child_xf(q);
-                if (!ray_may_hit(from, to, cx.t, len(box.half + v3(box.margin, box.margin, box.margin)))) continue;
-                if (ray_convex(from, to, box, cx, f, nn)) {
-                    if (len2(nn) > 0.0001f && f < frac) { frac = f; n = normalized(nn); hit_obj = q; }
-                }
+            if (ray_convex(from, to, shape, x, f, nn)) {
+                if (len2(nn) > 0.0001f && f < frac) { frac = f; n = normalized(nn); hit_obj = q; }
             }
         }
         if (hit_obj != -100) {
@@ -534,7 +541,7 @@ struct World {
                             other.demo_timer = A.mut.respawn_delay;
                         } else {
                             bool ground = flag(other.flags, RSG_CF_ON_GROUND);
-                            float base = curve_eval(ground ? curve_bump_ground() : curve_bump_air(), speed_towards);
+                            float base = ground ? curve_eval(curve_bump_ground(), speed_towards) : curve_eval(curve_bump_air(), speed_towards);
                             V3 up = ground ? car_up(other) : v3(0, 0, 1);
                             V3 imp = vel_dir * base + up * curve_eval(curve_bump_upward(), speed_towards) *
                                                       A.mut.bump_force_scale;
@@ -586,7 +593,7 @@ struct World {
         const PlaneDef& pd = static_plane(*geo, s);
         Xf px = xf_from(pd.origin, m3_identity());
         Car& c = A.cars[code - 1];
-        const CarPhys& cp = c.phys;
+        const CarPhys& cp = *c.phys;
         Xf cx = xf_mul(xf_from(c.b.pos, c.b.rot), xf_from(cp.box_offset, m3_identity()));
         Xf plane_in_convex = xf_mul(xf_inverse(cx), px);
         Xf convex_in_plane = xf_mul(xf_inverse(px), cx);
@@ -607,11 +614,15 @@ struct World {
     // Sphere vs one mesh triangle (SphereTriangleDetector::collide, with the
     // closest-point-on-triangle capsule test RocketSim uses).
     RSG_FN void sphere_triangle(int mi, const V3 v[3], int tri) {
-        Body& b = A.ball.b;
-        V3 center = b.pos;  // triangle space = world (mesh at identity)
-        float radius = make_ball_phys(A.ball.radius_uu, A.ball.mass).radius;
-        float thr = mf[mi].threshold + 0.f;
-        float rwt = radius + thr;
+        V3 n, pt;
+        float depth;
+        if (sphere_triangle_contact(A.ball.b.pos, make_ball_phys(A.ball.radius_uu, A.ball.mass).radius, mf[mi].threshold, v,
+                                    n, pt, depth))
+            add_contact(mi, n, pt, depth, tri);
+    }
+    RSG_FN static bool sphere_triangle_contact(V3 center, float radius, float thr, const V3 v[3], V3& rn, V3& pt,
+                                               float& depth) {
+        float rwt = radius + thr;  // triangle space = world (mesh at identity)
         V3 normal = cross(v[1] - v[0], v[2] - v[0]);
         float l2 = len2(normal);
         bool has = false;
@@ -634,12 +645,10 @@ struct World {
                 }
             }
         }
-        if (!has) return;
+        if (!has) return false;
         V3 c2c = center - cpt;
         float d2 = len2(c2c);
-        if (!(d2 < rwt * rwt)) return;
-        V3 rn, pt;
-        float depth;
+        if (!(d2 < rwt * rwt)) return false;
         if (d2 > FLT_EPS) {
             float dist = sqrtf(d2);
             rn = normalized(c2c);
@@ -650,7 +659,7 @@ struct World {
             pt = cpt;
             depth = -radius;
         }
-        add_contact(mi, rn, pt, depth, tri);
+        return true;
     }
 
     // SphereTriangleDetector::pointInTriangle (RocketSim variant)
@@ -688,11 +697,11 @@ struct World {
 
     RSG_FN Xf car_child_xf(int code) {
         Car& c = A.cars[code - 1];
-        const CarPhys& cp = c.phys;
+        const CarPhys& cp = *c.phys;
         return xf_mul(xf_from(c.b.pos, c.b.rot), xf_from(cp.box_offset, m3_identity()));
     }
     RSG_FN CShape car_box_shape(int code) {
-        const CarPhys& cp = A.cars[code - 1].phys;
+        const CarPhys& cp = *A.cars[code - 1].phys;
         return shape_box(cp.box_implicit, cp.box_margin);
     }
 
@@ -700,7 +709,7 @@ struct World {
     // per-triangle early out, then btConvexConvexAlgorithm (GJK) per triangle.
     RSG_FN void car_vs_mesh(int mi, int code) {
         Xf cx = car_child_xf(code);
-        const CarPhys& cp = A.cars[code - 1].phys;
+        const CarPhys& cp = *A.cars[code - 1].phys;
         V3 he = cp.box_implicit + v3(cp.box_margin, cp.box_margin, cp.box_margin);
         M3 ab = abs_m3(cx.R);
         V3 e = v3(dot(ab.r[0], he), dot(ab.r[1], he), dot(ab.r[2], he));
@@ -762,8 +771,8 @@ struct World {
     // box0 = the car of manifold body0.
     RSG_FN void car_vs_car(int mi, int c0, int c1) {
         Xf x0 = car_child_xf(c0), x1 = car_child_xf(c1);
-        const CarPhys& p0 = A.cars[c0 - 1].phys;
-        const CarPhys& p1 = A.cars[c1 - 1].phys;
+        const CarPhys& p0 = *A.cars[c0 - 1].phys;
+        const CarPhys& p1 = *A.cars[c1 - 1].phys;
         V3 h0 = p0.box_implicit + v3(p0.box_margin, p0.box_margin, p0.box_margin);
         V3 h1 = p1.box_implicit + v3(p1.box_margin, p1.box_margin, p1.box_margin);
         BoxBoxContacts bc;
@@ -839,21 +848,13 @@ struct World {
             Body& b = *body_ptr(i);
             if (b.active) b.force += b.grav;
         }
-        // predictUnconstraintMotion (damping on every dynamic body; the
-        // ball's linear damping is the arena's ballDrag, clamped to [0, 1]
-        // by btRigidBody::setDamping)
-        {
-            Body& bb = A.ball.b;
-            const float drag = fminf(fmaxf(A.mut.ball_drag, 0.f), 1.f);
-            bb.vel *= powf(1.f - drag, dt);
-            bb.ang *= powf(1.f - 0.f, dt);
-        }
+        world_ball_damping(A, dt);
     }
 
     // Proxy AABB of body i: its shape at the current and the predicted pose,
     // merged, +- the contact threshold (btCollisionWorld::updateSingleAabb
     // over predictIntegratedTransform).
-    RSG_FN void body_aabb(int i, float dt) {
+    RSG_FN void proxy_aabb(int i, float dt, V3& out_min, V3& out_max) {
         Body& b = *body_ptr(i);
         V3 pp; M3 pr;
         integrate_transform(b.pos, b.rot, b.vel, b.ang, dt, b.no_rot, pp, pr);
@@ -863,9 +864,10 @@ struct World {
         mn = mn - t; mx = mx + t;
         shape_aabb(i, pp, pr, mn2, mx2);
         mn2 = mn2 - t; mx2 = mx2 + t;
-        T->aabb_min[i] = v3(fminf(mn.x, mn2.x), fminf(mn.y, mn2.y), fminf(mn.z, mn2.z));
-        T->aabb_max[i] = v3(fmaxf(mx.x, mx2.x), fmaxf(mx.y, mx2.y), fmaxf(mx.z, mx2.z));
+        out_min = v3(fminf(mn.x, mn2.x), fminf(mn.y, mn2.y), fminf(mn.z, mn2.z));
+        out_max = v3(fmaxf(mx.x, mx2.x), fmaxf(mx.y, mx2.y), fmaxf(mx.z, mx2.z));
     }
+    RSG_FN void body_aabb(int i, float dt) { proxy_aabb(i, dt, T->aabb_min[i], T->aabb_max[i]); }
 
     RSG_FN void step_broadphase() {
         const int nb = num_bodies();
@@ -1275,7 +1277,7 @@ struct World {
             c.a = ia; c.b = ib;
             V3 rel1 = cp.pos_a - x0.t;
             V3 rel2 = cp.pos_b - x1.t;
-            setup_contact_row(S, c, ia, ib, rb0, rb1, cp.normal, cp.dist, cp.friction, cp.restitution, rel1, rel2);
+            setup_contact_row(A_, B_, S.dt, c, rb0, rb1, cp.normal, cp.dist, cp.friction, cp.restitution, rel1, rel2);
             c.special = cp.special;
             c.friction_index = S.n_fric;
             if (cp.special) {
@@ -1309,7 +1311,7 @@ struct World {
         V3 rel1 = normal * -distance;
         V3 rel2 = v3zero();
         const Body* rb0 = body_ptr(k);
-        setup_contact_row(S, c, ia, ib, rb0, nullptr, normal, distance, sp.friction, sp.restitution, rel1, rel2);
+        setup_contact_row(S.bodies[ia], S.bodies[ib], S.dt, c, rb0, nullptr, normal, distance, sp.friction, sp.restitution, rel1, rel2);
         c.special = false;
         c.friction_index = S.n_fric;
         add_friction_for(S, ia, ib, rb0, nullptr, normal, sp.friction, rel1, rel2, ci);

@@ -149,15 +149,24 @@ struct Curve {
 RSG_FN float curve_eval(const Curve& c, float input, float default_out = 1.f) {
     if (c.n == 0) return default_out;
     if (input <= c.x[0]) return c.y[0];
-    for (int i = 1; i < c.n; i++) {
-        if (c.x[i] > input) {
-            float range = c.x[i] - c.x[i - 1];
-            float diff = c.y[i] - c.y[i - 1];
-            float t = (input - c.x[i - 1]) / range;
-            return c.y[i - 1] + diff * t;
-        }
+    // the first segment that ends past the input, found by selects over
+    // constant indices: one interpolation, no table in memory
+    float x0 = 0.f, x1 = 1.f, y0 = c.y[c.n - 1], y1 = y0;
+    bool inside = false;
+    RSG_UNROLL
+    for (int i = 5; i >= 1; i--) {
+        const bool here = i < c.n && c.x[i] > input;
+        x0 = sel(here, c.x[i - 1], x0);
+        x1 = sel(here, c.x[i], x1);
+        y0 = sel(here, c.y[i - 1], y0);
+        y1 = sel(here, c.y[i], y1);
+        inside |= here;
     }
-    return c.y[c.n - 1];
+    if (!inside) return y0;
+    float range = x1 - x0;
+    float diff = y1 - y0;
+    float t = (input - x0) / range;
+    return y0 + diff * t;
 }
 
 #if defined(__HIPCC__)

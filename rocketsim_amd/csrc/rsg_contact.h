@@ -304,7 +304,7 @@ RSG_FN V3 quat_rotate(Q4 q, V3 w) {
     return v3(r.x, r.y, r.z);
 }
 
-RSG_FN float edge_angle_of(V3 a, V3 b, V3 c) { return atan2f(dot(c, a), dot(c, b)); }
+RSG_FN float edge_angle_of(V3 a, V3 b, V3 c) { return m_atan2(dot(c, a), dot(c, b)); }
 
 // btClampNormal (btInternalEdgeUtility.cpp:385-412)
 RSG_FN bool clamp_normal(V3 edge, V3 tri_normal, V3 local_n, float corrected, V3& out) {
@@ -334,62 +334,45 @@ RSG_FN void adjust_internal_edge(CPoint& cp, const MeshView& mesh, int tri) {
     V3 v[3];
     mesh_triangle(mesh, tri, v);
     V3 tri_normal = normalized(cross(v[1] - v[0], v[2] - v[0]));
-    V3 nearest;
-    nearest_on_segment(cp.local_b, v[0], v[1], nearest);
-    V3 contact = cp.local_b;
-    bool near_edge = false;
-    int concave_hits = 0;
-    V3 local_n = normalized(cp.normal);
+    const V3 local_n = normalized(cp.normal);
+    // the edge with an angle nearest the contact point (the first on ties);
+    // the reference visits every edge but acts on this one alone
     int best = -1;
     float best_d = 1e18f;
-    const float max_angle = TWO_PI_F;
-    const int ea[3] = {0, 1, 2}, eb[3] = {1, 2, 0};
     for (int e = 0; e < 3; e++) {
-        if (fabsf(info.edge_angle[e]) < max_angle) {
+        if (fabsf(info.edge_angle[e]) < TWO_PI_F) {
             V3 nn;
-            nearest_on_segment(cp.local_b, v[ea[e]], v[eb[e]], nn);
-            float l = len(contact - nn);
+            nearest_on_segment(cp.local_b, v[e], v[e == 2 ? 0 : e + 1], nn);
+            float l = len(cp.local_b - nn);
             if (l < best_d) { best = e; best_d = l; }
         }
     }
-    const uint32_t convex_bit[3] = {TRI_V0V1_CONVEX, TRI_V1V2_CONVEX, TRI_V2V0_CONVEX};
-    const uint32_t swap_bit[3] = {TRI_V0V1_SWAP, TRI_V1V2_SWAP, TRI_V2V0_SWAP};
-    for (int e = 0; e < 3; e++) {
-        if (e > 0) nearest_on_segment(contact, v[ea[e]], v[eb[e]], nearest);
-        if (!(fabsf(info.edge_angle[e]) < max_angle)) continue;
-        float l = len(contact - nearest);
-        if (!(l < 0.1f)) continue;  // m_edgeDistanceThreshold
-        if (best != e) continue;
-        V3 edge = v[ea[e]] - v[eb[e]];
-        near_edge = true;
-        float ang = info.edge_angle[e];
-        if (ang == 0.f) {
-            concave_hits++;
-        } else {
-            bool convex = (info.flags & convex_bit[e]) != 0;
-            float swap = convex ? 1.f : -1.f;
-            V3 nA = swap * tri_normal;
-            V3 comp_b = quat_rotate(q_axis_angle(edge, ang), tri_normal);
-            if (info.flags & swap_bit[e]) comp_b = comp_b * -1.f;
-            V3 nB = swap * comp_b;
-            float nda = dot(local_n, nA), ndb = dot(local_n, nB);
-            bool back = (nda < 0.f) && (ndb < 0.f);  // m_convexEpsilon = 0
-            if (back) {
-                concave_hits++;
-            } else {
-                V3 ln = (e == 0) ? local_n : cp.normal;
-                V3 clamped;
-                if (clamp_normal(edge, swap * tri_normal, ln, ang, clamped)) {
-                    if (dot(clamped, 1.f * tri_normal) > 0) {
-                        cp.normal = clamped;
-                        cp.pos_b = cp.pos_a - cp.normal * cp.dist;
-                        cp.local_b = cp.pos_b;
-                    }
+    if (best < 0 || !(best_d < 0.1f)) return;  // m_edgeDistanceThreshold
+    const float ang = pick(best, info.edge_angle[0], info.edge_angle[1], info.edge_angle[2]);
+    bool concave = ang == 0.f;
+    if (!concave) {
+        const V3 edge = best == 0 ? v[0] - v[1] : (best == 1 ? v[1] - v[2] : v[2] - v[0]);
+        const uint32_t convex_bit = best == 0 ? TRI_V0V1_CONVEX : (best == 1 ? TRI_V1V2_CONVEX : TRI_V2V0_CONVEX);
+        const uint32_t swap_bit = best == 0 ? TRI_V0V1_SWAP : (best == 1 ? TRI_V1V2_SWAP : TRI_V2V0_SWAP);
+        const float swap = (info.flags & convex_bit) ? 1.f : -1.f;
+        const V3 nA = swap * tri_normal;
+        V3 comp_b = quat_rotate(q_axis_angle(edge, ang), tri_normal);
+        if (info.flags & swap_bit) comp_b = comp_b * -1.f;
+        const V3 nB = swap * comp_b;
+        const float nda = dot(local_n, nA), ndb = dot(local_n, nB);
+        concave = (nda < 0.f) && (ndb < 0.f);  // back-facing both (m_convexEpsilon = 0)
+        if (!concave) {
+            V3 clamped;
+            if (clamp_normal(edge, swap * tri_normal, best == 0 ? local_n : cp.normal, ang, clamped)) {
+                if (dot(clamped, 1.f * tri_normal) > 0) {
+                    cp.normal = clamped;
+                    cp.pos_b = cp.pos_a - cp.normal * cp.dist;
+                    cp.local_b = cp.pos_b;
                 }
             }
         }
     }
-    if (near_edge && concave_hits > 0) {
+    if (concave) {
         V3 nn = tri_normal * 1.f;
         float d = dot(nn, local_n);
         if (d < 0) return;

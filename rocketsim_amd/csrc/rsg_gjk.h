@@ -51,7 +51,7 @@ RSG_FN V3 support_core(const CShape& s, V3 d) {
     if (s.kind == SHAPE_BOX) return v3(fsel(d.x, s.half.x, -s.half.x), fsel(d.y, s.half.y, -s.half.y), fsel(d.z, s.half.z, -s.half.z));
     if (s.kind == SHAPE_TRIANGLE) {
         V3 dots = v3(dot(d, s.v[0]), dot(d, s.v[1]), dot(d, s.v[2]));
-        return s.v[max_axis3(dots)];
+        return pick(max_axis3(dots), s.v[0], s.v[1], s.v[2]);
     }
     return v3zero();
 }
@@ -115,9 +115,16 @@ struct VoronoiSimplex {
     }
     RSG_FN void bc_reset() { degenerate = false; bc[0] = bc[1] = bc[2] = bc[3] = 0.f; used = 0; }
     RSG_FN bool bc_valid() const { return bc[0] >= 0.f && bc[1] >= 0.f && bc[2] >= 0.f && bc[3] >= 0.f; }
+    // Vertices are read and written through selects over constant indices, so
+    // that they stay in registers (an index known only at run time would put
+    // the arrays in private memory).
+    RSG_FN static V3 at(const V3 a[4], int i) { return pick(i, a[0], a[1], a[2], a[3]); }
+    RSG_FN static void put(V3 a[4], int i, V3 v) {
+        for (int k = 0; k < 4; k++) a[k] = sel(i == k, v, a[k]);
+    }
     RSG_FN void remove_vertex(int i) {
         n--;
-        W[i] = W[n]; P[i] = P[n]; Q[i] = Q[n];
+        put(W, i, at(W, n)); put(P, i, at(P, n)); put(Q, i, at(Q, n));
     }
     RSG_FN void reduce_vertices(uint32_t u) {
         if (n >= 4 && !(u & 8)) remove_vertex(3);
@@ -128,14 +135,14 @@ struct VoronoiSimplex {
     RSG_FN void add_vertex(V3 w, V3 p, V3 q) {
         last_w = w;
         needs_update = true;
-        W[n] = w; P[n] = p; Q[n] = q;
+        put(W, n, w); put(P, n, p); put(Q, n, q);
         n++;
     }
     RSG_FN bool in_simplex(V3 w) const {
         bool found = false;
-        for (int i = 0; i < n; i++) {
+        for (int i = 0; i < 4; i++) {
             V3 d = w - W[i];
-            if (len2(d) <= 0.0001f) { found = true; break; }
+            if (i < n && len2(d) <= 0.0001f) found = true;
         }
         if (w.x == last_w.x && w.y == last_w.y && w.z == last_w.z) return true;
         return found;
@@ -185,51 +192,37 @@ struct VoronoiSimplex {
         return signp * signd < 0.f ? 1 : 0;
     }
 
-    RSG_FN bool closest_tetra(V3 p, V3 a, V3 b, V3 c, V3 d) {
-        // finalResult starts as "the point itself, all four vertices"
-        used = 15;
-        int oabc = outside_plane(p, a, b, c, d);
-        int oacd = outside_plane(p, a, c, d, b);
-        int oadb = outside_plane(p, a, d, b, c);
-        int obdc = outside_plane(p, b, d, c, a);
-        if (oabc < 0 || oacd < 0 || oadb < 0 || obdc < 0) { degenerate = true; return false; }
-        if (!oabc && !oacd && !oadb && !obdc) return false;
+    // Closest point to the origin on the triangle (3 vertices) or the faces
+    // the origin is outside of (4 vertices): the vertices that carry it and
+    // their weights.  False when the origin is inside the tetrahedron, or the
+    // tetrahedron is degenerate.  Faces in the order abc, acd, adb, bdc, one
+    // instance of the triangle query for all of them.
+    RSG_FN bool closest_faces() {
+        const V3 p = v3zero();
+        uint32_t todo = 1u;
+        if (n == 4) {
+            // finalResult starts as "the point itself, all four vertices"
+            used = 15;
+            const int oabc = outside_plane(p, W[0], W[1], W[2], W[3]);
+            const int oacd = outside_plane(p, W[0], W[2], W[3], W[1]);
+            const int oadb = outside_plane(p, W[0], W[3], W[1], W[2]);
+            const int obdc = outside_plane(p, W[1], W[3], W[2], W[0]);
+            if (oabc < 0 || oacd < 0 || oadb < 0 || obdc < 0) { degenerate = true; return false; }
+            todo = (uint32_t)(oabc | oacd << 1 | oadb << 2 | obdc << 3);
+            if (!todo) return false;
+        }
         float best = 3.402823466e+38f;
-        V3 q; float w[3]; uint32_t u;
-        if (oabc) {
-            closest_tri(p, a, b, c, q, w, u);
-            float sq = dot(q - p, q - p);
-            if (sq < best) {
+        RSG_UNROLL_1
+        for (int f = 0; f < 4; f++) {
+            if (!(todo >> f & 1u)) continue;
+            const int i = f == 3 ? 1 : 0, j = f == 0 ? 1 : (f == 1 ? 2 : 3), k = f == 1 ? 3 : (f == 2 ? 1 : 2);
+            V3 q; float w[3]; uint32_t u;
+            closest_tri(p, at(W, i), at(W, j), at(W, k), q, w, u);
+            const float sq = dot(q - p, q - p);
+            if (n == 3 || sq < best) {
                 best = sq;
-                used = (u & 1) | (u & 2) | (u & 4);
-                bc[0] = w[0]; bc[1] = w[1]; bc[2] = w[2]; bc[3] = 0;
-            }
-        }
-        if (oacd) {
-            closest_tri(p, a, c, d, q, w, u);
-            float sq = dot(q - p, q - p);
-            if (sq < best) {
-                best = sq;
-                used = (u & 1) | ((u & 2) ? 4u : 0u) | ((u & 4) ? 8u : 0u);
-                bc[0] = w[0]; bc[1] = 0; bc[2] = w[1]; bc[3] = w[2];
-            }
-        }
-        if (oadb) {
-            closest_tri(p, a, d, b, q, w, u);
-            float sq = dot(q - p, q - p);
-            if (sq < best) {
-                best = sq;
-                used = (u & 1) | ((u & 4) ? 2u : 0u) | ((u & 2) ? 8u : 0u);
-                bc[0] = w[0]; bc[1] = w[2]; bc[2] = 0; bc[3] = w[1];
-            }
-        }
-        if (obdc) {
-            closest_tri(p, b, d, c, q, w, u);
-            float sq = dot(q - p, q - p);
-            if (sq < best) {
-                best = sq;
-                used = ((u & 1) ? 2u : 0u) | ((u & 4) ? 4u : 0u) | ((u & 2) ? 8u : 0u);
-                bc[0] = 0; bc[1] = w[0]; bc[2] = w[2]; bc[3] = w[1];
+                used = ((u & 1u) ? 1u << i : 0u) | ((u & 2u) ? 1u << j : 0u) | ((u & 4u) ? 1u << k : 0u);
+                for (int v = 0; v < 4; v++) bc[v] = pick(v == i ? 0 : (v == j ? 1 : (v == k ? 2 : 3)), w[0], w[1], w[2], 0.f);
             }
         }
         return true;
@@ -274,24 +267,8 @@ struct VoronoiSimplex {
             cv = cp1 - cp2;
             reduce_vertices(used);
             cached_valid = bc_valid();
-        } else if (n == 3) {
-            V3 q; float w[3]; uint32_t u;
-            closest_tri(v3zero(), W[0], W[1], W[2], q, w, u);
-            used = u;
-            bc[0] = w[0]; bc[1] = w[1]; bc[2] = w[2]; bc[3] = 0;
-            cp1 = P[0] * bc[0] + P[1] * bc[1] + P[2] * bc[2];
-            cp2 = Q[0] * bc[0] + Q[1] * bc[1] + Q[2] * bc[2];
-            cv = cp1 - cp2;
-            reduce_vertices(used);
-            cached_valid = bc_valid();
-        } else if (n == 4) {
-            bool sep = closest_tetra(v3zero(), W[0], W[1], W[2], W[3]);
-            if (sep) {
-                cp1 = P[0] * bc[0] + P[1] * bc[1] + P[2] * bc[2] + P[3] * bc[3];
-                cp2 = Q[0] * bc[0] + Q[1] * bc[1] + Q[2] * bc[2] + Q[3] * bc[3];
-                cv = cp1 - cp2;
-                reduce_vertices(used);
-            } else {
+        } else if (n == 3 || n == 4) {
+            if (!closest_faces()) {
                 if (degenerate) {
                     cached_valid = false;
                 } else {
@@ -300,6 +277,14 @@ struct VoronoiSimplex {
                 }
                 return cached_valid;
             }
+            cp1 = P[0] * bc[0] + P[1] * bc[1] + P[2] * bc[2];
+            cp2 = Q[0] * bc[0] + Q[1] * bc[1] + Q[2] * bc[2];
+            if (n == 4) {
+                cp1 += P[3] * bc[3];
+                cp2 += Q[3] * bc[3];
+            }
+            cv = cp1 - cp2;
+            reduce_vertices(used);
             cached_valid = bc_valid();
         } else {
             cached_valid = false;
@@ -339,7 +324,7 @@ RSG_FN V3 support_with_margin(const CShape& s, V3 d) {
     return v3zero() + s.margin * n;
 }
 
-RSG_FN bool ray_convex(V3 from, V3 to, const CShape& B, const Xf& tb, float& fraction, V3& normal) {
+RSG_COLD_FN bool ray_convex(V3 from, V3 to, const CShape& B, const Xf& tb, float& fraction, V3& normal) {
     VoronoiSimplex sx;
     sx.reset();
     V3 r = to - from;  // linVelA - linVelB (the shape is static)
@@ -688,6 +673,18 @@ struct PolyFace {
     bool live;
 };
 
+// One face of walk_horizon's path.
+struct PolyStep { int16_t f; uint8_t e, stage; };
+
+// Where a penetration query keeps its polytope: pools and their capacities.
+struct EpaWork {
+    SupportPt* pool;      // 4 + max_verts
+    PolyFace* faces;      // max_faces
+    int16_t* free_list;   // max_faces
+    PolyStep* steps;      // max_depth
+    int max_verts, max_faces, max_depth;
+};
+
 // Expanding polytope over a vertex pool (entries 4 on) and a face pool.
 // Outcome: 0 valid, 1 touching, 2 degenerate face, 3 non-convex, 4 bad
 // horizon, 5 out of faces, 6 out of vertices, 7 converged, 8 fallback
@@ -699,16 +696,24 @@ struct Polytope {
     float depth;
     SupportPt* pool;
     PolyFace* faces;
+    int max_verts, max_faces, max_depth;
     int n_used;       // faces[0 .. n_used) have been handed out at least once
-    int16_t free_list[POLY_MAX_FACES];
+    int16_t* free_list;
+    PolyStep* steps;  // walk_horizon's stack
     int n_free;
     int n_live;
     uint16_t clock;
     int next_vert;
+    bool full, too_deep;  // a capacity of the work space was reached
 
-    RSG_FN void reset(SupportPt* sp, PolyFace* fp) {
-        pool = sp;
-        faces = fp;
+    RSG_FN void reset(const EpaWork& w) {
+        pool = w.pool;
+        faces = w.faces;
+        free_list = w.free_list;
+        steps = w.steps;
+        max_verts = w.max_verts;
+        max_faces = w.max_faces;
+        max_depth = w.max_depth;
         outcome = 9;
         normal = v3zero();
         depth = 0;
@@ -717,6 +722,7 @@ struct Polytope {
         n_free = 0;
         n_live = 0;
         clock = 0;
+        full = too_deep = false;
     }
     RSG_FN void link(int fa, int ea, int fb, int eb) {
         faces[fa].nb_edge[ea] = (uint8_t)eb; faces[fa].nb[ea] = (int16_t)fb;
@@ -750,9 +756,10 @@ struct Polytope {
     RSG_FN int add_face(int a, int b, int c, bool forced) {
         int f;
         if (n_free > 0) f = free_list[--n_free];
-        else if (n_used < POLY_MAX_FACES) f = n_used++;
+        else if (n_used < max_faces) f = n_used++;
         else {
             outcome = 5;
+            full = true;
             return -1;
         }
         PolyFace& F = faces[f];
@@ -800,13 +807,12 @@ struct Polytope {
     // walks succeed; a face w does not see gets a new face on the shared
     // edge, linked to the previous new face along the horizon.
     RSG_FN bool walk_horizon(int mark, int w, int f0, int e0, Rim& rim) {
-        struct Step { int16_t f; uint8_t e, stage; };
-        Step st[POLY_WALK_DEPTH];
+        PolyStep* st = steps;
         int top = 0;
         st[0].f = (int16_t)f0; st[0].e = (uint8_t)e0; st[0].stage = 0;
         bool ok = false;
         while (top >= 0) {
-            Step& s = st[top];
+            PolyStep& s = st[top];
             const int f = s.f;
             const int ea = s.e == 2 ? 0 : s.e + 1;   // the edge after e
             const int eb = ea == 2 ? 0 : ea + 1;      // and the one after that
@@ -828,14 +834,14 @@ struct Polytope {
                 }
                 faces[f].mark = (uint8_t)mark;
                 s.stage = 1;
-                if (top + 1 >= POLY_WALK_DEPTH) { outcome = 4; return false; }
-                Step& c = st[++top];
+                if (top + 1 >= max_depth) { outcome = 4; too_deep = true; return false; }
+                PolyStep& c = st[++top];
                 c.f = faces[f].nb[ea]; c.e = faces[f].nb_edge[ea]; c.stage = 0;
             } else if (s.stage == 1) {
                 if (!ok) { top--; continue; }
                 s.stage = 2;
-                if (top + 1 >= POLY_WALK_DEPTH) { outcome = 4; return false; }
-                Step& c = st[++top];
+                if (top + 1 >= max_depth) { outcome = 4; too_deep = true; return false; }
+                PolyStep& c = st[++top];
                 c.f = faces[f].nb[eb]; c.e = faces[f].nb_edge[eb]; c.stage = 0;
             } else {
                 if (ok) retire(f);
@@ -873,7 +879,7 @@ struct Polytope {
                 link(t2, 2, t3, 1);
                 outcome = 0;
                 for (int step = 0; step < POLY_MAX_STEPS; step++) {
-                    if (next_vert >= POLY_MAX_VERTS) { outcome = 6; break; }
+                    if (next_vert >= max_verts) { outcome = 6; full = true; break; }
                     Rim rim{-1, -1, 0};
                     const int w = 4 + next_vert++;
                     faces[best].mark = (uint8_t)(++mark);
@@ -935,13 +941,14 @@ RSG_FN void mink_init(MinkDiff& md, const CShape& s0, const Xf& t0, const CShape
 // Penetration of the shapes with their margins (btGjkEpaSolver2::Penetration):
 // GJK, then the polytope when the origin is inside the difference.
 RSG_FN bool penetration(const CShape& s0, const Xf& t0, const CShape& s1, const Xf& t1, V3 guess, PenResult& res,
-                        SupportPt* pool, PolyFace* faces, Polytope& poly) {
+                        const EpaWork& work, Polytope& poly) {
     GjkQuery gjk;
+    SupportPt* pool = work.pool;
     mink_init(gjk.md, s0, t0, s1, t1, true);
     gjk.pool = pool;
     res.witness[0] = res.witness[1] = v3zero();
+    poly.reset(work);
     if (gjk.run(-guess) != 1) return false;
-    poly.reset(pool, faces);
     if (poly.expand(gjk, -guess) == 9) return false;
     V3 w0 = v3zero();
     for (int k = 0; k < poly.result.n; k++) w0 += gjk.md.support(pool[poly.result.idx[k]].dir, 0) * poly.result.bary[k];
@@ -974,48 +981,72 @@ RSG_FN bool separation(const CShape& s0, const Xf& t0, const CShape& s1, const X
     return true;
 }
 
-// Work space of a penetration query: the support-point pool and the
-// polytope's face pool.  The caller places it (private memory, or a
-// per-arena block in global memory that a lane reads without the per-lane
-// interleaving of private memory).
+// Work space of a penetration query at the reference's capacities.  The
+// caller places it (private memory, or a per-arena block in global memory).
 struct EpaSpace {
     SupportPt pool[SUPPORT_POOL];
     PolyFace faces[POLY_MAX_FACES];
+    int16_t free_list[POLY_MAX_FACES];
+    PolyStep steps[POLY_WALK_DEPTH];
 };
+RSG_FN EpaWork epa_work(EpaSpace& s) {
+    return EpaWork{s.pool, s.faces, s.free_list, s.steps, POLY_MAX_VERTS, POLY_MAX_FACES, POLY_WALK_DEPTH};
+}
+// A small one for LDS: queries of play use up to 9 vertices, 23 faces and a
+// path of a few; one that needs more runs again in the full space.
+struct EpaSmall {
+    SupportPt pool[4 + 16];
+    PolyFace faces[36];
+    int16_t free_list[36];
+    PolyStep steps[20];
+};
+RSG_FN EpaWork epa_work(EpaSmall& s) { return EpaWork{s.pool, s.faces, s.free_list, s.steps, 16, 36, 20}; }
 
 // Penetration depth with the reference's nine guess directions
 // (btGjkEpaPenetrationDepthSolver::calcPenDepth): the first guess for which
 // the penetration query succeeds gives the contact; a guess whose distance
-// query succeeds instead reports the shapes apart.
-RSG_FN bool calc_pen_depth(const CShape& a, const CShape& b, const Xf& ta, const Xf& tb, V3& v, V3& wa, V3& wb,
-                           EpaSpace& space) {
+// query succeeds instead reports the shapes apart.  Returns 1 or 0, and -1
+// when the query reached a capacity of `small` that the reference's are above.
+RSG_FN V3 pen_guess(int i, V3 ab) {
+    if (i == 0) return safe_normalized(ab);
+    if (i == 1) return safe_normalized(-ab);
+    const int code = i == 2 ? 1 : i == 3 ? 2 : i == 4 ? 4 : i == 5 ? 6 : i == 6 ? 7 : i == 7 ? 3 : 5;  // x 4, y 2, z 1
+    return v3((code & 4) ? 1.f : 0.f, (code & 2) ? 1.f : 0.f, (code & 1) ? 1.f : 0.f);
+}
+RSG_COLD_FN int calc_pen_depth(const CShape& a, const CShape& b, const Xf& ta, const Xf& tb, V3& v, V3& wa, V3& wb,
+                               const EpaWork& work) {
     Polytope poly;
-    const V3 guesses[9] = {safe_normalized(tb.t - ta.t), safe_normalized(ta.t - tb.t), v3(0, 0, 1), v3(0, 1, 0),
-                           v3(1, 0, 0), v3(1, 1, 0), v3(1, 1, 1), v3(0, 1, 1), v3(1, 0, 1)};
+    RSG_UNROLL_1
     for (int i = 0; i < 9; i++) {
         PenResult r;
-        if (penetration(a, ta, b, tb, guesses[i], r, space.pool, space.faces, poly)) {
+        const V3 guess = pen_guess(i, i == 1 ? -(ta.t - tb.t) : tb.t - ta.t);
+        if (penetration(a, ta, b, tb, guess, r, work, poly)) {
+            if ((poly.full && work.max_faces < POLY_MAX_FACES) || (poly.too_deep && work.max_depth < POLY_WALK_DEPTH))
+                return -1;
             wa = r.witness[0]; wb = r.witness[1]; v = r.normal;
-            return true;
+            return 1;
         }
-        if (separation(a, ta, b, tb, guesses[i], r, space.pool)) {
+        if ((poly.full && work.max_faces < POLY_MAX_FACES) || (poly.too_deep && work.max_depth < POLY_WALK_DEPTH))
+            return -1;
+        if (separation(a, ta, b, tb, guess, r, work.pool)) {
             wa = r.witness[0]; wb = r.witness[1]; v = r.normal;
-            return false;
+            return 0;
         }
     }
     wa = v3zero(); wb = v3zero(); v = v3zero();
-    return false;
+    return 0;
 }
 
 // ---------------------------------------------------------------------------
 // btGjkPairDetector::getClosestPointsNonVirtual.  Returns 1 with the
 // reported contact (normal on B pointing to A, point on B in world space,
 // signed distance) when the shapes are closer than sqrt(max_dist2), else 0.
-// Without a penetration work space (`space` null) a query that needs the
-// penetration pass returns -1 and reports nothing.
+// A query that needs the penetration pass runs it in the work space `first`
+// and, where that is too small, in `second`; without any (null) it returns -1
+// and reports nothing.
 
 RSG_FN int gjk_closest(const CShape& A, const CShape& B, const Xf& ta, const Xf& tb, float max_dist2,
-                       V3& normal_out, V3& point_b_out, float& dist_out, EpaSpace* space) {
+                       V3& normal_out, V3& point_b_out, float& dist_out, const EpaWork* first, const EpaWork* second) {
     const float REL_ERROR2 = 1.0e-6f;
     float distance = 0.f;
     V3 normalInB = v3zero();
@@ -1076,10 +1107,17 @@ RSG_FN int gjk_closest(const CShape& A, const CShape& B, const Xf& ta, const Xf&
     }
     bool catchDegenerate = degenerate != 0 && (distance + margin) < 0.01f;
     if (!isValid || catchDegenerate) {
-        if (!space) return -1;
-        V3 tA, tB;
-        sep = v3zero();
-        bool ok2 = calc_pen_depth(A, B, lta, ltb, sep, tA, tB, *space);
+        if (!first) return -1;
+        // copies for the call out of line: what it takes by reference lives in
+        // memory, and the loop's own values must not
+        const CShape shape_a = A, shape_b = B;
+        const Xf xf_a = lta, xf_b = ltb;
+        V3 tA, tB, axis = v3zero();
+        int ok2 = -1;
+        RSG_UNROLL_1
+        for (int k = 0; k < 2 && ok2 < 0; k++)
+            ok2 = calc_pen_depth(shape_a, shape_b, xf_a, xf_b, axis, tA, tB, k ? *second : *first);
+        sep = axis;
         if (ok2) {
             V3 tn = tB - tA;
             float ls = len2(tn);
@@ -1114,6 +1152,13 @@ RSG_FN int gjk_closest(const CShape& A, const CShape& B, const Xf& ta, const Xf&
         return 1;
     }
     return 0;
+}
+// The same with one work space at the reference's capacities (null: none).
+RSG_FN int gjk_closest(const CShape& A, const CShape& B, const Xf& ta, const Xf& tb, float max_dist2,
+                       V3& normal_out, V3& point_b_out, float& dist_out, EpaSpace* space) {
+    EpaWork w{};
+    if (space) w = epa_work(*space);
+    return gjk_closest(A, B, ta, tb, max_dist2, normal_out, point_b_out, dist_out, space ? &w : nullptr, &w);
 }
 
 }  // namespace rsg

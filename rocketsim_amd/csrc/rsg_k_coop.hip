@@ -1,31 +1,70 @@
-// rsg_k_coop.hip -- the cooperative step kernel: 4 lanes per car slot of an
-// arena share the tick's independent parts, the arena's working copy in LDS.
+// rsg_k_coop.hip -- the cooperative step kernel: a team of lanes (4 per car
+// slot) per arena runs the phases of rsg_team.h, the arena's working copy and
+// the tick's tables in LDS.
 #include <hip/hip_runtime.h>
 
 #include "rsg_kernels.h"
 #include "rsg_step.h"
+#include "rsg_team.h"
 
 using namespace rsg;
 
-// Cooperative variant: `lanes` lanes per arena (4 per car slot), arena in
-// LDS.  Lane 0 of each arena runs the serial parts of the tick; the lanes
-// share:
-//   * the wheel rays, one per lane, cast at the start of the pre-tick into
-//     LDS (unless a car respawns that tick: then lane 0 casts them in the
-//     loop as usual);
-//   * the car pre-ticks, one car per lane, when they are independent of
-//     their order (no wheel on a car);
-//   * the narrowphase of the world step, one planned pair per lane (the
-//     contact callbacks' effects on the arena recorded per pair and applied
-//     by lane 0 in pair order; a pair that needs the penetration pass is
-//     run again there);
-//   * the world step's per-body parts, one body per lane: the proxy AABBs
-//     (with the predicted pose) and the integration of the new poses;
-//   * the car post-ticks, one car per lane, and the boost-pad tests, pads
-//     spread over the lanes.
-// Per-arena LDS block: ArenaLocal prefix, ray results, two flag words.
+// Solver of every arena of the wave (Team::row_visit's passes): contact r of
+// an arena on its lane r, both rows in registers; an arena with more contacts
+// than lanes keeps its rows in global memory.  One loop runs the split-impulse
+// passes, then contact and friction rows in turn, level by level, so that a
+// row's update is in the code once.
+__device__ __forceinline__ void team_solve(Team& t, bool live, float dt, uint64_t team_mask) {
+    const int n = live ? t.h->n_rows : 0, levels = live ? t.h->n_levels : 0;
+    if (!__any(n > 0)) return;
+    const bool in_memory = n > t.lanes;
+    TeamRow row;
+    int level = -1;
+    RSG_UNROLL_1
+    for (int r = t.lane; r < n; r += t.lanes) {
+        t.row_setup(r, dt, row);
+        level = t.h->row.level[r];
+        if (in_memory) t.g->rows[r] = row;
+    }
+    int what = 0, it = 0;
+    bool go = n > 0;
+    RSG_UNROLL_1
+    while (true) {
+        bool moved = false;
+        RSG_UNROLL_1
+        for (int lv = 0; __any(go && lv < levels); lv++) {
+            if (go) {
+                RSG_UNROLL_1
+                for (int r = t.lane; r < n; r += t.lanes) {
+                    if ((in_memory ? (int)t.h->row.level[r] : level) != lv) continue;
+                    if (in_memory) row = t.g->rows[r];
+                    const float q = t.row_visit(row, what);
+                    moved |= !(q * q <= 0.f);
+                    if (in_memory) t.g->rows[r] = row;
+                }
+            }
+            __syncthreads();
+        }
+        if (what == 0) {
+            // an arena's split passes end once a pass moves nothing
+            go = go && (__ballot(moved) & team_mask) != 0;
+            if (++it < SOLVER_ITERATIONS && __any(go)) continue;
+            what = 1;
+            it = 0;
+            go = n > 0;
+        } else if (what == 1) {
+            what = 2;
+        } else {
+            if (++it == SOLVER_ITERATIONS) break;
+            what = 1;
+        }
+    }
+}
+
+// `lanes` lanes per arena, at most 64 per workgroup: a workgroup is one wave,
+// so its barriers only order the LDS accesses.
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RSG_COOP_WAVES_PER_EU)))
-rsg_step_arena_coop_kernel(BatchDev d, ArenaGeom geom, int ticks, int stride, int arena_bytes, int lanes) {
+rsg_step_arena_coop_kernel(BatchDev d, const ArenaGeom* geo, int ticks, int stride, int arena_bytes, int lanes) {
     extern __shared__ __align__(16) unsigned char rsg_lds[];
     const int slot = (int)threadIdx.x / lanes;
     const int k = (int)threadIdx.x - slot * lanes;
@@ -33,8 +72,6 @@ rsg_step_arena_coop_kernel(BatchDev d, ArenaGeom geom, int ticks, int stride, in
     const bool live = a < d.n;
     unsigned char* base = rsg_lds + (size_t)slot * (size_t)stride;
     ArenaLocal& A = *reinterpret_cast<ArenaLocal*>(base);
-    RayHit* hits = reinterpret_cast<RayHit*>(base + arena_bytes);
-    int* ahead = reinterpret_cast<int*>(base + arena_bytes + (size_t)(lanes) * sizeof(RayHit));
     TickParams P;
     P.mode = d.mode;
     P.dt = d.tick_time;
@@ -42,63 +79,114 @@ rsg_step_arena_coop_kernel(BatchDev d, ArenaGeom geom, int ticks, int stride, in
     P.arena_id = (uint32_t)a;
     P.synth_controls = d.synth_controls != 0;
     P.auto_reset = d.auto_reset != 0;
-    const ArenaGeom* mp = mode_has_arena(d.mode) ? &geom : nullptr;
-    StepSpace* ws = live ? arena_space(d, a) : nullptr;
-    PairLog* log = live ? arena_log(d, a) : nullptr;
-    int* concurrent = ahead + 1;
-    if (live && k == 0) load_arena(d, a, A);
+    const bool has_arena = geo != nullptr;
+    TeamGlobal* g = reinterpret_cast<TeamGlobal*>(&reinterpret_cast<ArenaSpace*>(d.space)[live ? a : 0]);
+    // The team, made anew for each phase from values the compiler cannot see
+    // through: what a phase derives from them (addresses, geometry) then lives
+    // for that phase alone.  Left to itself the compiler hoists all phases'
+    // invariants out of the tick loop, and at 256 registers that costs 260
+    // spilled registers and 400 reloads a tick.
+    auto team = [&]() {
+        unsigned off = (unsigned)slot * (unsigned)stride;
+        int lane = k, team_lanes = lanes;
+        const ArenaGeom* statics = geo;
+        TeamGlobal* space = g;
+        asm volatile("" : "+v"(off), "+v"(lane), "+s"(statics), "+s"(team_lanes), "+v"(space));
+        unsigned char* at = rsg_lds + off;
+        return Team(*reinterpret_cast<ArenaLocal*>(at), statics, at + arena_bytes, d.max_cars, space, lane, team_lanes);
+    };
+    // after the arenas' blocks: the wave's penetration work space
+    EpaSmall* small = reinterpret_cast<EpaSmall*>(rsg_lds + (size_t)(blockDim.x / lanes) * (size_t)stride);
+    const uint64_t team_mask = (lanes < 64 ? (1ull << lanes) - 1ull : ~0ull) << (slot * lanes);
+    // pairs can pass the capacity only with many statics
+    const int most_pairs = MAX_BODIES * (has_arena ? num_statics(*geo) : 0) + MAX_BODIES * (MAX_BODIES - 1) / 2;
+
+    if (live && k == 0) load_arena_scalars(d, a, A);
     __syncthreads();
-    for (int t = 0; t < ticks; t++) {
-        if (live && k == 0) *ahead = tick_begin(A, P) ? 1 : 0;
+    if (live && k < A.n_cars) load_arena_car(d, a, A, k);
+    if (live && has_arena)
+        for (int p = k; p < PAD_NUM; p += lanes) load_arena_pad(d, a, A, p);
+    __syncthreads();
+    RSG_UNROLL_1
+    for (int tick = 0; tick < ticks; tick++) {
+        if (live) team().begin(P);
         __syncthreads();
-        if (live && *ahead && k < 4 * A.n_cars) tick_cast_ray(A, P, mp, k >> 2, k & 3, hits[k]);
+        const bool respawn = live && team().any_respawn();
+        bool together = false;
+        int passes = 0;
+        // pass -1 casts every ray ahead of the cars' updates, unless a car
+        // respawns; then each pass casts its car's
+        RSG_UNROLL_1
+        for (int pass = -1; pass < 0 || __any(pass < passes); pass++) {
+            const bool on = pass < 0 ? live : pass < passes;
+            if (on && pass >= 0) team().car_begin(P, together, pass);
+            __syncthreads();
+            if (on && respawn == (pass >= 0)) team().rays(pass);
+            __syncthreads();
+            if (pass < 0) {
+                together = live && !respawn && team().independent();
+                passes = live ? team().car_passes(together) : 0;
+                continue;
+            }
+            if (on) team().wheels(P, together, pass);
+            __syncthreads();
+            if (on) team().car(P, together, pass);
+            __syncthreads();
+        }
+        if (live) team().body_begin(P);
         __syncthreads();
-        if (live && k == 0) {
-            const RayHit* pre = *ahead ? hits : nullptr;
-            *concurrent = car_pre_ticks_independent(A, pre) ? 1 : 0;
-            if (!*concurrent) {
-                World world(A, mp, mode_has_arena(d.mode));
-                for (int oi = 0; oi < A.n_cars; oi++) car_pre_tick(A, P, world, A.order[oi], pre);
+        if (live) team().ranks();
+        __syncthreads();
+        if (live) team().pairs();
+        __syncthreads();
+        if (most_pairs > MAX_PAIRS) {
+            if (live) team().trim();
+            __syncthreads();
+            if (live) team().drop_pairs();
+            __syncthreads();
+        }
+        if (live) team().plan();
+        __syncthreads();
+        // step 0: every lane its manifolds; then the effects, and the pairs that
+        // need the penetration pass, whose LDS space the wave's arenas take in turn
+        int redo_at = 0, redos = 0;
+        RSG_UNROLL_1
+        for (int step = 0; step < 2 || step <= redos; step++) {
+            if (live && (step == 0 || step == redo_at)) team().narrow(step ? 1 : 0, small);
+            __syncthreads();
+            if (step == 0) {
+                const bool redo = live && team().h->any_redo;
+                const uint64_t waiting = __ballot(redo && k == 0);
+                redos = __popcll(waiting);
+                redo_at = redo ? 1 + __popcll(waiting & ((1ull << (slot * lanes)) - 1ull)) : 1;
             }
         }
+        if (live) team().rows();
         __syncthreads();
-        if (live && *concurrent && k < A.n_cars) {
-            World world(A, mp, mode_has_arena(d.mode));
-            car_pre_tick(A, P, world, k, hits);
+        {
+            Team t = team();
+            team_solve(t, live, P.dt, team_mask);
         }
         __syncthreads();
-        if (live && k == 0) {
-            pads_pre_tick(A, P);
-            tick_world_prologue(A, P, mp, ws);
-        }
+        if (live) team().body_end(P);
         __syncthreads();
-        if (live) tick_world_aabbs(A, P, mp, ws, k, lanes);
+        if (live) team().pads(P);
         __syncthreads();
-        if (live && k == 0) tick_world_broadphase(A, P, mp, ws);
-        __syncthreads();
-        if (live) tick_world_pairs(A, P, mp, ws, log, k, lanes);
-        __syncthreads();
-        if (live && k == 0) tick_world_solve(A, P, mp, ws, log);
-        __syncthreads();
-        if (live) tick_world_integrate(A, P, mp, ws, k, lanes);
-        __syncthreads();
-        if (live && k < A.n_cars) car_post_tick(A, P, k);
-        __syncthreads();
-        if (live && mode_has_arena(d.mode))
-            for (int p = k; p < A.n_pads; p += lanes) pad_check_cars(A, p);
-        __syncthreads();
-        if (live && k == 0) tick_end(A, P);
+        if (live) team().end(P);
         __syncthreads();
     }
-    if (live && k == 0) store_arena(d, a, A);
+    if (live && k == 0) store_arena_scalars(d, a, A);
+    if (live && k < A.n_cars) store_arena_car(d, a, A, k);
+    if (live && has_arena)
+        for (int p = k; p < PAD_NUM; p += lanes) store_arena_pad(d, a, A, p);
 }
 
 namespace rsg {
 
-hipError_t launch_step_coop(const BatchDev& d, const ArenaGeom& geom, int ticks, int grid, int per_block, int stride,
+hipError_t launch_step_coop(const BatchDev& d, const ArenaGeom* geo, int ticks, int grid, int per_block, int stride,
                             int arena_bytes, int lanes, hipStream_t s) {
-    const size_t lds = (size_t)per_block * (size_t)stride;
-    hipLaunchKernelGGL(rsg_step_arena_coop_kernel, dim3(grid), dim3(per_block * lanes), lds, s, d, geom, ticks,
+    const size_t lds = (size_t)per_block * (size_t)stride + sizeof(EpaSmall);
+    hipLaunchKernelGGL(rsg_step_arena_coop_kernel, dim3(grid), dim3(per_block * lanes), lds, s, d, geo, ticks,
                        stride, arena_bytes, lanes);
     return hipGetLastError();
 }

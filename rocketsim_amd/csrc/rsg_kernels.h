@@ -22,7 +22,8 @@ hipError_t launch_step_plain(const BatchDev& d, const ArenaGeom& geom, int ticks
                              hipStream_t s);
 hipError_t launch_step_lds(const BatchDev& d, const ArenaGeom& geom, int ticks, int grid, int per_block, int stride,
                            hipStream_t s);
-hipError_t launch_step_coop(const BatchDev& d, const ArenaGeom& geom, int ticks, int grid, int per_block, int stride,
+// (`geo`: the arena's geometry in device memory, null for a mode without one)
+hipError_t launch_step_coop(const BatchDev& d, const ArenaGeom* geo, int ticks, int grid, int per_block, int stride,
                             int arena_bytes, int lanes, hipStream_t s);
 // Kickoff reset of arena `only_arena` (all arenas when < 0).
 hipError_t launch_reset(const BatchDev& d, int only_arena, uint64_t seed, hipStream_t s);

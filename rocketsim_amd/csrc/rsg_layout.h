@@ -134,6 +134,8 @@ struct BatchDev {
     const rsg_mutator_config* mut;
     // car config table: CW_CONFIG's low byte indexes it; null: the presets
     const rsg_car_config* cfgs;
+    // physics values of each entry of that table (make_car_phys)
+    const struct CarPhys* phys = nullptr;
 };
 
 }  // namespace rsg

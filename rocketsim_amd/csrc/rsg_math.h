@@ -13,8 +13,16 @@
 
 #if defined(__HIPCC__)
 #define RSG_FN __host__ __device__ __forceinline__
+// Rarely run and large: kept out of line, out of the hot loops' instruction
+// cache and registers.
+#define RSG_COLD_FN __host__ __device__ inline __attribute__((noinline))
+#define RSG_UNROLL_1 _Pragma("unroll 1")
+#define RSG_UNROLL _Pragma("unroll")
 #else
 #define RSG_FN inline
+#define RSG_COLD_FN inline
+#define RSG_UNROLL_1
+#define RSG_UNROLL
 #endif
 
 namespace rsg {
@@ -44,7 +52,24 @@ RSG_FN V3 cross(V3 a, V3 b) {
 RSG_FN float len2(V3 a) { return dot(a, a); }
 RSG_FN float len(V3 a) { return sqrtf(len2(a)); }
 RSG_FN bool is_zero(V3 a) { return a.x == 0.f && a.y == 0.f && a.z == 0.f; }
-RSG_FN float get(V3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
+// Values chosen by arithmetic selects over copies.  (A conditional over
+// lvalues or a conditional store would select an address, and an address
+// that is not constant puts the values into private memory.)
+RSG_FN float sel(bool c, float a, float b) {
+    const float x = a, y = b;
+    return c ? x : y;
+}
+RSG_FN int sel(bool c, int a, int b) {
+    const int x = a, y = b;
+    return c ? x : y;
+}
+RSG_FN V3 sel(bool c, V3 a, V3 b) { return v3(sel(c, a.x, b.x), sel(c, a.y, b.y), sel(c, a.z, b.z)); }
+// Element i of three or four.
+template <class T>
+RSG_FN T pick(int i, T a, T b, T c) { return sel(i == 0, a, sel(i == 1, b, c)); }
+template <class T>
+RSG_FN T pick(int i, T a, T b, T c, T d) { return sel(i == 0, a, sel(i == 1, b, sel(i == 2, c, d))); }
+RSG_FN float get(V3 a, int i) { return pick(i, a.x, a.y, a.z); }
 RSG_FN void set(V3& a, int i, float v) { if (i == 0) a.x = v; else if (i == 1) a.y = v; else a.z = v; }
 
 // v / |v| (Bullet normalize(): multiply by the reciprocal of the length).
@@ -113,6 +138,13 @@ RSG_FN M3 inverse(const M3& m) {
               v3(co.z * s, cofac(m, 0, 1, 2, 0) * s, cofac(m, 0, 0, 1, 1) * s));
 }
 
+// The library's trigonometry out of line: each inlined copy (with its large-
+// argument reduction) is 1-2 KB of code, and the tick has a dozen uses.
+RSG_COLD_FN float m_sin(float x) { return sinf(x); }
+RSG_COLD_FN float m_cos(float x) { return cosf(x); }
+RSG_COLD_FN float m_atan2(float y, float x) { return atan2f(y, x); }
+RSG_COLD_FN float m_pow(float x, float y) { return powf(x, y); }
+
 struct Q4 {
     float x, y, z, w;
 };
@@ -135,8 +167,8 @@ RSG_FN Q4 qmul(Q4 a, Q4 b) {
 // Axis-angle quaternion (btQuaternion::setRotation, LinearMath/btQuaternion.h:108-115).
 RSG_FN Q4 q_axis_angle(V3 axis, float angle) {
     float d = len(axis);
-    float s = sinf(angle * 0.5f) / d;
-    return q4(axis.x * s, axis.y * s, axis.z * s, cosf(angle * 0.5f));
+    float s = m_sin(angle * 0.5f) / d;
+    return q4(axis.x * s, axis.y * s, axis.z * s, m_cos(angle * 0.5f));
 }
 
 // Quaternion -> rotation matrix (btMatrix3x3::setRotation, SSE association,

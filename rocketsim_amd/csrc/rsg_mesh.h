@@ -216,7 +216,7 @@ RSG_FN void mesh_query_aabb(const MeshView& m, V3 qmin_f, V3 qmax_f, CB& cb) {
             MeshLeaf leaf[4];
             uint32_t mask = leaf_list_mask(m.box_grid, at, end, qmin_f, qmax_f, leaf);
             while (mask) {
-                const int t = (mask & 1u) ? leaf[0].tri : (mask & 2u) ? leaf[1].tri : (mask & 4u) ? leaf[2].tri : leaf[3].tri;
+                const int t = pick(__builtin_ctz(mask), leaf[0].tri, leaf[1].tri, leaf[2].tri, leaf[3].tri);
                 mask &= mask - 1u;
                 cb(t);
             }
@@ -293,8 +293,9 @@ RSG_FN void mesh_query_ray(const MeshView& m, V3 from, V3 to, CB& cb) {
             MeshLeaf leaf[4];
             uint32_t mask = leaf_list_mask(m.ray_grid, at, end, rmin, rmax, leaf);
             while (mask) {
-                const MeshLeaf& l = (mask & 1u) ? leaf[0] : (mask & 2u) ? leaf[1] : (mask & 4u) ? leaf[2] : leaf[3];
-                const int t = l.tri, node = l.node;
+                const int r4 = __builtin_ctz(mask);
+                const int t = pick(r4, leaf[0].tri, leaf[1].tri, leaf[2].tri, leaf[3].tri);
+                const int node = pick(r4, leaf[0].node, leaf[1].node, leaf[2].node, leaf[3].node);
                 mask &= mask - 1u;
                 if (ray_meets_node(m, m.nodes[node], r)) cb(t);
             }

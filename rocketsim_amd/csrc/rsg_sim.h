@@ -74,8 +74,8 @@ RSG_FN void integrate_transform(V3 pos, const M3& rot, V3 linvel, V3 angvel, flo
     if (a < 0.001f)
         axis = angvel * (0.5f * dt - (dt * dt * dt) * (0.020833333333f) * a * a);
     else
-        axis = angvel * (sinf(0.5f * a * dt) / a);
-    Q4 dorn = q4(axis.x, axis.y, axis.z, cosf(a * dt * 0.5f));
+        axis = angvel * (m_sin(0.5f * a * dt) / a);
+    Q4 dorn = q4(axis.x, axis.y, axis.z, m_cos(a * dt * 0.5f));
     Q4 orn0 = m3_to_quat(rot);
     Q4 pred = qmul(dorn, orn0);
     if (qlen2(pred) > FLT_EPS) pred = qnormalized(pred);
@@ -102,7 +102,7 @@ struct Car {
     M3 api_rot;        // CarState::rotMat: the body basis as of the last post-tick
                        // update of a car that was not demolished
     int preset, team;  // preset: the car's entry in the batch's config table
-    CarPhys phys;      // its CarConfig's physics values
+    const CarPhys* phys;  // its CarConfig's physics values
     uint32_t id;
     uint32_t flags;
     V3 flip_torque;
@@ -132,6 +132,7 @@ struct Ball {
 
 struct Pad {
     bool active;
+    uint8_t cell;       // pad grid cell, x | y << 4
     float cooldown;
     uint32_t prev_locked;
     int cur_locked;     // car index locked this tick, -1 none
@@ -241,7 +242,7 @@ RSG_FN float resolve_single_bilateral(const Body& b1, V3 pos1, const Body* other
 // used by the auto-flip.
 RSG_FN float basis_roll(const M3& m) {
     float pitch = asinf(clampf(-m.r[2].x, -1.f, 1.f));
-    float roll = atan2f(m.r[2].y, m.r[2].z);
+    float roll = m_atan2(m.r[2].y, m.r[2].z);
     if (fabsf(pitch) == 1.57079632679489661923f) {
         if (roll > 0) roll -= 3.14159265358979323846f; else roll += 3.14159265358979323846f;
     }
@@ -250,7 +251,7 @@ RSG_FN float basis_roll(const M3& m) {
 
 // Angle(yaw, 0, 0).ToRotMat(): setEulerZYX(0, 0, yaw) (MathTypes.cpp:72-78,
 // btMatrix3x3.h:304-321).
-RSG_FN M3 yaw_basis(float yaw) {
+RSG_COLD_FN M3 yaw_basis(float yaw) {
     float ci = cosf(-0.f), cj = cosf(-0.f), ch = cosf(yaw);
     float si = sinf(-0.f), sj = sinf(-0.f), sh = sinf(yaw);
     float cc = ci * ch, cs = ci * sh, sc = si * ch, ss = si * sh;
@@ -259,28 +260,30 @@ RSG_FN M3 yaw_basis(float yaw) {
               v3(-sj, cj * si, cj * ci));
 }
 
-RSG_FN V3 wheel_upwards_dir(const Car& c, const WheelT* wh) {
-    V3 sum = v3zero();
-    for (int i = 0; i < 4; i++)
-        if (wh[i].in_contact) sum += wh[i].contact_normal;
-    if (sum == v3zero()) return car_up(c);
-    return safe_normalized(sum);
+// Sum of the wheels' contact normals -> the direction they push the car
+// (Car.cpp _GetUpwardsDirFromWheelContacts).
+RSG_FN V3 upwards_dir(const Car& c, V3 normal_sum) {
+    if (normal_sum == v3zero()) return car_up(c);
+    return safe_normalized(normal_sum);
 }
 
-// _UpdateWheels (Car.cpp:339-484)
-RSG_FN void car_update_wheels(Car& c, WheelT* wh, const CarPhys& cp, float dt, int n_contact, float fwd_speed_uu) {
+// _UpdateWheels (Car.cpp:339-484) in parts: the powerslide value, the
+// throttle, the car's drive values, each wheel's friction and the force that
+// holds the car on its wheels.
+RSG_FN float car_next_handbrake(const Car& c, float dt) {
+    float h = c.handbrake;
+    if (c.ctrl.handbrake) h += POWERSLIDE_RISE_RATE * dt;
+    else h -= POWERSLIDE_FALL_RATE * dt;
+    return rs_min(rs_max(h, 0.f), 1.f);
+}
+RSG_FN float car_real_throttle(const Car& c) {
+    return c.ctrl.boost && c.boost > 0 ? 1.f : c.ctrl.throttle;
+}
+
+// Engine, brake and steering values; c.handbrake is this tick's.
+RSG_FN void car_update_drive(Car& c, const CarPhys& cp, int n_contact, float fwd_speed_uu, float real_throttle) {
     float abs_fwd = fabsf(fwd_speed_uu);
-    bool wheels_world = false;
-    for (int i = 0; i < 4; i++) wheels_world |= wh[i].with_world;
-
-    if (c.ctrl.handbrake) c.handbrake += POWERSLIDE_RISE_RATE * dt;
-    else c.handbrake -= POWERSLIDE_FALL_RATE * dt;
-    c.handbrake = rs_min(rs_max(c.handbrake, 0.f), 1.f);
-
-    float real_throttle = c.ctrl.throttle;
     float real_brake = 0;
-    if (c.ctrl.boost && c.boost > 0) real_throttle = 1;
-
     {
         float drive_scale = curve_eval(curve_drive_torque(), abs_fwd);
         float engine_throttle = real_throttle;
@@ -304,50 +307,49 @@ RSG_FN void car_update_wheels(Car& c, WheelT* wh, const CarPhys& cp, float dt, i
     }
 
     {
-        float steer_angle = curve_eval(cp.three_wheels ? curve_steer_angle_three_wheels() : curve_steer_angle(), abs_fwd);
+        float steer_angle = (cp.three_wheels ? curve_eval(curve_steer_angle_three_wheels(), abs_fwd) : curve_eval(curve_steer_angle(), abs_fwd));
         if (c.handbrake != 0.f)
             steer_angle += (curve_eval(curve_powerslide_steer(), abs_fwd) - steer_angle) * c.handbrake;
         steer_angle *= c.ctrl.steer;
         c.steer = steer_angle;
     }
+}
 
-    for (int i = 0; i < 4; i++) {
-        WheelT& w = wh[i];
-        if (w.ground != -1) {
-            V3 lat_dir = col(w.basis, 1);
-            V3 long_dir = cross(lat_dir, w.contact_normal);
-            float curve_in = 0;
-            V3 delta = w.hard_point - c.b.pos;
-            V3 cv = (cross(c.b.ang, delta) + c.b.vel) * BT_TO_UU;
-            float base_fr = fabsf(dot(cv, lat_dir));
-            if (base_fr > 5) curve_in = base_fr / (fabsf(dot(cv, long_dir)) + base_fr);
-            float lat_f = curve_eval(cp.three_wheels ? curve_lat_friction_three_wheels() : curve_lat_friction(), curve_in);
-            float long_f = curve_eval(curve_long_friction(), curve_in);
-            if (c.handbrake != 0.f) {
-                float hb = c.handbrake;
-                lat_f *= (curve_eval(curve_handbrake_lat(), curve_in) - 1) * hb + 1;
-                long_f *= (curve_eval(curve_handbrake_long(), curve_in) - 1) * hb + 1;
-            } else {
-                long_f = 1;
-            }
-            bool sticky = real_throttle != 0;
-            if (!sticky) {
-                float ns = curve_eval(curve_non_sticky(), w.contact_normal.z);
-                lat_f *= ns;
-                long_f *= ns;
-            }
-            c.lat[i] = lat_f;
-            c.lon[i] = long_f;
-        }
+// Lateral and longitudinal friction of wheel i (`handbrake` is this tick's).
+RSG_FN void wheel_update_friction(Car& c, const WheelT& w, const CarPhys& cp, int i, float handbrake,
+                                  float real_throttle) {
+    if (w.ground == -1) return;
+    V3 lat_dir = col(w.basis, 1);
+    V3 long_dir = cross(lat_dir, w.contact_normal);
+    float curve_in = 0;
+    V3 delta = w.hard_point - c.b.pos;
+    V3 cv = (cross(c.b.ang, delta) + c.b.vel) * BT_TO_UU;
+    float base_fr = fabsf(dot(cv, lat_dir));
+    if (base_fr > 5) curve_in = base_fr / (fabsf(dot(cv, long_dir)) + base_fr);
+    float lat_f = (cp.three_wheels ? curve_eval(curve_lat_friction_three_wheels(), curve_in) : curve_eval(curve_lat_friction(), curve_in));
+    float long_f = curve_eval(curve_long_friction(), curve_in);
+    if (handbrake != 0.f) {
+        float hb = handbrake;
+        lat_f *= (curve_eval(curve_handbrake_lat(), curve_in) - 1) * hb + 1;
+        long_f *= (curve_eval(curve_handbrake_long(), curve_in) - 1) * hb + 1;
+    } else {
+        long_f = 1;
     }
+    bool sticky = real_throttle != 0;
+    if (!sticky) {
+        float ns = curve_eval(curve_non_sticky(), w.contact_normal.z);
+        lat_f *= ns;
+        long_f *= ns;
+    }
+    c.lat[i] = lat_f;
+    c.lon[i] = long_f;
+}
 
-    if (wheels_world) {
-        V3 up_dir = wheel_upwards_dir(c, wh);
-        bool full_stick = (real_throttle != 0) || (abs_fwd > STOPPING_FORWARD_VEL);
-        float sticky_scale = cp.three_wheels ? 0.f : 0.5f;
-        if (full_stick) sticky_scale += 1 - fabsf(up_dir.z);
-        body_apply_central_force(c.b, up_dir * sticky_scale * (GRAVITY_Z * UU_TO_BT) * CAR_MASS_BT);
-    }
+RSG_FN void car_stick_force(Car& c, const CarPhys& cp, V3 up_dir, float fwd_speed_uu, float real_throttle) {
+    bool full_stick = (real_throttle != 0) || (fabsf(fwd_speed_uu) > STOPPING_FORWARD_VEL);
+    float sticky_scale = cp.three_wheels ? 0.f : 0.5f;
+    if (full_stick) sticky_scale += 1 - fabsf(up_dir.z);
+    body_apply_central_force(c.b, up_dir * sticky_scale * (GRAVITY_Z * UU_TO_BT) * CAR_MASS_BT);
 }
 
 // _UpdateBoost (Car.cpp:486-533), Soccar mutators (no recharge).
@@ -481,7 +483,7 @@ RSG_FN void car_update_double_jump_or_flip(Car& c, float dt, bool jump_pressed, 
 
         if (jump_pressed && c.air_time_since_jump < DOUBLEJUMP_MAX_DELAY) {
             float in_mag = fabsf(c.ctrl.yaw) + fabsf(c.ctrl.pitch) + fabsf(c.ctrl.roll);
-            bool is_flip = in_mag >= c.phys.dodge_deadzone;
+            bool is_flip = in_mag >= c.phys->dodge_deadzone;
             bool can_use = (!flag(c.flags, RSG_CF_HAS_DOUBLE_JUMPED) && !flag(c.flags, RSG_CF_HAS_FLIPPED)) ||
                            (is_flip ? M.unlimited_flips : M.unlimited_double_jumps);
             if (flag(c.flags, RSG_CF_AUTO_FLIPPING)) can_use = false;
@@ -526,7 +528,7 @@ RSG_FN void car_update_double_jump_or_flip(Car& c, float dt, bool jump_pressed, 
         c.flip_time += dt;
         if (c.flip_time <= FLIP_TORQUE_TIME) {
             if (c.flip_time >= FLIP_Z_DAMP_START && (c.b.vel.z < 0 || c.flip_time < FLIP_Z_DAMP_END)) {
-                c.b.vel.z *= powf(1 - FLIP_Z_DAMP_120, dt / (1 / 120.f));
+                c.b.vel.z *= m_pow(1 - FLIP_Z_DAMP_120, dt / (1 / 120.f));
             }
         }
     } else if (flag(c.flags, RSG_CF_HAS_FLIPPED)) {
@@ -558,8 +560,9 @@ RSG_FN void car_update_auto_flip(Car& c, float dt, bool jump_pressed) {
 }
 
 // _UpdateAutoRoll (Car.cpp:819-853)
-RSG_FN void car_update_auto_roll(Car& c, WheelT* wh, int n_contact) {
-    V3 ground_up = n_contact > 0 ? wheel_upwards_dir(c, wh) : c.world_normal;
+// (`ground_up`: the wheels' upwards direction, or the last world contact's
+// normal when no wheel touches).
+RSG_FN void car_update_auto_roll(Car& c, V3 ground_up) {
     V3 ground_down = -ground_up;
     V3 fwd = car_forward(c), right = car_right(c);
     V3 cross_right = cross(ground_up, fwd);
@@ -574,46 +577,43 @@ RSG_FN void car_update_auto_roll(Car& c, WheelT* wh, int n_contact) {
     body_apply_torque(c.b, inverse(c.b.inv_iw) * (t_fwd + t_right) * CAR_AUTOROLL_TORQUE);
 }
 
-// btVehicleRL::calcFrictionImpulses (btVehicleRL.cpp:306-380)
+// btVehicleRL::calcFrictionImpulses (btVehicleRL.cpp:306-380) of wheel i on
+// `ground` (null: the static world).
+RSG_FN void wheel_friction_impulse(const Car& c, WheelT& w, int i, const Body* ground, float dt) {
+    const float friction_scale = (1.f / c.b.inv_mass) / 3;  // getMass() = 1 / inverseMass
+    if (w.ground == -1) { w.impulse = v3zero(); return; }
+    V3 axle = col(w.basis, 1);
+    V3 n = w.contact_normal;
+    float proj = dot(axle, n);
+    axle -= n * proj;
+    axle = safe_normalized(axle);
+    V3 fwd = safe_normalized(cross(n, axle));
+    float side = resolve_single_bilateral(c.b, w.contact_point, ground, w.contact_point, axle);
+    float rolling;
+    if (c.engine == 0) {
+        if (c.brake != 0.f) {
+            V3 rel_car = w.contact_point - c.b.pos;
+            V3 v1 = body_vel_at(c.b, rel_car);
+            V3 v2 = ground ? body_vel_at(*ground, rel_car) : v3zero();
+            float rel_vel = dot(v1 - v2, fwd);
+            if (dt > (1 / 80.f)) {
+                float thr = -(1 / (dt * 150.f)) + 0.8f;
+                if (fabsf(rel_vel) < thr) rel_vel = 0;
+            }
+            rolling = clampf(-rel_vel * ROLLING_FRICTION_SCALE_MAGIC, -c.brake, c.brake);
+        } else {
+            rolling = 0;
+        }
+    } else {
+        rolling = -c.engine / friction_scale;
+    }
+    V3 total = (fwd * rolling * c.lon[i]) + (axle * side * c.lat[i]);
+    w.impulse = total * friction_scale;
+}
 template <class World>
 RSG_FN void vehicle_calc_friction(Car& c, WheelT* wh, World& world, float dt) {
-    float friction_scale = CAR_MASS_BT / 3;  // getMass() = 1 / inverseMass
-    friction_scale = (1.f / c.b.inv_mass) / 3;
-    for (int i = 0; i < 4; i++) {
-        WheelT& w = wh[i];
-        if (w.ground != -1) {
-            const Body* ground = w.ground >= 0 ? world.body_ptr(w.ground) : nullptr;
-            V3 axle = col(w.basis, 1);
-            V3 n = w.contact_normal;
-            float proj = dot(axle, n);
-            axle -= n * proj;
-            axle = safe_normalized(axle);
-            V3 fwd = safe_normalized(cross(n, axle));
-            float side = resolve_single_bilateral(c.b, w.contact_point, ground, w.contact_point, axle);
-            float rolling;
-            if (c.engine == 0) {
-                if (c.brake != 0.f) {
-                    V3 rel_car = w.contact_point - c.b.pos;
-                    V3 v1 = body_vel_at(c.b, rel_car);
-                    V3 v2 = ground ? body_vel_at(*ground, rel_car) : v3zero();
-                    float rel_vel = dot(v1 - v2, fwd);
-                    if (dt > (1 / 80.f)) {
-                        float thr = -(1 / (dt * 150.f)) + 0.8f;
-                        if (fabsf(rel_vel) < thr) rel_vel = 0;
-                    }
-                    rolling = clampf(-rel_vel * ROLLING_FRICTION_SCALE_MAGIC, -c.brake, c.brake);
-                } else {
-                    rolling = 0;
-                }
-            } else {
-                rolling = -c.engine / friction_scale;
-            }
-            V3 total = (fwd * rolling * c.lon[i]) + (axle * side * c.lat[i]);
-            w.impulse = total * friction_scale;
-        } else {
-            w.impulse = v3zero();
-        }
-    }
+    for (int i = 0; i < 4; i++)
+        wheel_friction_impulse(c, wh[i], i, wh[i].ground >= 0 ? world.body_ptr(wh[i].ground) : nullptr, dt);
 }
 
 // The suspension ray of wheel i (btVehicleRL.cpp:123-131): from the wheel's
@@ -626,23 +626,13 @@ RSG_FN void wheel_ray(const Car& c, const CarPhys& cp, int i, V3& source, V3& ta
     target = source + (w.dir_ws * ray_len);
 }
 
-// btVehicleRL::rayCast (btVehicleRL.cpp:120-209).  `pre`, when given, is this
-// wheel's ray result cast earlier in the same pre-tick (nothing it depends on
-// has changed since).
-template <class World>
-RSG_FN void vehicle_ray_cast(Car& c, WheelT* wh, const CarPhys& cp, int i, World& world, int self_body, const SolverInfo& si,
-                             const RayHit* pre) {
-    WheelT& w = wh[i];
-    wheel_transforms_ws(c, cp, i, w);
+// btVehicleRL::rayCast (btVehicleRL.cpp:120-209) of wheel i, given its ray's
+// result.
+RSG_FN void wheel_contact(Car& c, WheelT& w, const CarPhys& cp, int i, const RayHit& h, const SolverInfo& si) {
     float travel = cp.max_susp_travel;
     float rest = cp.wheel_rest[i];
     float radius = cp.wheel_radius[i];
-    float ray_len = rest + travel + radius - SUSPENSION_SUBTRACTION;
-    V3 source = w.hard_point;
-    V3 target = source + (w.dir_ws * ray_len);
-    w.contact_point = target;
     w.ground = -1;
-    RayHit h = pre ? *pre : world.raycast(source, target, self_body);
     V3 up = car_up(c);
     if (h.hit) {
         w.contact_point = h.point;
@@ -673,6 +663,8 @@ RSG_FN void vehicle_ray_cast(Car& c, WheelT* wh, const CarPhys& cp, int i, World
             }
         }
     } else {
+        float ray_len = rest + travel + radius - SUSPENSION_SUBTRACTION;
+        w.contact_point = w.hard_point + (w.dir_ws * ray_len);
         w.susp_len = rest + travel;
         w.susp_rel_vel = 0;
         w.contact_normal = -w.dir_ws;
@@ -680,58 +672,77 @@ RSG_FN void vehicle_ray_cast(Car& c, WheelT* wh, const CarPhys& cp, int i, World
         c.push[i] = 0;
     }
 }
+// The same with the ray cast here, unless `pre` holds its result, cast
+// earlier in the same pre-tick (nothing it depends on has changed since).
+template <class World>
+RSG_FN void vehicle_ray_cast(Car& c, WheelT* wh, const CarPhys& cp, int i, World& world, int self_body, const SolverInfo& si,
+                             const RayHit* pre) {
+    WheelT& w = wh[i];
+    wheel_transforms_ws(c, cp, i, w);
+    float ray_len = cp.wheel_rest[i] + cp.max_susp_travel + cp.wheel_radius[i] - SUSPENSION_SUBTRACTION;
+    V3 source = w.hard_point;
+    V3 target = source + (w.dir_ws * ray_len);
+    wheel_contact(c, w, cp, i, pre ? *pre : world.raycast(source, target, self_body), si);
+}
 
-// btVehicleRL::updateSuspension + applyFrictionImpulses (btVehicleRL.cpp:270-395)
-RSG_FN void vehicle_second(Car& c, WheelT* wh, const CarPhys& cp, float dt) {
-    for (int i = 0; i < 4; i++) {
-        WheelT& w = wh[i];
-        if (w.in_contact) {
-            float force = (cp.wheel_rest[i] - w.susp_len) * SUSPENSION_STIFFNESS * w.clipped_inv;
-            float damp = (w.susp_rel_vel < 0) ? WHEELS_DAMPING_COMPRESSION : WHEELS_DAMPING_RELAXATION;
-            w.susp_force = force - (damp * w.susp_rel_vel);
-            w.susp_force *= cp.wheel_force_scale[i];
-            if (w.susp_force < 0) w.susp_force = 0;
-        } else {
-            w.susp_force = 0;
-        }
+// btVehicleRL::updateSuspension (btVehicleRL.cpp:270-304) of wheel i.
+RSG_FN void wheel_susp_force(WheelT& w, const CarPhys& cp, int i) {
+    if (w.in_contact) {
+        float force = (cp.wheel_rest[i] - w.susp_len) * SUSPENSION_STIFFNESS * w.clipped_inv;
+        float damp = (w.susp_rel_vel < 0) ? WHEELS_DAMPING_COMPRESSION : WHEELS_DAMPING_RELAXATION;
+        w.susp_force = force - (damp * w.susp_rel_vel);
+        w.susp_force *= cp.wheel_force_scale[i];
+        if (w.susp_force < 0) w.susp_force = 0;
+    } else {
+        w.susp_force = 0;
     }
-    for (int i = 0; i < 4; i++) {
-        WheelT& w = wh[i];
-        if (w.susp_force != 0) {
-            V3 off = w.contact_point - c.b.pos;
-            float base = (w.susp_force * dt) + c.push[i];
-            V3 f = w.contact_normal * base;
-            body_apply_impulse(c.b, f, off);
-        }
-    }
+}
+// Wheel i's two impulses (suspension; tire friction: applyFrictionImpulses,
+// btVehicleRL.cpp:382-395) and where they act.
+RSG_FN void wheel_susp_impulse(const Car& c, const WheelT& w, int i, float dt, V3& impulse, V3& rel) {
+    rel = w.contact_point - c.b.pos;
+    float base = (w.susp_force * dt) + c.push[i];
+    impulse = w.contact_normal * base;
+}
+RSG_FN void wheel_tire_impulse(const Car& c, const WheelT& w, float dt, V3& impulse, V3& rel) {
     V3 up = car_up(c);
-    for (int i = 0; i < 4; i++) {
-        WheelT& w = wh[i];
-        if (!is_zero(w.impulse)) {
-            V3 off = w.contact_point - c.b.pos;
-            float d = dot(up, off);
-            V3 rel = off - up * d;
-            body_apply_impulse(c.b, w.impulse * dt, rel);
+    V3 off = w.contact_point - c.b.pos;
+    float d = dot(up, off);
+    rel = off - up * d;
+    impulse = w.impulse * dt;
+}
+RSG_FN void vehicle_second(Car& c, WheelT* wh, const CarPhys& cp, float dt) {
+    V3 imp, rel;
+    for (int i = 0; i < 4; i++) wheel_susp_force(wh[i], cp, i);
+    for (int i = 0; i < 4; i++)
+        if (wh[i].susp_force != 0) {
+            wheel_susp_impulse(c, wh[i], i, dt, imp, rel);
+            body_apply_impulse(c.b, imp, rel);
         }
-    }
+    for (int i = 0; i < 4; i++)
+        if (!is_zero(wh[i].impulse)) {
+            wheel_tire_impulse(c, wh[i], dt, imp, rel);
+            body_apply_impulse(c.b, imp, rel);
+        }
 }
 
 // Car::Respawn (Car.cpp:43-56) at a given respawn slot of the mode's table.
-RSG_FN void car_respawn_state(Car& c, int mode, int slot, float boost_amount) {
+RSG_COLD_FN void car_respawn_state(Car& c, int mode, int slot, float boost_amount) {
     SpawnPos sp = respawn_spawn_of(mode, slot);
     V3 pos_uu = v3(sp.x, sp.y * (c.team == RSG_TEAM_BLUE ? 1.f : -1.f), CAR_RESPAWN_Z);
     float yaw = (float)((double)sp.yaw + (c.team == RSG_TEAM_BLUE ? 0.0 : PI_D));
-    // CarState() defaults then SetState (Car.cpp:23-36)
-    Car keep = c;
-    c = Car();
-    c.b = keep.b;
-    c.preset = keep.preset; c.team = keep.team; c.id = keep.id;
-    c.phys = keep.phys;
-    c.ctrl = keep.ctrl;
-    c.gen_redraw = keep.gen_redraw; c.gen_left = keep.gen_left;
-    // Per-wheel values persist across SetState in the reference.
-    c.engine = keep.engine; c.brake = keep.brake; c.steer = keep.steer;
-    for (int i = 0; i < 4; i++) { c.lat[i] = keep.lat[i]; c.lon[i] = keep.lon[i]; c.push[i] = keep.push[i]; }
+    // CarState() defaults then SetState (Car.cpp:23-36); the body's mass
+    // properties, the config, the controls and the per-wheel values stay
+    const uint32_t body_flag = c.flags & RSG_CF_BODY_DISABLED;
+    c.flip_torque = v3zero();
+    c.jump_time = c.flip_time = c.air_time = c.air_time_since_jump = 0.f;
+    c.time_since_boosted = c.boosting_time = c.supersonic_time = c.handbrake = 0.f;
+    c.af_timer = c.af_scale = 0.f;
+    c.world_normal = v3zero();
+    c.other_id = 0;
+    c.car_cooldown = c.demo_timer = 0.f;
+    c.hit_rel_pos = c.hit_ball_pos = c.hit_extra_vel = v3zero();
+    c.last = Ctrl();
     c.vel_cache = v3zero();
     c.b.pos = pos_uu * UU_TO_BT;
     c.b.rot = yaw_basis(yaw);
@@ -741,7 +752,7 @@ RSG_FN void car_respawn_state(Car& c, int mode, int slot, float boost_amount) {
     body_update_inertia(c.b);
     // CarState default isOnGround = true; the body flag is not part of the
     // state SetState writes
-    c.flags = RSG_CF_ON_GROUND | (keep.flags & RSG_CF_BODY_DISABLED);
+    c.flags = RSG_CF_ON_GROUND | body_flag;
     c.boost = boost_amount;
     c.hit_tick = ~0ull;
     c.hit_extra_tick = ~0ull;

@@ -126,12 +126,10 @@ RSG_FN int solver_body_id(Solver& S, int body, BodyAt& body_at) {
 }
 
 // setupContactConstraint (btSequentialImpulseConstraintSolver.cpp:795-976)
-RSG_FN void setup_contact_row(Solver& S, SRow& c, int ia, int ib, const Body* rb0, const Body* rb1,
+RSG_FN void setup_contact_row(const SBody& A, const SBody& B, float dt, SRow& c, const Body* rb0, const Body* rb1,
                               V3 normal, float dist, float friction, float restitution_coef,
                               V3 rel1, V3 rel2) {
-    SBody& A = S.bodies[ia];
-    SBody& B = S.bodies[ib];
-    float inv_dt = 1.f / S.dt;
+    float inv_dt = 1.f / dt;
     float cfm = 0.f;  // m_globalCfm
     float erp = SOLVER_ERP2;
     cfm *= inv_dt;
@@ -191,11 +189,8 @@ RSG_FN void setup_contact_row(Solver& S, SRow& c, int ia, int ib, const Body* rb
 }
 
 // setupFrictionConstraint (btSequentialImpulseConstraintSolver.cpp:513-602)
-RSG_FN void setup_friction_row(Solver& S, SRow& c, int ia, int ib, const Body* rb0, const Body* rb1,
+RSG_FN void setup_friction_row(const SBody& A, const SBody& B, SRow& c, const Body* rb0, const Body* rb1,
                                V3 axis, float friction, V3 rel1, V3 rel2) {
-    SBody& A = S.bodies[ia];
-    SBody& B = S.bodies[ib];
-    c.a = ia; c.b = ib;
     c.friction = friction;
     c.applied = 0.f;
     c.applied_push = 0.f;
@@ -239,10 +234,7 @@ RSG_FN void setup_friction_row(Solver& S, SRow& c, int ia, int ib, const Body* r
 // convertContactInner's friction part with SOLVER_USE_WARMSTARTING | SOLVER_SIMD
 // (btSequentialImpulseConstraintSolver.cpp:1071-1161): one friction row along
 // the relative tangential velocity, or btPlaneSpace1 of the normal when slow.
-RSG_FN void add_friction_for(Solver& S, int ia, int ib, const Body* rb0, const Body* rb1,
-                             V3 normal, float friction, V3 rel1, V3 rel2, int contact_index) {
-    SBody& A = S.bodies[ia];
-    SBody& B = S.bodies[ib];
+RSG_FN V3 friction_direction(const SBody& A, const SBody& B, V3 normal, V3 rel1, V3 rel2) {
     V3 vel1 = A.body >= 0 ? (A.lin + A.ext_f) + cross(A.ang + A.ext_t, rel1) : v3zero();
     V3 vel2 = B.body >= 0 ? (B.lin + B.ext_f) + cross(B.ang + B.ext_t, rel2) : v3zero();
     V3 vel = vel1 - vel2;
@@ -255,36 +247,49 @@ RSG_FN void add_friction_for(Solver& S, int ia, int ib, const Body* rb0, const B
         V3 d2;
         plane_space(normal, dir, d2);
     }
+    return dir;
+}
+RSG_FN void add_friction_for(Solver& S, int ia, int ib, const Body* rb0, const Body* rb1,
+                             V3 normal, float friction, V3 rel1, V3 rel2, int contact_index) {
+    const V3 dir = friction_direction(S.bodies[ia], S.bodies[ib], normal, rel1, rel2);
     if (S.n_fric >= MAX_ROWS) { S.overflow = true; return; }
     SRow& f = S.fric[S.n_fric++];
-    setup_friction_row(S, f, ia, ib, rb0, rb1, dir, friction, rel1, rel2);
+    f.a = ia; f.b = ib;
+    setup_friction_row(S.bodies[ia], S.bodies[ib], f, rb0, rb1, dir, friction, rel1, rel2);
     f.friction_index = contact_index;
 }
 
-RSG_FN float resolve_lower(Solver& S, SRow& c) {
-    SBody& A = S.bodies[c.a];
-    SBody& B = S.bodies[c.b];
-    float delta = c.rhs - c.applied * c.cfm;
-    float d1 = sdot(c.n1, A.dv) + sdot(c.rc1, A.dw);
-    float d2 = sdot(c.n2, B.dv) + sdot(c.rc2, B.dw);
+// One body's side of a row: its solver velocities (fixed: none) and inverse mass.
+struct RowSide {
+    bool dynamic;
+    V3 inv_mass;
+    V3 lin, ang;
+};
+
+// The rows' updates over the two sides' velocities (resolveSingleConstraintRow*,
+// btSequentialImpulseConstraintSolver.cpp:136-262).
+RSG_FN float row_delta(const SRow& c, float rhs, float applied, const RowSide& A, const RowSide& B) {
+    float delta = rhs - applied * c.cfm;
+    float d1 = sdot(c.n1, A.lin) + sdot(c.rc1, A.ang);
+    float d2 = sdot(c.n2, B.lin) + sdot(c.rc2, B.ang);
     delta = delta - d1 * c.jac_inv;
     delta = delta - d2 * c.jac_inv;
+    return delta;
+}
+RSG_FN void row_apply(const SRow& c, float delta, RowSide& A, RowSide& B) {
+    if (A.dynamic) { A.lin += (c.n1 * A.inv_mass) * delta; A.ang += c.ang_a * delta; }
+    if (B.dynamic) { B.lin += (c.n2 * B.inv_mass) * delta; B.ang += c.ang_b * delta; }
+}
+RSG_FN float row_lower(SRow& c, RowSide& A, RowSide& B) {
+    float delta = row_delta(c, c.rhs, c.applied, A, B);
     float sum = c.applied + delta;
     if (sum < c.lo) { delta = c.lo - c.applied; c.applied = c.lo; }
     else c.applied = sum;
-    if (A.body >= 0) { A.dv += (c.n1 * A.inv_mass) * delta; A.dw += c.ang_a * delta; }
-    if (B.body >= 0) { B.dv += (c.n2 * B.inv_mass) * delta; B.dw += c.ang_b * delta; }
+    row_apply(c, delta, A, B);
     return delta / c.jac_inv;
 }
-
-RSG_FN float resolve_generic(Solver& S, SRow& c) {
-    SBody& A = S.bodies[c.a];
-    SBody& B = S.bodies[c.b];
-    float delta = c.rhs - c.applied * c.cfm;
-    float d1 = sdot(c.n1, A.dv) + sdot(c.rc1, A.dw);
-    float d2 = sdot(c.n2, B.dv) + sdot(c.rc2, B.dw);
-    delta = delta - d1 * c.jac_inv;
-    delta = delta - d2 * c.jac_inv;
+RSG_FN float row_generic(SRow& c, RowSide& A, RowSide& B) {
+    float delta = row_delta(c, c.rhs, c.applied, A, B);
     float sum = c.applied + delta;
     bool lower_less = sum < c.lo;
     bool upper_less = sum < c.hi;
@@ -294,26 +299,45 @@ RSG_FN float resolve_generic(Solver& S, SRow& c) {
     float upper_min_applied = c.hi - c.applied;
     delta = upper_less ? delta : upper_min_applied;
     c.applied = upper_less ? app : c.hi;
-    if (A.body >= 0) { A.dv += (c.n1 * A.inv_mass) * delta; A.dw += c.ang_a * delta; }
-    if (B.body >= 0) { B.dv += (c.n2 * B.inv_mass) * delta; B.dw += c.ang_b * delta; }
+    row_apply(c, delta, A, B);
     return delta / c.jac_inv;
+}
+// The split-impulse row: the sides carry the push and turn velocities.
+RSG_FN float row_split(SRow& c, RowSide& A, RowSide& B) {
+    float delta = row_delta(c, c.rhs_pen, c.applied_push, A, B);
+    float sum = c.applied_push + delta;
+    if (sum < c.lo) { delta = c.lo - c.applied_push; c.applied_push = c.lo; }
+    else c.applied_push = sum;
+    row_apply(c, delta, A, B);
+    return delta * (1.f / c.jac_inv);
+}
+
+RSG_FN RowSide side_vel(const SBody& b) { return RowSide{b.body >= 0, b.inv_mass, b.dv, b.dw}; }
+RSG_FN RowSide side_push(const SBody& b) { return RowSide{b.body >= 0, b.inv_mass, b.push, b.turn}; }
+
+RSG_FN float resolve_lower(Solver& S, SRow& c) {
+    RowSide A = side_vel(S.bodies[c.a]), B = side_vel(S.bodies[c.b]);
+    const float r = row_lower(c, A, B);
+    if (A.dynamic) { S.bodies[c.a].dv = A.lin; S.bodies[c.a].dw = A.ang; }
+    if (B.dynamic) { S.bodies[c.b].dv = B.lin; S.bodies[c.b].dw = B.ang; }
+    return r;
+}
+
+RSG_FN float resolve_generic(Solver& S, SRow& c) {
+    RowSide A = side_vel(S.bodies[c.a]), B = side_vel(S.bodies[c.b]);
+    const float r = row_generic(c, A, B);
+    if (A.dynamic) { S.bodies[c.a].dv = A.lin; S.bodies[c.a].dw = A.ang; }
+    if (B.dynamic) { S.bodies[c.b].dv = B.lin; S.bodies[c.b].dw = B.ang; }
+    return r;
 }
 
 RSG_FN float resolve_split(Solver& S, SRow& c) {
     if (!(c.rhs_pen != 0.f)) return 0.f;
-    SBody& A = S.bodies[c.a];
-    SBody& B = S.bodies[c.b];
-    float delta = c.rhs_pen - c.applied_push * c.cfm;
-    float d1 = sdot(c.n1, A.push) + sdot(c.rc1, A.turn);
-    float d2 = sdot(c.n2, B.push) + sdot(c.rc2, B.turn);
-    delta = delta - d1 * c.jac_inv;
-    delta = delta - d2 * c.jac_inv;
-    float sum = c.applied_push + delta;
-    if (sum < c.lo) { delta = c.lo - c.applied_push; c.applied_push = c.lo; }
-    else c.applied_push = sum;
-    if (A.body >= 0) { A.push += (c.n1 * A.inv_mass) * delta; A.turn += c.ang_a * delta; }
-    if (B.body >= 0) { B.push += (c.n2 * B.inv_mass) * delta; B.turn += c.ang_b * delta; }
-    return delta * (1.f / c.jac_inv);
+    RowSide A = side_push(S.bodies[c.a]), B = side_push(S.bodies[c.b]);
+    const float r = row_split(c, A, B);
+    if (A.dynamic) { S.bodies[c.a].push = A.lin; S.bodies[c.a].turn = A.ang; }
+    if (B.dynamic) { S.bodies[c.b].push = B.lin; S.bodies[c.b].turn = B.ang; }
+    return r;
 }
 
 RSG_FN void solver_iterate(Solver& S) {

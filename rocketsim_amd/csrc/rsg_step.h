@@ -9,10 +9,12 @@
 namespace rsg {
 
 // Waves per SIMD the step kernels are compiled for (register budget).  The
-// plain and LDS kernels run fastest with the whole register file (1); the
-// cooperative kernel, whose lanes wait on each other at every barrier, gains
-// from a second wave per SIMD to switch to (measured at 2v2 x 16384 arenas:
-// 0.98 ms per tick at 2 against 1.16 ms at 1, 1.03 at 3 and 1.08 at 4).
+// plain and LDS kernels run fastest with the whole register file (1).  The
+// cooperative kernel waits on memory and on its slowest lane half of the time
+// and gains from a second wave per SIMD where there are waves to fill it
+// (2v2 x 16384 arenas: 0.515 ms a tick at 2, 0.561 at 1; 32768 arenas of 1v1
+// to 3v3: 0.81 and 1.14), and loses a little to its spills where there are
+// not (2v2 x 4096: 0.303 and 0.271).
 #ifndef RSG_STEP_WAVES_PER_EU
 #define RSG_STEP_WAVES_PER_EU 1
 #endif
@@ -23,9 +25,6 @@ namespace rsg {
 // Arena `a`'s block of the batch's global work space.
 RSG_FN StepSpace* arena_space(const BatchDev& d, int a) {
     return &reinterpret_cast<ArenaSpace*>(d.space)[a].step;
-}
-RSG_FN PairLog* arena_log(const BatchDev& d, int a) {
-    return &reinterpret_cast<ArenaSpace*>(d.space)[a].log;
 }
 
 RSG_FN void step_arena(const BatchDev& d, const ArenaGeom& geom, int a, int ticks, ArenaLocal& A, StepSpace* ws) {

@@ -153,7 +153,7 @@ RSG_FN void store_car(const CarRef& r, const Car& c) {
 // The car body's mass properties: the preset's unless the arena's
 // SetMutatorConfig replaced them (`inv_mass`, `inertia_mass` nonzero).
 RSG_FN void car_init_body(Car& c, float inv_mass, float inertia_mass) {
-    const CarPhys& cp = c.phys;
+    const CarPhys& cp = *c.phys;
     c.b.force = v3zero();
     c.b.torque = v3zero();
     c.b.inv_i_local = cp.inv_inertia_local;
@@ -177,7 +177,14 @@ RSG_FN void ball_init_body(Ball& b) {
     b.vel_cache = v3zero();
 }
 
-RSG_FN void load_arena(const BatchDev& d, int a, ArenaLocal& A) {
+// BoostPadGrid::Add cell of each pad; the grid maps each occupied (x,y) cell
+// to one pad (src/Sim/BoostPad/BoostPadGrid/BoostPadGrid.cpp:27-41).
+RSG_FN int pad_cell_x(V3 p) { return (int)(p.x / PAD_GRID_CELL_SIZE_X + (PAD_GRID_CELLS_X / 2)); }
+RSG_FN int pad_cell_y(V3 p) { return (int)(p.y / PAD_GRID_CELL_SIZE_Y + (PAD_GRID_CELLS_Y / 2)); }
+
+// An arena's gather in parts that lanes can share: the scalars and the ball,
+// car i, pad p.
+RSG_FN void load_arena_scalars(const BatchDev& d, int a, ArenaLocal& A) {
     CarRef ar = arena_ref(d, a);
     A.tick = ar.u64(AW_TICK);
     A.n_cars = (int)ar.u(AW_NUM_CARS);
@@ -213,15 +220,7 @@ RSG_FN void load_arena(const BatchDev& d, int a, ArenaLocal& A) {
     }
     A.si.erp = 0.2f;
     A.si.time_step = d.tick_time;
-    for (int i = 0; i < A.n_cars; i++) {
-        CarRef cr = car_ref(d, a, i);
-        load_car(cr, A.cars[i]);
-        A.cars[i].phys = make_car_phys(d.cfgs ? d.cfgs[A.cars[i].preset] : preset_config(A.cars[i].preset));
-        car_init_body(A.cars[i], cr.f(CW_BODY_INV_MASS), cr.f(CW_BODY_INERTIA_MASS));
-        A.cars[i].b.grav = cr.v(CW_BODY_GRAVITY);
-        A.cars[i].b.active = !flag(A.cars[i].flags, RSG_CF_BODY_DISABLED);
-        load_bp(cr, CW_BP_CELL, CW_BP_SEQ, A.bp_cell[1 + i], A.bp_seq[1 + i]);
-    }
+    A.ball_damping = m_pow(1.f - fminf(fmaxf(A.mut.ball_drag, 0.f), 1.f), d.tick_time);
     CarRef br = ball_ref(d, a);
     A.ball.b.pos = br.v(BW_POS);
     A.ball.b.rot = load_rot(br, BW_ROT);
@@ -238,18 +237,42 @@ RSG_FN void load_arena(const BatchDev& d, int a, ArenaLocal& A) {
     A.ball.hs_speed = br.f(BW_HS + 1);
     A.ball.hs_time = br.f(BW_HS + 2);
     load_bp(br, BW_BP_CELL, BW_BP_SEQ, A.bp_cell[0], A.bp_seq[0]);
-    if (mode_has_arena(d.mode)) {
-        for (int p = 0; p < PAD_NUM; p++) {
-            CarRef pr = pad_ref(d, a, p);
-            A.pads[p].active = pr.u(PW_ACTIVE) != 0;
-            A.pads[p].cooldown = pr.f(PW_COOLDOWN);
-            A.pads[p].prev_locked = pr.u(PW_PREV_LOCKED);
-            A.pads[p].cur_locked = -1;
-        }
+}
+RSG_FN void load_arena_car(const BatchDev& d, int a, ArenaLocal& A, int i) {
+    CarRef cr = car_ref(d, a, i);
+    load_car(cr, A.cars[i]);
+#if defined(__HIPCC__)
+    A.cars[i].phys = &d.phys[A.cars[i].preset];
+#else
+    A.own_phys[i] = make_car_phys(d.cfgs ? d.cfgs[A.cars[i].preset] : preset_config(A.cars[i].preset));
+    A.cars[i].phys = &A.own_phys[i];
+#endif
+    car_init_body(A.cars[i], cr.f(CW_BODY_INV_MASS), cr.f(CW_BODY_INERTIA_MASS));
+    A.cars[i].b.grav = cr.v(CW_BODY_GRAVITY);
+    A.cars[i].b.active = !flag(A.cars[i].flags, RSG_CF_BODY_DISABLED);
+    load_bp(cr, CW_BP_CELL, CW_BP_SEQ, A.bp_cell[1 + i], A.bp_seq[1 + i]);
+}
+RSG_FN void load_arena_pad(const BatchDev& d, int a, ArenaLocal& A, int p) {
+    CarRef pr = pad_ref(d, a, p);
+    A.pads[p].active = pr.u(PW_ACTIVE) != 0;
+    A.pads[p].cooldown = pr.f(PW_COOLDOWN);
+    A.pads[p].prev_locked = pr.u(PW_PREV_LOCKED);
+    A.pads[p].cur_locked = -1;
+    A.pads[p].cell = 0;
+    if (!A.custom_pads) {
+        const V3 pl = pad_location(A.mode, p);
+        A.pads[p].cell = (uint8_t)(pad_cell_x(pl) | pad_cell_y(pl) << 4);
     }
 }
+RSG_FN void load_arena(const BatchDev& d, int a, ArenaLocal& A) {
+    load_arena_scalars(d, a, A);
+    for (int i = 0; i < A.n_cars; i++) load_arena_car(d, a, A, i);
+    if (mode_has_arena(d.mode))
+        for (int p = 0; p < PAD_NUM; p++) load_arena_pad(d, a, A, p);
+}
 
-RSG_FN void store_arena(const BatchDev& d, int a, const ArenaLocal& A) {
+// The scatter, in the same parts.
+RSG_FN void store_arena_scalars(const BatchDev& d, int a, const ArenaLocal& A) {
     CarRef ar = arena_ref(d, a);
     ar.su64(AW_TICK, A.tick);
     ar.u(AW_GOALS_BLUE) = A.goals_blue;
@@ -263,12 +286,6 @@ RSG_FN void store_arena(const BatchDev& d, int a, const ArenaLocal& A) {
         for (int k = 0; k < MAX_CARS; k++) ow |= (uint32_t)(A.order[k] & 0xFu) << (4 * k);
         ar.u(AW_CAR_ORDER) = ow;
     }
-    for (int i = 0; i < A.n_cars; i++) {
-        CarRef cr = car_ref(d, a, i);
-        store_car(cr, A.cars[i]);
-        cr.u(CW_BP_CELL) = (uint32_t)A.bp_cell[1 + i];
-        cr.u(CW_BP_SEQ) = A.bp_seq[1 + i];
-    }
     CarRef br = ball_ref(d, a);
     br.u(BW_BP_CELL) = (uint32_t)A.bp_cell[0];
     br.u(BW_BP_SEQ) = A.bp_seq[0];
@@ -281,14 +298,24 @@ RSG_FN void store_arena(const BatchDev& d, int a, const ArenaLocal& A) {
     br.sf(BW_HS + 1, A.ball.hs_speed);
     br.sf(BW_HS + 2, A.ball.hs_time);
     br.u(BW_AWAKE) = A.ball.b.active ? 1u : 0u;
-    if (mode_has_arena(d.mode)) {
-        for (int p = 0; p < PAD_NUM; p++) {
-            CarRef pr = pad_ref(d, a, p);
-            pr.u(PW_ACTIVE) = A.pads[p].active ? 1u : 0u;
-            pr.sf(PW_COOLDOWN, A.pads[p].cooldown);
-            pr.u(PW_PREV_LOCKED) = A.pads[p].prev_locked;
-        }
-    }
+}
+RSG_FN void store_arena_car(const BatchDev& d, int a, const ArenaLocal& A, int i) {
+    CarRef cr = car_ref(d, a, i);
+    store_car(cr, A.cars[i]);
+    cr.u(CW_BP_CELL) = (uint32_t)A.bp_cell[1 + i];
+    cr.u(CW_BP_SEQ) = A.bp_seq[1 + i];
+}
+RSG_FN void store_arena_pad(const BatchDev& d, int a, const ArenaLocal& A, int p) {
+    CarRef pr = pad_ref(d, a, p);
+    pr.u(PW_ACTIVE) = A.pads[p].active ? 1u : 0u;
+    pr.sf(PW_COOLDOWN, A.pads[p].cooldown);
+    pr.u(PW_PREV_LOCKED) = A.pads[p].prev_locked;
+}
+RSG_FN void store_arena(const BatchDev& d, int a, const ArenaLocal& A) {
+    store_arena_scalars(d, a, A);
+    for (int i = 0; i < A.n_cars; i++) store_arena_car(d, a, A, i);
+    if (mode_has_arena(d.mode))
+        for (int p = 0; p < PAD_NUM; p++) store_arena_pad(d, a, A, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -372,11 +399,6 @@ RSG_FN V3 arena_pad_location(const ArenaLocal& A, int p) {
     return pad_location(A.mode, p);
 }
 
-// BoostPadGrid::Add cell of each pad; the grid maps each occupied (x,y) cell
-// to one pad (src/Sim/BoostPad/BoostPadGrid/BoostPadGrid.cpp:27-41).
-RSG_FN int pad_cell_x(V3 p) { return (int)(p.x / PAD_GRID_CELL_SIZE_X + (PAD_GRID_CELLS_X / 2)); }
-RSG_FN int pad_cell_y(V3 p) { return (int)(p.y / PAD_GRID_CELL_SIZE_Y + (PAD_GRID_CELLS_Y / 2)); }
-
 RSG_FN void pad_check_collide(const ArenaLocal& A, Pad& pad, int p, const Car& c, int car_idx, const CarPhys& cp) {
     V3 pos_uu = arena_pad_location(A, p);
     V3 pos_bt = pos_uu * UU_TO_BT;
@@ -406,30 +428,33 @@ RSG_FN void pad_check_collide(const ArenaLocal& A, Pad& pad, int p, const Car& c
 // ---------------------------------------------------------------------------
 // The tick
 
+// Car i's controls of the tick, drawn from the seeded process.
+RSG_FN void tick_car_controls(ArenaLocal& A, const TickParams& P, int i) {
+    if (!P.synth_controls) return;
+    Car& c = A.cars[i];
+    rsg_ctrl_gen g = {c.gen_redraw, c.gen_left};
+    rsg_controls rc;
+    rc.throttle = c.ctrl.throttle; rc.steer = c.ctrl.steer; rc.pitch = c.ctrl.pitch;
+    rc.yaw = c.ctrl.yaw; rc.roll = c.ctrl.roll;
+    rc.jump = c.ctrl.jump; rc.boost = c.ctrl.boost; rc.handbrake = c.ctrl.handbrake;
+    rsg_ctrl_next(P.seed, P.arena_id, (uint32_t)i, &g, &rc);
+    c.gen_redraw = g.redraw; c.gen_left = g.ticks_left;
+    c.ctrl.throttle = rc.throttle; c.ctrl.steer = rc.steer; c.ctrl.pitch = rc.pitch;
+    c.ctrl.yaw = rc.yaw; c.ctrl.roll = rc.roll;
+    c.ctrl.jump = rc.jump; c.ctrl.boost = rc.boost; c.ctrl.handbrake = rc.handbrake;
+}
+// The ball's sleep flag (Arena.cpp:694-700).
+RSG_FN void tick_ball_sleep(ArenaLocal& A) {
+    A.ball.b.active = !(len2(A.ball.b.vel) == 0.f && len2(A.ball.b.ang) == 0.f);
+}
+
 // Start of Arena::Step: the synthetic controls and the ball's sleep flag.
 // Returns whether every wheel ray of the tick may be cast before the per-car
 // pre-tick loop: true unless a demolished car respawns this tick, which moves
 // it in the middle of the loop.
 RSG_FN bool tick_begin(ArenaLocal& A, const TickParams& P) {
-    if (P.synth_controls) {
-        for (int i = 0; i < A.n_cars; i++) {
-            Car& c = A.cars[i];
-            rsg_ctrl_gen g = {c.gen_redraw, c.gen_left};
-            rsg_controls rc;
-            rc.throttle = c.ctrl.throttle; rc.steer = c.ctrl.steer; rc.pitch = c.ctrl.pitch;
-            rc.yaw = c.ctrl.yaw; rc.roll = c.ctrl.roll;
-            rc.jump = c.ctrl.jump; rc.boost = c.ctrl.boost; rc.handbrake = c.ctrl.handbrake;
-            rsg_ctrl_next(P.seed, P.arena_id, (uint32_t)i, &g, &rc);
-            c.gen_redraw = g.redraw; c.gen_left = g.ticks_left;
-            c.ctrl.throttle = rc.throttle; c.ctrl.steer = rc.steer; c.ctrl.pitch = rc.pitch;
-            c.ctrl.yaw = rc.yaw; c.ctrl.roll = rc.roll;
-            c.ctrl.jump = rc.jump; c.ctrl.boost = rc.boost; c.ctrl.handbrake = rc.handbrake;
-        }
-    }
-
-    // 1. ball sleep flag (Arena.cpp:694-700)
-    A.ball.b.active = !(len2(A.ball.b.vel) == 0.f && len2(A.ball.b.ang) == 0.f);
-
+    for (int i = 0; i < A.n_cars; i++) tick_car_controls(A, P, i);
+    tick_ball_sleep(A);
     for (int i = 0; i < A.n_cars; i++) {
         const Car& c = A.cars[i];
         if (flag(c.flags, RSG_CF_DEMOED) && rs_max(c.demo_timer - P.dt, 0.f) == 0.f) return false;
@@ -437,27 +462,10 @@ RSG_FN bool tick_begin(ArenaLocal& A, const TickParams& P) {
     return true;
 }
 
-// Wheel ray `wheel` of car `ci` as the pre-tick loop will cast it, computed
-// ahead of the loop (valid when tick_begin returned true): poses, broadphase
-// cells and contact-response flags are those the car sees at its turn.
-RSG_FN void tick_cast_ray(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, int ci, int wheel, RayHit& out) {
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr);
-    int pos = 0;
-    while (pos < A.n_cars && A.order[pos] != ci) pos++;
-    world.ray_caster_pos = pos;
-    const Car& c = A.cars[ci];
-    const CarPhys& cp = c.phys;
-    V3 source, target;
-    wheel_ray(c, cp, wheel, source, target);
-    out = world.raycast(source, target, 1 + ci);
-}
-
-// Car pre-tick (Car.cpp:58-131) of car `ci`.  `pre` holds every wheel's ray
-// result (car-major, 4 per car) when cast ahead, else null.
-RSG_FN void car_pre_tick(ArenaLocal& A, const TickParams& P, World& world, int ci, const RayHit* pre) {
-    const float dt = P.dt;
+// Car pre-tick (Car.cpp:58-131) of car `ci`, in parts.  First: the controls'
+// range, respawn and the body's activation.
+RSG_FN void car_pre_begin(ArenaLocal& A, const TickParams& P, int ci) {
     Car& c = A.cars[ci];
-    const CarPhys& cp = c.phys;
     c.ctrl.throttle = clampf(c.ctrl.throttle, -1, 1);
     c.ctrl.steer = clampf(c.ctrl.steer, -1, 1);
     c.ctrl.pitch = clampf(c.ctrl.pitch, -1, 1);
@@ -465,7 +473,7 @@ RSG_FN void car_pre_tick(ArenaLocal& A, const TickParams& P, World& world, int c
     c.ctrl.roll = clampf(c.ctrl.roll, -1, 1);
 
     if (flag(c.flags, RSG_CF_DEMOED)) {
-        c.demo_timer = rs_max(c.demo_timer - dt, 0.f);
+        c.demo_timer = rs_max(c.demo_timer - P.dt, 0.f);
         if (c.demo_timer == 0) {
             int slot = (int)(rsg_draw(P.seed ^ 0xDE40ull, P.arena_id, (uint32_t)ci, (uint32_t)A.tick, 9) % 4u);
             car_respawn_state(c, A.mode, slot, A.mut.car_spawn_boost_amount);
@@ -475,26 +483,27 @@ RSG_FN void car_pre_tick(ArenaLocal& A, const TickParams& P, World& world, int c
         c.b.active = true;
     }
     setflag(c.flags, RSG_CF_BODY_DISABLED, !c.b.active);
-    if (flag(c.flags, RSG_CF_DEMOED)) return;
+}
 
-    // updateVehicleFirst (btVehicleRL.cpp:215-228)
-    // btVehicleRL's wheel records: rebuilt every tick, used only in this pre-tick
-    WheelT wh[4];
-    for (int i = 0; i < 4; i++) wheel_update_transform(c, cp, i, wh[i]);
-    for (int i = 0; i < 4; i++) {
-        vehicle_ray_cast(c, wh, cp, i, world, 1 + ci, A.si, pre ? &pre[ci * 4 + i] : nullptr);
-    }
-    vehicle_calc_friction(c, wh, world, dt);
-
+// The car's game logic after updateVehicleFirst (btVehicleRL.cpp:215-228):
+// `contact` has a bit per wheel that touches something, `on_world` whether one
+// touches the arena, `normal_sum` is the sum of their contact normals.
+RSG_FN void car_pre_logic(ArenaLocal& A, const TickParams& P, Car& c, uint32_t contact, bool on_world, V3 normal_sum) {
+    const float dt = P.dt;
+    const CarPhys& cp = *c.phys;
     bool jump_pressed = c.ctrl.jump && !c.last.jump;
     int n_contact = 0;
     for (int i = 0; i < 4; i++) {
-        setflag(c.flags, RSG_CF_WHEEL0 << i, wh[i].in_contact);
-        n_contact += wh[i].in_contact ? 1 : 0;
+        setflag(c.flags, RSG_CF_WHEEL0 << i, (contact >> i & 1u) != 0);
+        n_contact += (int)(contact >> i & 1u);
     }
     setflag(c.flags, RSG_CF_ON_GROUND, n_contact >= 3);
     float fwd_speed_uu = dot(c.b.vel, car_forward(c)) * BT_TO_UU;
-    car_update_wheels(c, wh, cp, dt, n_contact, fwd_speed_uu);
+    const V3 up_dir = n_contact > 0 ? upwards_dir(c, normal_sum) : c.world_normal;
+    const float real_throttle = car_real_throttle(c);
+    c.handbrake = car_next_handbrake(c, dt);
+    car_update_drive(c, cp, n_contact, fwd_speed_uu, real_throttle);
+    if (on_world) car_stick_force(c, cp, up_dir, fwd_speed_uu, real_throttle);
     if (n_contact < 3)
         car_update_air_torque(c, dt, n_contact == 0);
     else
@@ -503,32 +512,50 @@ RSG_FN void car_pre_tick(ArenaLocal& A, const TickParams& P, World& world, int c
     car_update_auto_flip(c, dt, jump_pressed);
     car_update_double_jump_or_flip(c, dt, jump_pressed, fwd_speed_uu, A.mut);
     if (c.ctrl.throttle != 0.f && ((n_contact > 0 && n_contact < 4) || flag(c.flags, RSG_CF_WORLD_CONTACT)))
-        car_update_auto_roll(c, wh, n_contact);
+        car_update_auto_roll(c, up_dir);
     setflag(c.flags, RSG_CF_WORLD_CONTACT, false);
+}
+
+// The whole pre-tick on one lane.  `pre` holds every wheel's ray result
+// (car-major, 4 per car) when cast ahead, else null.
+RSG_FN void car_pre_tick(ArenaLocal& A, const TickParams& P, World& world, int ci, const RayHit* pre) {
+    const float dt = P.dt;
+    Car& c = A.cars[ci];
+    const CarPhys& cp = *c.phys;
+    car_pre_begin(A, P, ci);
+    if (flag(c.flags, RSG_CF_DEMOED)) return;
+    // btVehicleRL's wheel records: rebuilt every tick, used only in this pre-tick
+    WheelT wh[4];
+    for (int i = 0; i < 4; i++) wheel_update_transform(c, cp, i, wh[i]);
+    RSG_UNROLL_1
+    for (int i = 0; i < 4; i++) {
+        vehicle_ray_cast(c, wh, cp, i, world, 1 + ci, A.si, pre ? &pre[ci * 4 + i] : nullptr);
+    }
+    vehicle_calc_friction(c, wh, world, dt);
+    uint32_t contact = 0;
+    bool on_world = false;
+    V3 normal_sum = v3zero();
+    for (int i = 0; i < 4; i++) {
+        wheel_update_friction(c, wh[i], cp, i, car_next_handbrake(c, dt), car_real_throttle(c));
+        on_world |= wh[i].with_world;
+        if (!wh[i].in_contact) continue;
+        contact |= 1u << i;
+        normal_sum += wh[i].contact_normal;
+    }
+    car_pre_logic(A, P, c, contact, on_world, normal_sum);
     vehicle_second(c, wh, cp, dt);
     car_update_boost(c, dt, A.mut);
 }
 
-// Whether the car pre-ticks of this tick are independent of their order, so
-// that they may run concurrently: the rays were cast ahead and no wheel rests
-// on a car (tire friction reads the velocity of a car ground, which that
-// car's own pre-tick changes).
-RSG_FN bool car_pre_ticks_independent(const ArenaLocal& A, const RayHit* pre) {
-    if (!pre) return false;
-    for (int k = 0; k < 4 * A.n_cars; k++)
-        if (pre[k].hit && !pre[k].is_static && pre[k].body >= 1) return false;
-    return true;
-}
-
 // Pads pre-tick (BoostPad.cpp:51-60).
+RSG_FN void pad_pre_tick(Pad& pad, float dt) {
+    if (pad.cooldown > 0) pad.cooldown = rs_max(pad.cooldown - dt, 0.f);
+    pad.active = (pad.cooldown == 0);
+    pad.cur_locked = -1;
+}
 RSG_FN void pads_pre_tick(ArenaLocal& A, const TickParams& P) {
     if (!mode_has_arena(P.mode) || A.n_cars == 0) return;
-    for (int p = 0; p < A.n_pads; p++) {
-        Pad& pad = A.pads[p];
-        if (pad.cooldown > 0) pad.cooldown = rs_max(pad.cooldown - P.dt, 0.f);
-        pad.active = (pad.cooldown == 0);
-        pad.cur_locked = -1;
-    }
+    for (int p = 0; p < A.n_pads; p++) pad_pre_tick(A.pads[p], P.dt);
 }
 
 // Car post-tick (Car.cpp:133-193) and _FinishPhysicsTick of car `ci`.
@@ -563,6 +590,19 @@ RSG_FN void car_post_tick(ArenaLocal& A, const TickParams& P, int ci) {
     c.ticks_since_set++;
 }
 
+// The boost-pad grid window of a car (BoostPadGrid.cpp:5-25); false when the
+// car takes no pads.
+RSG_FN bool car_pad_window(const ArenaLocal& A, const Car& c, int& x0, int& x1, int& y0, int& y1) {
+    if (flag(c.flags, RSG_CF_DEMOED) || c.boost >= BOOST_MAX) return false;
+    V3 cp_uu = c.b.pos * BT_TO_UU;
+    if (cp_uu.z > PAD_GRID_EXTENT_Z) return false;
+    int ix = (int)(cp_uu.x / PAD_GRID_CELL_SIZE_X + (PAD_GRID_CELLS_X / 2));
+    int iy = (int)(cp_uu.y / PAD_GRID_CELL_SIZE_Y + (PAD_GRID_CELLS_Y / 2));
+    x0 = ix - 1 > 0 ? ix - 1 : 0; x1 = ix + 1 < PAD_GRID_CELLS_X - 1 ? ix + 1 : PAD_GRID_CELLS_X - 1;
+    y0 = iy - 1 > 0 ? iy - 1 : 0; y1 = iy + 1 < PAD_GRID_CELLS_Y - 1 ? iy + 1 : PAD_GRID_CELLS_Y - 1;
+    return true;
+}
+
 // Boost pad p against every car, in the car update order (the reference
 // checks each car against the pads of its 3x3 grid window right after the
 // car's post-tick, Arena.cpp:720-734 and BoostPadGrid.cpp:5-25; a pad's
@@ -574,71 +614,59 @@ RSG_FN void pad_check_cars(ArenaLocal& A, int p) {
         // early outs (Arena.cpp:723-728)
         for (int oi = 0; oi < A.n_cars; oi++) {
             const int ci = A.order[oi];
-            pad_check_collide(A, A.pads[p], p, A.cars[ci], ci, A.cars[ci].phys);
+            pad_check_collide(A, A.pads[p], p, A.cars[ci], ci, *A.cars[ci].phys);
         }
         return;
     }
-    V3 pl = pad_location(A.mode, p);
-    int px = pad_cell_x(pl), py = pad_cell_y(pl);
+    const int px = A.pads[p].cell & 15, py = A.pads[p].cell >> 4;
     for (int oi = 0; oi < A.n_cars; oi++) {
         const int ci = A.order[oi];
         const Car& c = A.cars[ci];
-        if (flag(c.flags, RSG_CF_DEMOED) || c.boost >= BOOST_MAX) continue;
-        V3 cp_uu = c.b.pos * BT_TO_UU;
-        if (cp_uu.z > PAD_GRID_EXTENT_Z) continue;
-        int ix = (int)(cp_uu.x / PAD_GRID_CELL_SIZE_X + (PAD_GRID_CELLS_X / 2));
-        int iy = (int)(cp_uu.y / PAD_GRID_CELL_SIZE_Y + (PAD_GRID_CELLS_Y / 2));
-        int x0 = ix - 1 > 0 ? ix - 1 : 0, x1 = ix + 1 < PAD_GRID_CELLS_X - 1 ? ix + 1 : PAD_GRID_CELLS_X - 1;
-        int y0 = iy - 1 > 0 ? iy - 1 : 0, y1 = iy + 1 < PAD_GRID_CELLS_Y - 1 ? iy + 1 : PAD_GRID_CELLS_Y - 1;
-        if (px >= x0 && px <= x1 && py >= y0 && py <= y1) pad_check_collide(A, A.pads[p], p, c, ci, c.phys);
+        int x0, x1, y0, y1;
+        if (!car_pad_window(A, c, x0, x1, y0, y1)) continue;
+        if (px >= x0 && px <= x1 && py >= y0 && py <= y1) pad_check_collide(A, A.pads[p], p, c, ci, *c.phys);
     }
 }
 
-// End of Arena::Step: pads post-tick, ball finish, goal test, tick count,
-// kickoff reset on goal.
-RSG_FN void tick_end(ArenaLocal& A, const TickParams& P) {
-    const float dt = P.dt;
-    const bool soccar = mode_has_arena(P.mode);
-    // 6. pads post-tick (BoostPad.cpp:88-107)
-    if (soccar && A.n_cars > 0) {
-        for (int p = 0; p < A.n_pads; p++) {
-            Pad& pad = A.pads[p];
-            uint32_t locked_id = 0;
-            if (pad.cur_locked >= 0) {
-                Car& c = A.cars[pad.cur_locked];
-                locked_id = c.id;
-                if (pad.active) {
-                    float add = pad_is_big(A, p) ? PAD_BOOST_AMOUNT_BIG : PAD_BOOST_AMOUNT_SMALL;
-                    c.boost = rs_min(c.boost + add, BOOST_MAX);
-                    pad.active = false;
-                    pad.cooldown = pad_is_big(A, p) ? A.mut.boost_pad_cooldown_big : A.mut.boost_pad_cooldown_small;
-                }
-            }
-            pad.prev_locked = locked_id;
+// Pad p's post-tick (BoostPad.cpp:88-107).
+RSG_FN void pad_post_tick(ArenaLocal& A, int p) {
+    Pad& pad = A.pads[p];
+    uint32_t locked_id = 0;
+    if (pad.cur_locked >= 0) {
+        Car& c = A.cars[pad.cur_locked];
+        locked_id = c.id;
+        if (pad.active) {
+            float add = pad_is_big(A, p) ? PAD_BOOST_AMOUNT_BIG : PAD_BOOST_AMOUNT_SMALL;
+            c.boost = rs_min(c.boost + add, BOOST_MAX);
+            pad.active = false;
+            pad.cooldown = pad_is_big(A, p) ? A.mut.boost_pad_cooldown_big : A.mut.boost_pad_cooldown_small;
         }
     }
+    pad.prev_locked = locked_id;
+}
 
-    // 7. ball finish (Ball.cpp:117-143)
-    {
-        Body& b = A.ball.b;
-        if (!is_zero(A.ball.vel_cache)) {
-            b.vel += A.ball.vel_cache;
-            A.ball.vel_cache = v3zero();
-        }
-        V3 v = b.vel, w = b.ang;
-        float max_bt = A.mut.ball_max_speed * UU_TO_BT;
-        if (len2(v) > max_bt * max_bt) v = normalized(v) * max_bt;
-        if (len2(w) > (BALL_MAX_ANG_SPEED * BALL_MAX_ANG_SPEED)) w = normalized(w) * BALL_MAX_ANG_SPEED;
-        b.vel = v;
-        b.ang = w;
-        A.ball.ticks_since_set++;
+// Ball finish (Ball.cpp:117-143).
+RSG_FN void ball_finish(ArenaLocal& A) {
+    Body& b = A.ball.b;
+    if (!is_zero(A.ball.vel_cache)) {
+        b.vel += A.ball.vel_cache;
+        A.ball.vel_cache = v3zero();
     }
+    V3 v = b.vel, w = b.ang;
+    float max_bt = A.mut.ball_max_speed * UU_TO_BT;
+    if (len2(v) > max_bt * max_bt) v = normalized(v) * max_bt;
+    if (len2(w) > (BALL_MAX_ANG_SPEED * BALL_MAX_ANG_SPEED)) w = normalized(w) * BALL_MAX_ANG_SPEED;
+    b.vel = v;
+    b.ang = w;
+    A.ball.ticks_since_set++;
+}
 
-    A.si.time_step = dt;
-
-    // 8. goal test (Arena.cpp:893-901) and optional kickoff reset
+// The goal test (Arena.cpp:893-901), the tick count and the finiteness test;
+// returns whether the arena takes a kickoff reset.
+RSG_FN bool tick_finish(ArenaLocal& A, const TickParams& P) {
+    A.si.time_step = P.dt;
     bool scored = false;
-    if (soccar) {
+    if (mode_has_arena(P.mode)) {
         float y = A.ball.b.pos.y * BT_TO_UU;
         if (ball_scored(A.mode, A.ball.b.pos, A.mut)) {
             scored = true;
@@ -654,7 +682,16 @@ RSG_FN void tick_end(ArenaLocal& A, const TickParams& P) {
         for (int i = 0; i < A.n_cars; i++) s += A.cars[i].b.pos + A.cars[i].b.vel + A.cars[i].b.ang;
         if (!(isfinite(s.x) && isfinite(s.y) && isfinite(s.z))) A.status |= RSG_STATUS_NONFINITE;
     }
-    if (scored && P.auto_reset) arena_kickoff_reset(A, P.seed, P.arena_id);
+    return scored && P.auto_reset;
+}
+
+// End of Arena::Step: pads post-tick, ball finish, goal test, tick count,
+// kickoff reset on goal.
+RSG_FN void tick_end(ArenaLocal& A, const TickParams& P) {
+    if (mode_has_arena(P.mode) && A.n_cars > 0)
+        for (int p = 0; p < A.n_pads; p++) pad_post_tick(A, p);
+    ball_finish(A);
+    if (tick_finish(A, P)) arena_kickoff_reset(A, P.seed, P.arena_id);
 }
 
 // Angle::FromVec (src/Math/MathTypes/MathTypes.cpp:80-100): yaw and pitch
@@ -662,9 +699,9 @@ RSG_FN void tick_end(ArenaLocal& A, const TickParams& P) {
 RSG_FN void hs_angle_from_vec(V3 f, float& yaw, float& pitch) {
     const float eps = 1.1920928955078125e-07f;
     if (fabsf(f.y) > eps || fabsf(f.x) > eps) {
-        yaw = atan2f(f.y, f.x);
+        yaw = m_atan2(f.y, f.x);
         float d2 = sqrtf(f.x * f.x + f.y * f.y);
-        pitch = -atan2f(-f.z, d2);
+        pitch = -m_atan2(-f.z, d2);
     } else {
         yaw = 0;
         pitch = f.z > eps ? (float)(PI_D / 2) : (f.z < -eps ? (float)(-PI_D / 2) : 0.f);
@@ -691,7 +728,7 @@ RSG_FN float hs_round_ue3(float a) {
 // Ball::_PreTickUpdate for Heatseeker (src/Sim/Ball/Ball.cpp:161-206): once
 // a team has touched it, the ball turns its velocity towards the target net
 // and blends its speed towards the target speed.
-RSG_FN void ball_pre_tick_heatseeker(Ball& ball, float dt) {
+RSG_COLD_FN void ball_pre_tick_heatseeker(Ball& ball, float dt) {
     if (ball.hs_dir == 0) return;
     const float pi_f = (float)PI_D, half_pi_f = (float)(PI_D / 2);
     V3 pos = ball.b.pos * BT_TO_UU, vel = ball.b.vel * BT_TO_UU;
@@ -711,7 +748,7 @@ RSG_FN void ball_pre_tick_heatseeker(Ball& ball, float dt) {
     pitch = hs_round_ue3(pitch);
     float new_speed = speed + ((ball.hs_speed - speed) * HS_SPEED_BLEND);
     // Angle::GetForwardVec (MathTypes.cpp:102-110)
-    float cp = cosf(-pitch), cy = cosf(yaw), sy = sinf(yaw), sp = sinf(-pitch);
+    float cp = m_cos(-pitch), cy = m_cos(yaw), sy = m_sin(yaw), sp = m_sin(-pitch);
     V3 dir = v3(cp * cy, cp * sy, -sp);
     ball.b.vel = (dir * new_speed) * UU_TO_BT;
     ball.hs_time += dt;

@@ -1,0 +1,92 @@
+// Host run of the team tick (rocketsim_amd/csrc/rsg_team.h), phase by phase
+// and lane by lane, as the cooperative kernel's lanes run it; th_step of
+// tick_host.cpp with the phases in place of arena_tick.
+#include <memory>
+#include <vector>
+#define th_step th_step_serial
+#include "tick_host.cpp"
+#undef th_step
+#include "../../rocketsim_amd/csrc/rsg_team.h"
+
+namespace {
+// The lanes run last to first in every phase (none depends on another's).
+template <class F>
+void each_lane(ArenaLocal& A, const ArenaGeom* geo, unsigned char* local, int max_cars, TeamGlobal* g, int lanes, F&& f) {
+    for (int k = lanes - 1; k >= 0; k--) {
+        Team t(A, geo, local, max_cars, g, k, lanes);
+        f(t);
+    }
+}
+}  // namespace
+
+void team_tick(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, unsigned char* local, int max_cars,
+               TeamGlobal* g, int lanes) {
+    auto each = [&](auto&& f) { each_lane(A, geo, local, max_cars, g, lanes, f); };
+    TeamHead* h = reinterpret_cast<TeamHead*>(local);
+    each([&](Team& t) { t.begin(P); });
+    Team t0(A, geo, local, max_cars, g, 0, lanes);
+    const bool respawn = t0.any_respawn();
+    if (!respawn) each([&](Team& t) { t.rays(-1); });
+    const bool together = !respawn && t0.independent();
+    for (int pass = 0; pass < t0.car_passes(together); pass++) {
+        each([&](Team& t) { t.car_begin(P, together, pass); });
+        if (respawn) each([&](Team& t) { t.rays(pass); });
+        each([&](Team& t) { t.wheels(P, together, pass); });
+        each([&](Team& t) { t.car(P, together, pass); });
+    }
+    each([&](Team& t) { t.body_begin(P); });
+    each([&](Team& t) { t.ranks(); });
+    each([&](Team& t) { t.pairs(); });
+    each([&](Team& t) { t.trim(); });
+    each([&](Team& t) { t.drop_pairs(); });
+    each([&](Team& t) { t.plan(); });
+    EpaSmall small;
+    each([&](Team& t) { t.narrow(0, &small); });
+    each([&](Team& t) { t.narrow(1, &small); });
+    each([&](Team& t) { t.rows(); });
+    const int n = h->n_rows;
+    std::vector<TeamRow> rows((size_t)n);
+    for (int r = 0; r < n; r++) t0.row_setup(r, P.dt, rows[(size_t)r]);
+    auto visit = [&](int what) {
+        bool moved = false;
+        for (int lv = 0; lv < h->n_levels; lv++)
+            for (int r = n - 1; r >= 0; r--)
+                if (h->row.level[r] == lv) {
+                    const float q = t0.row_visit(rows[(size_t)r], what);
+                    moved |= !(q * q <= 0.f);
+                }
+        return moved;
+    };
+    for (int it = 0; it < SOLVER_ITERATIONS; it++)
+        if (!visit(0)) break;
+    for (int it = 0; it < SOLVER_ITERATIONS; it++) {
+        visit(1);
+        visit(2);
+    }
+    each([&](Team& t) { t.body_end(P); });
+    each([&](Team& t) { t.pads(P); });
+    each([&](Team& t) { t.end(P); });
+}
+
+extern "C" void th_step(void* p, int ticks) {
+    HostBatch& h = *(HostBatch*)p;
+    const ArenaGeom mv = h.geo.geom();
+    const ArenaGeom* mp = mode_has_arena(h.dev.mode) ? &mv : nullptr;
+    auto A = std::make_unique<ArenaLocal>();
+    auto g = std::make_unique<ArenaSpace>();
+    const int max_cars = h.dev.max_cars, lanes = 4 * max_cars < 12 ? 12 : 4 * max_cars;
+    std::vector<uint64_t> local(team_local_bytes(max_cars) / 8 + 1);
+    for (int a = 0; a < h.dev.n; a++) {
+        load_arena(h.dev, a, *A);
+        TickParams P;
+        P.mode = h.dev.mode;
+        P.dt = h.dev.tick_time;
+        P.seed = h.dev.seed;
+        P.arena_id = (uint32_t)a;
+        P.synth_controls = h.dev.synth_controls != 0;
+        P.auto_reset = h.dev.auto_reset != 0;
+        for (int t = 0; t < ticks; t++)
+            team_tick(*A, P, mp, (unsigned char*)local.data(), max_cars, reinterpret_cast<TeamGlobal*>(g.get()), lanes);
+        store_arena(h.dev, a, *A);
+    }
+}

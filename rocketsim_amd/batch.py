@@ -7,6 +7,8 @@ the get/set methods replace Car/Ball/BoostPad Get/SetState.
 """
 import ctypes as C
 
+import numpy as np
+
 from . import native
 from .state import (ARENA_MODES, ArenaSnapshot, BallState, BatchDesc, BoostPadConfig, CarState, Controls, Event, MODE_HEATSEEKER,
                     MODE_HOOPS, MODE_SOCCAR, MODE_THE_VOID,
@@ -75,6 +77,20 @@ def deserialize_snapshot(data):
     out = ArenaSnapshot()
     native.check(native.lib().rsg_snapshot_deserialize(bytes(data), len(data), C.byref(out)))
     return out
+
+
+def _records(record, n):
+    """An array of n records for a getter to fill.  A large one lies in memory
+    that is not cleared first."""
+    size = n * C.sizeof(record)
+    if size < 1 << 20:
+        return (record * n)()
+    return (record * n).from_buffer(np.empty(size, np.uint8))
+
+
+def _array(record, n, values):
+    """`values` as an array of n records: itself if it is one, else a copy."""
+    return values if isinstance(values, record * n) else (record * n)(*values)
 
 
 class ArenaBatch:
@@ -156,34 +172,34 @@ class ArenaBatch:
 
     # -- state ------------------------------------------------------------
     def get_cars(self):
-        out = (CarState * max(self.n_cars, 1))()
+        out = _records(CarState, max(self.n_cars, 1))
         native.check(self.L.rsg_batch_get_cars(self.h, out))
         return out
 
     def set_cars(self, states):
-        arr = (CarState * max(self.n_cars, 1))(*states)
+        arr = _array(CarState, max(self.n_cars, 1), states)
         native.check(self.L.rsg_batch_set_cars(self.h, arr))
 
     def get_balls(self):
-        out = (BallState * self.n_arenas)()
+        out = _records(BallState, self.n_arenas)
         native.check(self.L.rsg_batch_get_balls(self.h, out))
         return out
 
     def set_balls(self, states):
-        arr = (BallState * self.n_arenas)(*states)
+        arr = _array(BallState, self.n_arenas, states)
         native.check(self.L.rsg_batch_set_balls(self.h, arr))
 
     def get_pads(self):
-        out = (PadState * (NUM_PADS * self.n_arenas))()
+        out = _records(PadState, NUM_PADS * self.n_arenas)
         native.check(self.L.rsg_batch_get_pads(self.h, out))
         return out
 
     def set_pads(self, states):
-        arr = (PadState * (NUM_PADS * self.n_arenas))(*states)
+        arr = _array(PadState, NUM_PADS * self.n_arenas, states)
         native.check(self.L.rsg_batch_set_pads(self.h, arr))
 
     def set_controls(self, controls):
-        arr = (Controls * max(self.n_cars, 1))(*controls)
+        arr = _array(Controls, max(self.n_cars, 1), controls)
         native.check(self.L.rsg_batch_set_controls(self.h, arr))
 
     def get_controls(self):

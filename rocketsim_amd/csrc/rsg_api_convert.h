@@ -2,7 +2,8 @@
 // (include/rsg_state.h, public units: uu, uu/s, column-major RotMat) and the
 // word-plane records in memory (Bullet units, basis rows), as the reference's
 // Car/Ball Get/SetState convert (src/Sim/Car/Car.cpp:10-36,
-// src/Sim/Ball/Ball.cpp:27-51).  Host code only.
+// src/Sim/Ball/Ball.cpp:27-51).  The reads also run on the device
+// (rsg_k_records.hip); the rest is host code.
 #pragma once
 
 #include <cmath>
@@ -18,7 +19,7 @@ inline void rot_api_to_rows(const float* api, M3& m) {
     // api: forward, right, up columns (RotMat, src/Math/MathTypes/MathTypes.h:169-170)
     for (int r = 0; r < 3; r++) m.r[r] = v3(api[0 + r], api[3 + r], api[6 + r]);
 }
-inline void rot_rows_to_api(const M3& m, float* api) {
+RSG_FN void rot_rows_to_api(const M3& m, float* api) {
     for (int r = 0; r < 3; r++) {
         api[0 + r] = m.r[r].x;
         api[3 + r] = m.r[r].y;
@@ -26,20 +27,20 @@ inline void rot_rows_to_api(const M3& m, float* api) {
     }
 }
 
-inline Ctrl ctrl_from_api(const rsg_controls& c) {
+RSG_FN Ctrl ctrl_from_api(const rsg_controls& c) {
     Ctrl o;
     o.throttle = c.throttle; o.steer = c.steer; o.pitch = c.pitch; o.yaw = c.yaw; o.roll = c.roll;
     o.jump = c.jump != 0; o.boost = c.boost != 0; o.handbrake = c.handbrake != 0;
     return o;
 }
-inline rsg_controls ctrl_to_api(const Ctrl& c) {
+RSG_FN rsg_controls ctrl_to_api(const Ctrl& c) {
     rsg_controls o;
     o.throttle = c.throttle; o.steer = c.steer; o.pitch = c.pitch; o.yaw = c.yaw; o.roll = c.roll;
     o.jump = c.jump; o.boost = c.boost; o.handbrake = c.handbrake; o._pad = 0;
     return o;
 }
 
-inline void car_to_api(const CarRef& r, rsg_car_state& s) {
+RSG_FN void car_to_api(const CarRef& r, rsg_car_state& s) {
     Car c;
     load_car(r, c);
     std::memset(&s, 0, sizeof(s));
@@ -113,7 +114,7 @@ inline void car_from_api(const CarRef& r, const rsg_car_state& s) {
     r.u(CW_BP_SEQ) = s.bp_seq;
 }
 
-inline void ball_to_api(const CarRef& r, rsg_ball_state& s) {
+RSG_FN void ball_to_api(const CarRef& r, rsg_ball_state& s) {
     std::memset(&s, 0, sizeof(s));
     V3 p = r.v(BW_POS) * BT_TO_UU, v = r.v(BW_VEL) * BT_TO_UU, w = r.v(BW_ANGVEL);
     s.pos[0] = p.x; s.pos[1] = p.y; s.pos[2] = p.z;
@@ -333,7 +334,7 @@ inline void init_arena_record(const BatchDev& h, int a, int n_cars, const uint8_
         for (int p = 0; p < PAD_NUM; p++) pad_ref(h, a, p).u(PW_ACTIVE) = 1;
 }
 
-inline void pad_to_api(const CarRef& r, rsg_pad_state& s) {
+RSG_FN void pad_to_api(const CarRef& r, rsg_pad_state& s) {
     s.is_active = r.u(PW_ACTIVE);
     s.cooldown = r.f(PW_COOLDOWN);
     s.prev_locked_car_id = r.u(PW_PREV_LOCKED);

@@ -13,11 +13,15 @@
 //   rsg_shot_forward_kernel,    differentiable aerial shot (rsg_shot.h):
 //   rsg_shot_backward_kernel    rollout with checkpoints; backward with one
 //                               lane per tangent input of each pair
+//   rsg_records_read_kernel,    public records of cars, balls and pads out of
+//   rsg_controls_write_kernel   the word planes; controls into them
 //   rsg_game_events_kernel      GameEventTracker (rsg_game_events.h)
 //   rsg_reset_kernel            kickoff reset of one / all arenas
 //
-// Host side keeps a mirror of the SoA state for the get/set API; it is
-// uploaded lazily before the next step and downloaded lazily on the next get.
+// After a step, the cars, balls and pads are read through the records kernel,
+// and controls go in through theirs.  The rest of the get/set API works on a
+// host mirror of the SoA state, downloaded when it is older than the device's
+// and uploaded before the next step.
 
 #include <hip/hip_runtime.h>
 
@@ -27,6 +31,7 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/rsg.h"
@@ -152,6 +157,13 @@ struct rsg_batch {
     bool host_dirty = false;  // host mirror newer than device
     bool dev_newer = false;   // device newer than host mirror
     hipStream_t last_stream = nullptr;
+    int32_t* car_at = nullptr;          // arena << 4 | slot of each car (launch_records_read)
+    unsigned char* records = nullptr;   // pinned: what the records kernel writes
+    size_t records_bytes = 0;
+    bool records_fresh = false;         // they hold every record of the device's state (small batches)
+    rsg_controls* controls = nullptr;   // pinned: the controls set last
+    bool controls_pending = false;      // they are newer than the mirror's and the device's
+    bool synced = false;                // no device work of this batch since the device was waited for
     int arenas_per_block = 0;  // 0: derived from the device's SIMD count
     int kernel = RSG_KERNEL_AUTO;
     bool strict = false;       // fail a step that leaves an arena with a status bit set
@@ -183,19 +195,71 @@ BatchDev host_view(rsg_batch* b) {
     return h;
 }
 
-int upload(rsg_batch* b) {
-    if (!b->host_dirty) return 0;
-    HIP_OK(hipMemcpy(b->dev.car, b->h_car.data(), car_words(b) * 4, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(b->dev.ball, b->h_ball.data(), ball_words(b) * 4, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(b->dev.pad, b->h_pad.data(), pad_words(b) * 4, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(b->dev.arena, b->h_arena.data(), arena_words(b) * 4, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(const_cast<rsg_mutator_config*>(b->dev.mut), b->h_mut.data(),
-                     b->h_mut.size() * sizeof(rsg_mutator_config), hipMemcpyHostToDevice));
-    b->host_dirty = false;
+// The device's state has changed, or will have on `s`.
+void ran_on(rsg_batch* b, hipStream_t s) {
+    b->last_stream = s;
+    b->dev_newer = true;
+    b->records_fresh = false;
+    b->synced = false;
+}
+
+void mirror_controls(rsg_batch* b, const rsg_controls* in) {
+    BatchDev h = host_view(b);
+    for (int a = 0; a < b->dev.n; a++)
+        for (int i = 0; i < b->cars_per_arena[a]; i++)
+            store_ctrl(car_ref(h, a, i), CW_CTRL, ctrl_from_api(in[b->car_offset[a] + i]));
+    b->host_dirty = true;
+}
+
+// Controls set since the last launch, to the device ahead of the next work on
+// `s`.  rsg_batch_set_controls waits for the device before it writes to the
+// staging memory again.
+int flush_controls(rsg_batch* b, hipStream_t s) {
+    HIP_OK(launch_controls_write(b->dev, b->car_at, b->controls, b->total_cars, s));
+    b->controls_pending = false;
+    b->dev_newer = true;
+    b->synced = false;
     return 0;
 }
 
+int upload(rsg_batch* b) {
+    if (b->host_dirty) {
+        HIP_OK(hipMemcpy(b->dev.car, b->h_car.data(), car_words(b) * 4, hipMemcpyHostToDevice));
+        HIP_OK(hipMemcpy(b->dev.ball, b->h_ball.data(), ball_words(b) * 4, hipMemcpyHostToDevice));
+        HIP_OK(hipMemcpy(b->dev.pad, b->h_pad.data(), pad_words(b) * 4, hipMemcpyHostToDevice));
+        HIP_OK(hipMemcpy(b->dev.arena, b->h_arena.data(), arena_words(b) * 4, hipMemcpyHostToDevice));
+        HIP_OK(hipMemcpy(const_cast<rsg_mutator_config*>(b->dev.mut), b->h_mut.data(),
+                         b->h_mut.size() * sizeof(rsg_mutator_config), hipMemcpyHostToDevice));
+        b->host_dirty = false;
+    }
+    if (b->controls_pending) {
+        if (flush_controls(b, nullptr) != 0) return -1;
+        HIP_OK(hipStreamSynchronize(nullptr));
+    }
+    return 0;
+}
+
+// The same ahead of a step on `s`: the controls go in on the step's stream,
+// except while it records a graph, into which they do not belong (the wait of
+// the other way is refused there).
+int upload_for_step(rsg_batch* b, hipStream_t s) {
+    if (!b->host_dirty && b->controls_pending) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_OK(hipStreamIsCapturing(s, &cap));
+        if (cap == hipStreamCaptureStatusNone) return flush_controls(b, s);
+    }
+    return upload(b);
+}
+
 int download(rsg_batch* b) {
+    if (b->controls_pending) {
+        if (b->dev_newer) {
+            if (upload(b) != 0) return -1;
+        } else {
+            mirror_controls(b, b->controls);
+            b->controls_pending = false;
+        }
+    }
     if (!b->dev_newer) return 0;
     if (b->last_stream) HIP_OK(hipStreamSynchronize(b->last_stream));
     HIP_OK(hipDeviceSynchronize());
@@ -204,6 +268,106 @@ int download(rsg_batch* b) {
     HIP_OK(hipMemcpy(b->h_pad.data(), b->dev.pad, pad_words(b) * 4, hipMemcpyDeviceToHost));
     HIP_OK(hipMemcpy(b->h_arena.data(), b->dev.arena, arena_words(b) * 4, hipMemcpyDeviceToHost));
     b->dev_newer = false;
+    b->synced = true;
+    return 0;
+}
+
+enum RecordKind { REC_CARS, REC_BALLS, REC_PADS };
+
+size_t record_bytes(RecordKind kind) {  // of one car, one ball, one arena's pads
+    return kind == REC_CARS ? sizeof(rsg_car_state)
+         : kind == REC_BALLS ? sizeof(rsg_ball_state) : PAD_NUM * sizeof(rsg_pad_state);
+}
+int record_count(const rsg_batch* b, RecordKind kind) { return kind == REC_CARS ? b->total_cars : b->dev.n; }
+
+// Large copies into memory that is often not yet backed by pages are shared by
+// a few threads, 2 MB or more each (38 MB of cars: 1.6 ms with the read, where
+// one thread's copy alone takes 4).
+void copy_out(void* dst, const void* src, size_t bytes) {
+    constexpr size_t SHARE = (size_t)2 << 20;
+    constexpr int MOST = 8;
+    const int parts = (int)std::min<size_t>(MOST, bytes / SHARE);
+    auto copy = [=](int i) {
+        const size_t a = bytes / parts * i / 4096 * 4096, e = i + 1 == parts ? bytes : bytes / parts * (i + 1) / 4096 * 4096;
+        std::memcpy(static_cast<char*>(dst) + a, static_cast<const char*>(src) + a, e - a);
+    };
+    if (parts < 2) {
+        std::memcpy(dst, src, bytes);
+        return;
+    }
+    std::thread t[MOST];
+    int started = 1;
+    try {
+        for (; started < parts; started++) t[started] = std::thread(copy, started);
+    } catch (const std::exception&) {  // no more threads: the rest is done here
+    }
+    copy(0);
+    for (int i = started; i < parts; i++) copy(i);
+    for (int i = 1; i < started; i++) t[i].join();
+}
+
+// Records of one kind from the device's state, which is newer than the mirror.
+// Converted on the device and written to pinned memory, then copied: 2v2 x
+// 4096 arenas 0.39 ms for all three kinds, where copying the word planes into
+// the mirror and converting them on the CPU took 13 ms and more; one 1v1 arena
+// 13 us, once, against four copies.
+// A batch whose records take up to SMALL bytes has them all read in one launch
+// by the first getter after a step, as one launch and one wait cost more than
+// the records; a larger one has each kind read by its getter, RECORDS_MAX bytes
+// at a time.
+int read_records(rsg_batch* b, RecordKind kind, void* out) {
+    constexpr size_t SMALL = (size_t)256 << 10, RECORDS_MAX = (size_t)64 << 20;
+    size_t at[3], all = 0, largest = 0;
+    for (int k = 0; k < 3; k++) {
+        const size_t bytes = record_bytes((RecordKind)k) * (size_t)record_count(b, (RecordKind)k);
+        at[k] = all;
+        all += (bytes + 15) & ~(size_t)15;
+        largest = std::max(largest, bytes);
+    }
+    const bool together = all <= SMALL;
+    const size_t one = record_bytes(kind), n = (size_t)record_count(b, kind);
+    if (!b->records) {
+        const size_t bytes = together ? all : std::min(largest, RECORDS_MAX);
+        HIP_OK(hipHostMalloc((void**)&b->records, bytes, hipHostMallocDefault));
+        b->records_bytes = bytes;
+    }
+    auto launch = [&](RecordsOut o) -> int {
+        HIP_OK(launch_records_read(b->dev, b->car_at, o, b->last_stream));
+        HIP_OK(hipDeviceSynchronize());
+        b->synced = true;
+        return 0;
+    };
+    if (together) {
+        if (!b->records_fresh) {
+            RecordsOut o;
+            o.cars = reinterpret_cast<rsg_car_state*>(b->records + at[REC_CARS]);
+            o.balls = reinterpret_cast<rsg_ball_state*>(b->records + at[REC_BALLS]);
+            o.pads = reinterpret_cast<rsg_pad_state*>(b->records + at[REC_PADS]);
+            o.n_cars = b->total_cars;
+            o.n_balls = o.n_pad_arenas = b->dev.n;
+            if (launch(o) != 0) return -1;
+            b->records_fresh = true;
+        }
+        std::memcpy(out, b->records + at[kind], one * n);
+        return 0;
+    }
+    const size_t most = b->records_bytes / one;
+    for (size_t first = 0; first < n; first += most) {
+        const int count = (int)std::min(most, n - first);
+        RecordsOut o;
+        if (kind == REC_CARS) {
+            o.cars = reinterpret_cast<rsg_car_state*>(b->records);
+            o.first_car = (int)first, o.n_cars = count;
+        } else if (kind == REC_BALLS) {
+            o.balls = reinterpret_cast<rsg_ball_state*>(b->records);
+            o.first_ball = (int)first, o.n_balls = count;
+        } else {
+            o.pads = reinterpret_cast<rsg_pad_state*>(b->records);
+            o.first_pad_arena = (int)first, o.n_pad_arenas = count;
+        }
+        if (launch(o) != 0) return -1;
+        copy_out(static_cast<char*>(out) + first * one, b->records, (size_t)count * one);
+    }
     return 0;
 }
 
@@ -328,6 +492,9 @@ rsg_batch* rsg_batch_create(const rsg_batch_desc* desc) {
     b->h_arena.assign(arena_words(b), 0);
     b->h_mut.assign((size_t)b->dev.n, desc->mutators ? *desc->mutators : mutator_defaults(b->dev.mode));
     hipError_t e = hipSuccess;
+    std::vector<int32_t> car_at;
+    for (int a = 0; a < b->dev.n; a++)
+        for (int i = 0; i < b->cars_per_arena[a]; i++) car_at.push_back(a << 4 | i);
     std::vector<CarPhys> phys;
     for (const rsg_car_config& c : b->h_cfgs) phys.push_back(make_car_phys(c));
     rsg_mutator_config* dmut = nullptr;
@@ -340,6 +507,11 @@ rsg_batch* rsg_batch_create(const rsg_batch_desc* desc) {
         (e = hipMalloc(&b->d_cfgs, b->h_cfgs.size() * sizeof(rsg_car_config))) != hipSuccess ||
         (e = hipMemcpy(b->d_cfgs, b->h_cfgs.data(), b->h_cfgs.size() * sizeof(rsg_car_config),
                        hipMemcpyHostToDevice)) != hipSuccess ||
+        (total > 0 &&
+         ((e = hipMalloc(&b->car_at, car_at.size() * sizeof(int32_t))) != hipSuccess ||
+          (e = hipMemcpy(b->car_at, car_at.data(), car_at.size() * sizeof(int32_t), hipMemcpyHostToDevice)) != hipSuccess ||
+          (e = hipHostMalloc((void**)&b->controls, (size_t)total * sizeof(rsg_controls), hipHostMallocDefault)) !=
+              hipSuccess)) ||
         (e = hipMalloc(&b->d_phys, phys.size() * sizeof(CarPhys))) != hipSuccess ||
         (e = hipMemcpy(b->d_phys, phys.data(), phys.size() * sizeof(CarPhys), hipMemcpyHostToDevice)) != hipSuccess ||
         (!b->h_custom_pads.empty() &&
@@ -379,6 +551,9 @@ void rsg_batch_destroy(rsg_batch* b) {
     if (b->d_cfgs) (void)hipFree(b->d_cfgs);
     if (b->d_phys) (void)hipFree(b->d_phys);
     if (b->d_custom_pads) (void)hipFree(b->d_custom_pads);
+    if (b->car_at) (void)hipFree(b->car_at);
+    if (b->records) (void)hipHostFree(b->records);
+    if (b->controls) (void)hipHostFree(b->controls);
     if (b->status_partials) (void)hipFree(b->status_partials);
     if (b->dev.ev_buf) (void)hipFree(b->dev.ev_buf);
     if (b->dev.ev_count) (void)hipFree(b->dev.ev_count);
@@ -561,11 +736,10 @@ int rsg_batch_step(rsg_batch* b, int ticks, void* stream) {
     if (!b) return fail("null batch");
     if (ticks < 0) return fail("rsg_batch_step: ticks must be >= 0");
     if (ticks == 0) return 0;
-    if (upload(b) != 0) return -1;
     hipStream_t s = (hipStream_t)stream;
+    if (upload_for_step(b, s) != 0) return -1;
     if (launch_step(b, b->dev, choose_launch(b), ticks, s) != 0) return -1;
-    b->last_stream = s;
-    b->dev_newer = true;
+    ran_on(b, s);
     return check_strict(b, "rsg_batch_step");
 }
 
@@ -682,11 +856,10 @@ int rsg_batch_graph_create(rsg_batch* b, int ticks_per_launch, int launches) {
 int rsg_batch_graph_launch(rsg_batch* b, void* stream) {
     if (!b) return fail("null batch");
     if (!b->graph_exec) return fail("rsg_batch_graph_launch: no graph (call rsg_batch_graph_create)");
-    if (upload(b) != 0) return -1;
     hipStream_t s = (hipStream_t)stream;
+    if (upload_for_step(b, s) != 0) return -1;
     HIP_OK(hipGraphLaunch(b->graph_exec, s));
-    b->last_stream = s;
-    b->dev_newer = true;
+    ran_on(b, s);
     return check_strict(b, "rsg_batch_graph_launch");
 }
 
@@ -831,14 +1004,14 @@ int rsg_batch_reset_kickoff(rsg_batch* b, int arena, uint64_t seed) {
     if (upload(b) != 0) return -1;
     if (download(b) != 0) return -1;
     HIP_OK(launch_reset(b->dev, arena, seed, b->last_stream));
-    b->dev_newer = true;
+    ran_on(b, b->last_stream);
     return 0;
 }
 
 int rsg_batch_get_cars(rsg_batch* b, rsg_car_state* out) {
     if (!b || (!out && b->total_cars > 0)) return fail("rsg_batch_get_cars: null argument");
     if (b->total_cars == 0) return 0;
-    if (download(b) != 0) return -1;
+    if (b->dev_newer) return read_records(b, REC_CARS, out);
     BatchDev h = host_view(b);
     for (int a = 0; a < b->dev.n; a++)
         for (int i = 0; i < b->cars_per_arena[a]; i++)
@@ -862,7 +1035,7 @@ int rsg_batch_set_cars(rsg_batch* b, const rsg_car_state* in) {
 
 int rsg_batch_get_balls(rsg_batch* b, rsg_ball_state* out) {
     if (!b || !out) return fail("rsg_batch_get_balls: null argument");
-    if (download(b) != 0) return -1;
+    if (b->dev_newer) return read_records(b, REC_BALLS, out);
     BatchDev h = host_view(b);
     for (int a = 0; a < b->dev.n; a++) {
         ball_to_api(ball_ref(h, a), out[a]);
@@ -883,7 +1056,7 @@ int rsg_batch_set_balls(rsg_batch* b, const rsg_ball_state* in) {
 
 int rsg_batch_get_pads(rsg_batch* b, rsg_pad_state* out) {
     if (!b || !out) return fail("rsg_batch_get_pads: null argument");
-    if (download(b) != 0) return -1;
+    if (b->dev_newer) return read_records(b, REC_PADS, out);
     BatchDev h = host_view(b);
     for (int a = 0; a < b->dev.n; a++)
         for (int p = 0; p < PAD_NUM; p++) pad_to_api(pad_ref(h, a, p), out[a * PAD_NUM + p]);
@@ -903,12 +1076,18 @@ int rsg_batch_set_pads(rsg_batch* b, const rsg_pad_state* in) {
 int rsg_batch_set_controls(rsg_batch* b, const rsg_controls* in) {
     if (!b || (!in && b->total_cars > 0)) return fail("rsg_batch_set_controls: null argument");
     if (b->total_cars == 0) return 0;
-    if (download(b) != 0) return -1;
-    BatchDev h = host_view(b);
-    for (int a = 0; a < b->dev.n; a++)
-        for (int i = 0; i < b->cars_per_arena[a]; i++)
-            store_ctrl(car_ref(h, a, i), CW_CTRL, ctrl_from_api(in[b->car_offset[a] + i]));
-    b->host_dirty = true;
+    if (b->host_dirty) {
+        mirror_controls(b, in);
+        return 0;
+    }
+    // earlier launches may still read the controls before these
+    if (!b->synced) {
+        if (b->last_stream) HIP_OK(hipStreamSynchronize(b->last_stream));
+        HIP_OK(hipDeviceSynchronize());
+        b->synced = true;
+    }
+    std::memcpy(b->controls, in, (size_t)b->total_cars * sizeof(rsg_controls));
+    b->controls_pending = true;
     return 0;
 }
 
@@ -1419,7 +1598,7 @@ int pred_launch(rsg_ball_pred* p, int kind, const BatchDev* src, hipStream_t s) 
     int stride = pred_stride();
     int grid = (p->n + per - 1) / per;
     HIP_OK(launch_ball_pred(a->dev, mv, d, kind, src ? *src : a->dev, stride, per, grid, s));
-    a->dev_newer = true;
+    ran_on(a, a->last_stream);
     p->last_stream = s;
     p->pending = true;
     return 0;

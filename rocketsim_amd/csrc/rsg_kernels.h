@@ -28,6 +28,23 @@ hipError_t launch_step_coop(const BatchDev& d, const ArenaGeom* geo, int ticks, 
 // Kickoff reset of arena `only_arena` (all arenas when < 0).
 hipError_t launch_reset(const BatchDev& d, int only_arena, uint64_t seed, hipStream_t s);
 
+// Public records (rsg_k_records.hip) of a batch's cars, balls and arenas' pads
+// from `first` on, into device-writable memory aligned to 16 bytes; a count of
+// 0 leaves a kind out.  `car_at`: arena << 4 | slot of each car, in the records'
+// order (device memory).
+struct RecordsOut {
+    rsg_car_state* cars = nullptr;
+    rsg_ball_state* balls = nullptr;
+    rsg_pad_state* pads = nullptr;
+    int first_car = 0, n_cars = 0;
+    int first_ball = 0, n_balls = 0;
+    int first_pad_arena = 0, n_pad_arenas = 0;
+};
+hipError_t launch_records_read(const BatchDev& d, const int32_t* car_at, const RecordsOut& o, hipStream_t s);
+// ... and all cars' controls, from device-readable memory.
+hipError_t launch_controls_write(const BatchDev& d, const int32_t* car_at, const rsg_controls* in, int n,
+                                 hipStream_t s);
+
 // Differentiable rollouts (rsg_k_diff.hip).
 constexpr int AIR_MAX_K = 32;
 hipError_t launch_air_forward(int n, int ticks, int K, float dt, const float* s0, const float* ctrl,

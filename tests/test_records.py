@@ -1,0 +1,77 @@
+"""Reading cars, balls and pads from the device and writing controls to it
+(csrc/rsg_k_records.hip) against the host's conversion of the downloaded
+state: the same bytes, for the smallest batch, ragged ones around a wave's 64
+records, arenas without cars, a batch read in one launch and ones read kind by
+kind and in several pieces; and controls that take the one way or the other."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from rocketsim_amd.batch import ArenaBatch
+from rocketsim_amd.state import Controls, MODE_HEATSEEKER, MODE_HOOPS, MODE_SOCCAR, MODE_THE_VOID
+
+pytestmark = pytest.mark.gpu
+
+
+def _batch(per_arena, mode=MODE_SOCCAR, **kw):
+    teams = sum(([i % 2 for i in range(k)] for k in per_arena), [])
+    return ArenaBatch(list(per_arena), teams, [i % 6 for i in range(len(teams))], mode=mode, seed=7, **kw)
+
+
+def _records(b):
+    return bytes(b.get_cars()), bytes(b.get_balls()), bytes(b.get_pads())
+
+
+@pytest.mark.parametrize("mode,per_arena", [
+    (MODE_SOCCAR, [1]), (MODE_SOCCAR, [0]), (MODE_SOCCAR, [2] * 31 + [3]), (MODE_HOOPS, [0, 6, 1, 3, 2] * 13),
+    (MODE_THE_VOID, [1] * 64), (MODE_HEATSEEKER, [8] * 65 + [0]), (MODE_SOCCAR, [4, 2, 6] * 700),
+    (MODE_SOCCAR, [8] * 26900),   # more than one piece of cars
+], ids=lambda v: str(v) if isinstance(v, int) else f"{len(v)}x{max(v)}")
+def test_device_records_equal_the_mirrors(mode, per_arena):
+    b = _batch(per_arena, mode, synth_controls=True, auto_reset=True, ball_rotation=True)
+    b.step(20 if len(per_arena) > 10000 else 90)
+    got = _records(b)
+    again = _records(b)
+    b.get_goals()               # downloads the mirror, which then serves the getters
+    want = _records(b)
+    for what, x, y, z in zip(("cars", "balls", "pads"), got, again, want):
+        assert x == z, what
+        assert y == z, what + " read again"
+    b.close()
+
+
+@pytest.mark.parametrize("arenas", [1, 33, 1500])
+def test_controls_on_either_way(arenas):
+    def play(mirror):
+        b = _batch([2] * arenas)
+        rng = np.random.default_rng(3)
+        out = []
+        for t in range(6):
+            ctl = (Controls * b.n_cars)()
+            v = np.frombuffer(ctl, dtype=np.dtype(Controls))
+            for f in ("throttle", "steer", "pitch", "yaw", "roll"):
+                v[f] = rng.uniform(-1, 1, b.n_cars)
+            for f in ("jump", "boost", "handbrake"):
+                v[f] = rng.integers(0, 3, b.n_cars)
+            if mirror:
+                b.set_tick_counts(b.get_tick_counts())      # the mirror is the newest now
+            b.set_controls(ctl if t % 2 else list(ctl))
+            if t == 2:
+                b.set_controls(ctl)                         # again before any step
+            if t == 3:
+                out.append(bytes(b.get_controls()))
+            if t == 4:
+                b.set_balls(b.get_balls())                  # the mirror takes them over
+            b.step(3)
+            if t != 1:                                      # once without a read in between
+                out += _records(b)
+            out.append(bytes(b.get_controls()))
+        b.graph_create(2, 2)
+        b.set_controls((Controls * b.n_cars)(*[Controls(throttle=1.0)] * b.n_cars))
+        b.graph_launch()
+        out += _records(b)
+        b.close()
+        return out
+
+    assert play(False) == play(True)

@@ -207,7 +207,6 @@ RSG_FN uint32_t leaf_list_mask(const LeafGrid& g, uint32_t at, uint32_t end, V3 
 // triangle's quantized box contains it, so none is missed).
 template <class CB>
 RSG_FN void mesh_query_aabb(const MeshView& m, V3 qmin_f, V3 qmax_f, CB& cb) {
-    if (mesh_region_empty(m, qmin_f, qmax_f)) return;
     uint32_t at, end;
     const int listed = leaf_list(m.box_grid, qmin_f, qmax_f, at, end);
     if (listed == 0) return;
@@ -223,6 +222,7 @@ RSG_FN void mesh_query_aabb(const MeshView& m, V3 qmin_f, V3 qmax_f, CB& cb) {
         }
         return;
     }
+    if (mesh_region_empty(m, qmin_f, qmax_f)) return;
     uint16_t qmin[3], qmax[3];
     quantize_clamp(m, qmin, qmin_f, 0);
     quantize_clamp(m, qmax, qmax_f, 1);
@@ -276,10 +276,9 @@ template <class CB>
 RSG_FN void mesh_query_ray(const MeshView& m, V3 from, V3 to, CB& cb) {
     const V3 rmin = v3(fminf(from.x, to.x), fminf(from.y, to.y), fminf(from.z, to.z));
     const V3 rmax = v3(fmaxf(from.x, to.x), fmaxf(from.y, to.y), fmaxf(from.z, to.z));
-    if (mesh_region_empty(m, rmin, rmax)) return;
     uint32_t at = 0, end = 0;
     const int listed = leaf_list(m.ray_grid, rmin, rmax, at, end);
-    if (listed == 0) return;
+    if (listed == 0 || (listed < 0 && mesh_region_empty(m, rmin, rmax))) return;
     TreeRay r;
     const V3 dir = safe_normalized(to - from);
     r.from = from;

@@ -148,10 +148,10 @@ struct MeshBoxIter {
         m = mesh; lo = l; hi = h;
         mask = 0; at = end = 0;
         mode = 0;
-        if (mesh_region_empty(*m, lo, hi)) return;
         const int listed = leaf_list(m->box_grid, lo, hi, at, end);
         if (listed == 0) return;
         if (listed > 0) { mode = 1; return; }
+        if (mesh_region_empty(*m, lo, hi)) return;
         mode = 2;
         quantize_clamp(*m, qmin, lo, 0);
         quantize_clamp(*m, qmax, hi, 1);

@@ -5,61 +5,9 @@
 
 #include "rsg_kernels.h"
 #include "rsg_step.h"
-#include "rsg_team.h"
+#include "rsg_team_wave.h"
 
 using namespace rsg;
-
-// Solver of every arena of the wave (Team::row_visit's passes): contact r of
-// an arena on its lane r, both rows in registers; an arena with more contacts
-// than lanes keeps its rows in global memory.  One loop runs the split-impulse
-// passes, then contact and friction rows in turn, level by level, so that a
-// row's update is in the code once.
-__device__ __forceinline__ void team_solve(Team& t, bool live, float dt, uint64_t team_mask) {
-    const int n = live ? t.h->n_rows : 0, levels = live ? t.h->n_levels : 0;
-    if (!__any(n > 0)) return;
-    const bool in_memory = n > t.lanes;
-    TeamRow row;
-    int level = -1;
-    RSG_UNROLL_1
-    for (int r = t.lane; r < n; r += t.lanes) {
-        t.row_setup(r, dt, row);
-        level = t.h->row.level[r];
-        if (in_memory) t.g->rows[r] = row;
-    }
-    int what = 0, it = 0;
-    bool go = n > 0;
-    RSG_UNROLL_1
-    while (true) {
-        bool moved = false;
-        RSG_UNROLL_1
-        for (int lv = 0; __any(go && lv < levels); lv++) {
-            if (go) {
-                RSG_UNROLL_1
-                for (int r = t.lane; r < n; r += t.lanes) {
-                    if ((in_memory ? (int)t.h->row.level[r] : level) != lv) continue;
-                    if (in_memory) row = t.g->rows[r];
-                    const float q = t.row_visit(row, what);
-                    moved |= !(q * q <= 0.f);
-                    if (in_memory) t.g->rows[r] = row;
-                }
-            }
-            __syncthreads();
-        }
-        if (what == 0) {
-            // an arena's split passes end once a pass moves nothing
-            go = go && (__ballot(moved) & team_mask) != 0;
-            if (++it < SOLVER_ITERATIONS && __any(go)) continue;
-            what = 1;
-            it = 0;
-            go = n > 0;
-        } else if (what == 1) {
-            what = 2;
-        } else {
-            if (++it == SOLVER_ITERATIONS) break;
-            what = 1;
-        }
-    }
-}
 
 // `lanes` lanes per arena, at most 64 per workgroup: a workgroup is one wave,
 // so its barriers only order the LDS accesses.

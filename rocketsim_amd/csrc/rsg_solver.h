@@ -267,7 +267,8 @@ struct RowSide {
 };
 
 // The rows' updates over the two sides' velocities (resolveSingleConstraintRow*,
-// btSequentialImpulseConstraintSolver.cpp:136-262).
+// btSequentialImpulseConstraintSolver.cpp:136-262): the impulse's change (0: the
+// row and both sides are as before), of a split-impulse row the residual.
 RSG_FN float row_delta(const SRow& c, float rhs, float applied, const RowSide& A, const RowSide& B) {
     float delta = rhs - applied * c.cfm;
     float d1 = sdot(c.n1, A.lin) + sdot(c.rc1, A.ang);
@@ -286,7 +287,7 @@ RSG_FN float row_lower(SRow& c, RowSide& A, RowSide& B) {
     if (sum < c.lo) { delta = c.lo - c.applied; c.applied = c.lo; }
     else c.applied = sum;
     row_apply(c, delta, A, B);
-    return delta / c.jac_inv;
+    return delta;
 }
 RSG_FN float row_generic(SRow& c, RowSide& A, RowSide& B) {
     float delta = row_delta(c, c.rhs, c.applied, A, B);
@@ -300,7 +301,7 @@ RSG_FN float row_generic(SRow& c, RowSide& A, RowSide& B) {
     delta = upper_less ? delta : upper_min_applied;
     c.applied = upper_less ? app : c.hi;
     row_apply(c, delta, A, B);
-    return delta / c.jac_inv;
+    return delta;
 }
 // The split-impulse row: the sides carry the push and turn velocities.
 RSG_FN float row_split(SRow& c, RowSide& A, RowSide& B) {

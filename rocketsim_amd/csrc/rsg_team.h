@@ -484,6 +484,19 @@ struct Team {
         if (over) h->overflow[p] |= RSG_STATUS_CONTACT_OVERFLOW;
     }
 
+    // Whether any planned manifold can hold a point: false if all are of meshes
+    // with no leaf about the ball.  (Ball-only arenas.)
+    RSG_FN bool ball_meets() {
+        const float r = make_ball_phys(A.ball.radius_uu, A.ball.mass).radius + 0.08f;
+        const V3 lo = A.ball.b.pos - v3(r, r, r), hi = A.ball.b.pos + v3(r, r, r);
+        for (int m = 0; m < h->n_mf; m++) {
+            const int s = -1 - h->mf_b1[m];
+            uint32_t at, end;
+            if (!static_is_mesh(*geo, s) || leaf_list(geo->meshes[s].box_grid, lo, hi, at, end) != 0) return true;
+        }
+        return false;
+    }
+
     // -----------------------------------------------------------------------
     // Narrowphase
 
@@ -970,7 +983,7 @@ struct Team {
         else { body[code].dv = r.lin; body[code].dw = r.ang; }
     }
     // One visit of a row: 0 its split-impulse row, 1 its contact row, 2 its
-    // friction row.  Returns the split row's residual.
+    // friction row.  Returns the split row's residual, the others' change.
     RSG_FN float row_visit(TeamRow& row, int what) {
         if (what == 0 && !(row.c.rhs_pen != 0.f)) return 0.f;
         if (what == 1 && row.c.special) return 0.f;
@@ -980,11 +993,11 @@ struct Team {
         if (what == 0) {
             r = row_split(row.c, a, b);
         } else if (what == 1) {
-            row_lower(row.c, a, b);
+            r = row_lower(row.c, a, b);
         } else {
             row.f.lo = -(row.f.friction * row.c.applied);
             row.f.hi = row.f.friction * row.c.applied;
-            row_generic(row.f, a, b);
+            r = row_generic(row.f, a, b);
         }
         put_side(row.a, what == 0, a);
         put_side(row.b, what == 0, b);

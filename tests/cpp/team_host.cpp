@@ -53,15 +53,15 @@ void team_tick(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, unsigne
             for (int r = n - 1; r >= 0; r--)
                 if (h->row.level[r] == lv) {
                     const float q = t0.row_visit(rows[(size_t)r], what);
-                    moved |= !(q * q <= 0.f);
+                    moved |= what == 0 ? !(q * q <= 0.f) : q != 0.f;
                 }
         return moved;
     };
     for (int it = 0; it < SOLVER_ITERATIONS; it++)
         if (!visit(0)) break;
     for (int it = 0; it < SOLVER_ITERATIONS; it++) {
-        visit(1);
-        visit(2);
+        const bool contacts = visit(1), friction = visit(2);
+        if (!contacts && !friction) break;
     }
     each([&](Team& t) { t.body_end(P); });
     each([&](Team& t) { t.pads(P); });

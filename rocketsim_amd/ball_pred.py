@@ -13,6 +13,7 @@ ball of arena i (its own ball-only arena, as the reference's tracker keeps).
 import ctypes as C
 
 from . import native
+from .batch import _array
 from .state import BallPredView, BallState, MODE_HEATSEEKER, MODE_SOCCAR
 
 
@@ -43,13 +44,13 @@ class BallPredTracker:
     def update_pred_manual(self, cur_ball_states, ticks_since_last_update, stream=None):
         """UpdatePredManual (BallPredTracker.cpp:25-61): one state and one tick
         count per tracker."""
-        cur = (BallState * self.n)(*cur_ball_states)
+        cur = _array(BallState, self.n, cur_ball_states)
         ticks = (C.c_int32 * self.n)(*ticks_since_last_update)
         native.check(self.L.rsg_ball_pred_update_manual(self.h, cur, ticks, stream))
 
     def force_update_all_pred(self, initial_ball_states, stream=None):
         """ForceUpdateAllPred (BallPredTracker.cpp:63-71) for every tracker."""
-        init = (BallState * self.n)(*initial_ball_states)
+        init = _array(BallState, self.n, initial_ball_states)
         native.check(self.L.rsg_ball_pred_force_update(self.h, init, stream))
 
     def pred_data(self, tracker):

@@ -66,24 +66,21 @@ RSG_FN bool pred_matches(const uint32_t* a, size_t sa, const uint32_t* b, size_t
            pred_dist_sq(pred_v3(a, sa, RSG_PRED_ANG_VEL), pred_v3(b, sb, RSG_PRED_ANG_VEL)) < mw * mw;
 }
 
-// Tracker i's update.  kind: PRED_FORCE = ForceUpdateAllPred (:63-71),
-// PRED_MANUAL = UpdatePredManual (:25-61), PRED_FROM_BATCH =
-// UpdatePredFromArena (:18-23) on arena i of `src`.  `pa` holds the trackers'
-// ball-only prediction arenas; `A` is the working copy of arena i.
-RSG_FN void ball_pred_update(const BatchDev& pa, const ArenaGeom* mp, const PredDev& p, int kind, const BatchDev& src,
-                             int i, ArenaLocal& A, StepSpace* ws) {
-    load_arena(pa, i, A);
-    TickParams P;
-    P.mode = pa.mode;
-    P.dt = pa.tick_time;
-    P.seed = pa.seed;
-    P.arena_id = (uint32_t)i;
-    P.synth_controls = false;
-    P.auto_reset = false;
-    const int T = p.T;
-    const size_t s = (size_t)pa.n;
+// What an update of a tracker has to do: the ring's head and its valid rows
+// once the starting row is in place; rows [size, T) are to be predicted.
+struct PredRun {
+    int head, size;
+    bool fresh;      // the whole prediction anew, from the current state
+    bool from_last;  // go on from the last valid row
+    int ticks;       // ticks since the last update
+};
 
-    uint32_t cur[RSG_PRED_WORDS];
+// Tracker i's update, up to its first tick.  kind: PRED_FORCE =
+// ForceUpdateAllPred (:63-71), PRED_MANUAL = UpdatePredManual (:25-61),
+// PRED_FROM_BATCH = UpdatePredFromArena (:18-23) on arena i of `src`.  `cur`
+// becomes the current state's record.
+RSG_FN PredRun pred_begin(const PredDev& p, int kind, const BatchDev& src, int i, size_t s, uint32_t* cur) {
+    const int T = p.T;
     int k = 0;
     if (kind == PRED_FROM_BATCH) {
         CarRef br = ball_ref(src, i);
@@ -102,39 +99,66 @@ RSG_FN void ball_pred_update(const BatchDev& pa, const ArenaGeom* mp, const Pred
         for (int w = 0; w < RSG_PRED_WORDS; w++) cur[w] = p.cur[w * s + i];
         if (kind == PRED_MANUAL) k = p.ticks[i];
     }
-
+    const uint32_t* traj = p.traj + i;
+    const size_t row_words = (size_t)RSG_PRED_WORDS * s;
+    PredRun r{p.head[i], p.size[i], true, false, k};
+    if (kind != PRED_FORCE && k >= 0 && k < r.size &&
+        pred_matches(traj + (size_t)((r.head + k) % T) * row_words, s, cur, 1)) {
+        r.fresh = false;
+        if (k > 0) {
+            // drop the k oldest ticks, predict k new ones from the last
+            r.head = (r.head + k) % T;
+            r.size -= k;
+            r.from_last = true;
+        }
+    }
+    return r;
+}
+// The ball, and a fresh prediction's first row, from which the ticks go on.
+RSG_FN void pred_start(const PredDev& p, PredRun& r, int i, size_t s, const uint32_t* cur, Ball& ball) {
     uint32_t* traj = p.traj + i;
     const size_t row_words = (size_t)RSG_PRED_WORDS * s;
-    int head = p.head[i], size = p.size[i];
-    bool full = true;
-    if (kind != PRED_FORCE && k >= 0 && k < size) {
-        if (pred_matches(traj + (size_t)((head + k) % T) * row_words, s, cur, 1)) {
-            full = false;
-            if (k > 0) {
-                // drop the k oldest ticks, predict k new ones from the last
-                head = (head + k) % T;
-                size -= k;
-                pred_set(A.ball, traj + (size_t)((head + size - 1) % T) * row_words, s);
-                for (; size < T; size++) {
-                    arena_tick(A, P, mp, ws);
-                    pred_put(traj + (size_t)((head + size) % T) * row_words, s, A.ball);
-                }
-            }
-        }
-    }
-    if (full) {
-        pred_set(A.ball, cur, 1);
-        uint32_t* r0 = traj + (size_t)head * row_words;
+    if (r.fresh) {
+        pred_set(ball, cur, 1);
+        uint32_t* r0 = traj + (size_t)r.head * row_words;
         for (int w = 0; w < RSG_PRED_WORDS; w++) r0[w * s] = cur[w];
-        for (int t = 1; t < T; t++) {
-            arena_tick(A, P, mp, ws);
-            pred_put(traj + (size_t)((head + t) % T) * row_words, s, A.ball);
-        }
-        size = T;
+    } else if (r.from_last) {
+        pred_set(ball, traj + (size_t)((r.head + r.size - 1) % p.T) * row_words, s);
     }
-    if (kind != PRED_FORCE) p.last[i] = (int32_t)((uint32_t)p.last[i] + (uint32_t)k);
-    p.head[i] = head;
-    p.size[i] = size;
+}
+RSG_FN void pred_end(const PredDev& p, int kind, const PredRun& r, int i) {
+    if (kind != PRED_FORCE) p.last[i] = (int32_t)((uint32_t)p.last[i] + (uint32_t)r.ticks);
+    p.head[i] = r.head;
+    p.size[i] = r.fresh || r.from_last ? p.T : r.size;
+}
+RSG_FN TickParams pred_tick_params(const BatchDev& pa, int i) {
+    TickParams P;
+    P.mode = pa.mode;
+    P.dt = pa.tick_time;
+    P.seed = pa.seed;
+    P.arena_id = (uint32_t)i;
+    P.synth_controls = false;
+    P.auto_reset = false;
+    return P;
+}
+
+// The whole update by one lane, as host builds run it.  `pa` holds the
+// trackers' ball-only prediction arenas; `A` is the working copy of arena i.
+RSG_FN void ball_pred_update(const BatchDev& pa, const ArenaGeom* mp, const PredDev& p, int kind, const BatchDev& src,
+                             int i, ArenaLocal& A, StepSpace* ws) {
+    load_arena(pa, i, A);
+    const TickParams P = pred_tick_params(pa, i);
+    const int T = p.T;
+    const size_t s = (size_t)pa.n;
+    uint32_t cur[RSG_PRED_WORDS];
+    PredRun r = pred_begin(p, kind, src, i, s, cur);
+    pred_start(p, r, i, s, cur, A.ball);
+    if (r.fresh || r.from_last)
+        for (int t = r.fresh ? 1 : r.size; t < T; t++) {
+            arena_tick(A, P, mp, ws);
+            pred_put(p.traj + i + (size_t)((r.head + t) % T) * RSG_PRED_WORDS * s, s, A.ball);
+        }
+    pred_end(p, kind, r, i);
     store_arena(pa, i, A);
 }
 

@@ -1560,13 +1560,18 @@ struct rsg_ball_pred {
 
 namespace {
 
-int pred_stride() {
-    return (int)((offsetof(ArenaLocal, cars) + 15) & ~(size_t)15);
-}
+// A tracker's LDS: its arena without cars, and its team's block.
+int pred_arena_bytes() { return (int)((offsetof(ArenaLocal, cars) + 15) & ~(size_t)15); }
+int pred_stride() { return (int)((pred_arena_bytes() + team_local_bytes(1) + 15) & ~(size_t)15); }
 
+constexpr int PRED_LANES = 16;
+
+// Trackers per wave: as few as give every SIMD one wave, as a wave waits for
+// its slowest tracker (4096 trackers of 720 ticks at 1, 2, 3, 4 a wave: 36.0,
+// 31.9, 31.3, 34.1 ms; the longest chain of contacts alone takes 28).
 int pred_per_wave(int n) {
     int per = (n + device_simds() - 1) / device_simds();
-    return per < 1 ? 1 : (per > 64 ? 64 : per);
+    return per < 1 ? 1 : per;
 }
 
 int pred_wait(rsg_ball_pred* p) {
@@ -1580,11 +1585,11 @@ int pred_wait(rsg_ball_pred* p) {
 int pred_launch(rsg_ball_pred* p, int kind, const BatchDev* src, hipStream_t s) {
     rsg_batch* a = p->arena;
     if (upload(a) != 0) return -1;
-    ArenaGeom mv{};
+    const ArenaGeom* geo = nullptr;
     if (mode_has_arena(a->dev.mode)) {
         const DeviceArena& ga = g_arenas[arena_kind(a->dev.mode)];
         if (!ga.ready) return fail("rsg_ball_pred: no arena mesh (call rsg_init_mesh first)");
-        mv = ga.geom;
+        geo = ga.dev_geom;
     }
     PredDev d;
     d.traj = p->traj;
@@ -1594,10 +1599,12 @@ int pred_launch(rsg_ball_pred* p, int kind, const BatchDev* src, hipStream_t s) 
     d.cur = p->cur;
     d.ticks = p->ticks;
     d.T = p->T;
+    const int stride = pred_stride();
     int per = p->per_wave > 0 ? p->per_wave : pred_per_wave(p->n);
-    int stride = pred_stride();
-    int grid = (p->n + per - 1) / per;
-    HIP_OK(launch_ball_pred(a->dev, mv, d, kind, src ? *src : a->dev, stride, per, grid, s));
+    per = std::min(per, (int)(LDS_PER_WAVE / (size_t)stride));
+    const int lanes = std::min(64 / per, PRED_LANES);
+    const int grid = (p->n + per - 1) / per;
+    HIP_OK(launch_ball_pred(a->dev, geo, d, kind, src ? *src : a->dev, stride, pred_arena_bytes(), per, lanes, grid, s));
     ran_on(a, a->last_stream);
     p->last_stream = s;
     p->pending = true;

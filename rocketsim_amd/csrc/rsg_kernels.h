@@ -57,9 +57,10 @@ hipError_t launch_shot_forward(int n, int ticks, int K, float dt, const float* s
 hipError_t launch_shot_backward(int n, int ticks, int K, float dt, const float* ctrl, const float* target,
                                 const float* ckpt, const float* dloss, float* dctrl, float* ds0, hipStream_t s);
 
-// Ball prediction (rsg_k_pred.hip): `grid` workgroups of `per_wave` trackers.
-hipError_t launch_ball_pred(const BatchDev& pa, const ArenaGeom& geom, const PredDev& p, int kind, const BatchDev& src,
-                            int stride, int per_wave, int grid, hipStream_t s);
+// Ball prediction (rsg_k_pred.hip): `grid` workgroups of `per_wave` trackers,
+// `lanes` lanes each.  (`geo`: the arena's geometry in device memory, or null.)
+hipError_t launch_ball_pred(const BatchDev& pa, const ArenaGeom* geo, const PredDev& p, int kind, const BatchDev& src,
+                            int stride, int arena_bytes, int per_wave, int lanes, int grid, hipStream_t s);
 
 // GameEventTracker update of every arena (rsg_k_events.hip).
 hipError_t launch_game_events(const BatchDev& d, const GameEventDev& g, const rsg_game_event_config& cfg,

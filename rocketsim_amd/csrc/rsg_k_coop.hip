@@ -95,20 +95,7 @@ rsg_step_arena_coop_kernel(BatchDev d, const ArenaGeom* geo, int ticks, int stri
         }
         if (live) team().plan();
         __syncthreads();
-        // step 0: every lane its manifolds; then the effects, and the pairs that
-        // need the penetration pass, whose LDS space the wave's arenas take in turn
-        int redo_at = 0, redos = 0;
-        RSG_UNROLL_1
-        for (int step = 0; step < 2 || step <= redos; step++) {
-            if (live && (step == 0 || step == redo_at)) team().narrow(step ? 1 : 0, small);
-            __syncthreads();
-            if (step == 0) {
-                const bool redo = live && team().h->any_redo;
-                const uint64_t waiting = __ballot(redo && k == 0);
-                redos = __popcll(waiting);
-                redo_at = redo ? 1 + __popcll(waiting & ((1ull << (slot * lanes)) - 1ull)) : 1;
-            }
-        }
+        team_narrow(team, live, small, team_mask);
         if (live) team().rows();
         __syncthreads();
         {

@@ -88,18 +88,7 @@ rsg_ball_pred_kernel(BatchDev pa, const ArenaGeom* geo, PredDev p, int kind, Bat
         const uint64_t meeting = __ballot(meets);
         if (meeting) {
             const bool in = (meeting & team_mask) != 0;
-            int redo_at = 0, redos = 0;
-            RSG_UNROLL_1
-            for (int step = 0; step < 2 || step <= redos; step++) {
-                if (in && (step == 0 || step == redo_at)) team().narrow(step ? 1 : 0, small);
-                __syncthreads();
-                if (step == 0) {
-                    const bool redo = in && team().h->any_redo;
-                    const uint64_t waiting = __ballot(redo && k == 0);
-                    redos = __popcll(waiting);
-                    redo_at = redo ? 1 + __popcll(waiting & ((1ull << (slot * lanes)) - 1ull)) : 1;
-                }
-            }
+            team_narrow(team, in, small, team_mask);
             if (in) team().rows();
             __syncthreads();
             {

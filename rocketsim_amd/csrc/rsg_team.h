@@ -14,9 +14,13 @@
 //   body_begin   one body per lane: gravity, damping, proxy AABB, cell
 //   ranks, pairs, plan   one body per lane: broadphase order, its pairs, their
 //                manifolds
-//   narrow       one manifold per lane; the contact callbacks' effects recorded
-//   effects      lane 0, in pair order (pairs that need the penetration pass or
-//                more effects than fit run here)
+//   narrow 0     one manifold per lane: planes, two cars
+//   search       in rounds: the cars' contacts with the ball, then each mesh
+//                manifold's triangles, one a lane; the points go in in lane order,
+//                their callbacks' effects recorded
+//   refresh_all  one manifold per lane
+//   narrow 1     lane 0, in pair order: the effects (pairs with more than fit the
+//                record run again here)
 //   rows         lane 0: islands, the contact rows and their levels
 //   solve        one contact (its normal and friction row) per lane
 //   body_end     one body per lane: write-back, integration, post-tick
@@ -53,7 +57,7 @@ struct TeamManifold {
     uint8_t n;
     uint8_t special;   // ball against the world: solved through the averaged row
     uint8_t n_effects;
-    uint8_t redo;      // run again in order (penetration pass, effects past the record)
+    uint8_t redo;      // run again in order (effects past the record)
     TeamPoint p[MAX_POINTS_PER_MANIFOLD];
     int eff_code;      // the first effect (kind | car a << 8), unless car-car
     V3 eff_v;
@@ -90,7 +94,7 @@ struct TeamHead {
     uint8_t on_car[4 * RSG_MAX_CARS];     // wheel rests on a car
     uint8_t order[MAX_BODIES];            // bodies by broadphase rank
     uint8_t overflow[MAX_BODIES];         // RSG_STATUS_* found by a body's lane
-    uint8_t any_redo, any_locked;
+    uint8_t any_locked;
     int8_t mf_b0[MAX_MANIFOLDS], mf_b1[MAX_MANIFOLDS];
     uint8_t im[MAX_MANIFOLDS];            // island manifolds, sorted
     union {
@@ -134,19 +138,21 @@ RSG_COLD_FN void team_apply_effect(ArenaLocal& A, int code, V3 v0, V3 v1) {
 }
 RSG_COLD_FN void team_kickoff(ArenaLocal& A, uint64_t seed, uint32_t arena_id) { arena_kickoff_reset(A, seed, arena_id); }
 
-// The triangles a box meets, one at a time (mesh_query_aabb as an iterator).
+// The triangles a box meets (mesh_query_aabb), handed to a team's lanes: of a
+// leaf list one item a lane and round, of the tree, which serves what the lists
+// do not, one a round to lane 0 (every lane walks it).  The order of the query's report is that of
+// the rounds, and of the lanes within a round.
 struct MeshBoxIter {
     const MeshView* m;
     V3 lo, hi;
     int mode;            // 0: done, 1: leaf list, 2: tree
-    uint32_t at, end, mask;
-    int tri[4];
+    uint32_t at, end;
     uint16_t qmin[3], qmax[3];
     int sub, cur, cur_end;
 
     RSG_FN void start(const MeshView* mesh, V3 l, V3 h) {
         m = mesh; lo = l; hi = h;
-        mask = 0; at = end = 0;
+        at = end = 0;
         mode = 0;
         const int listed = leaf_list(m->box_grid, lo, hi, at, end);
         if (listed == 0) return;
@@ -158,23 +164,22 @@ struct MeshBoxIter {
         sub = -1;
         cur = cur_end = 0;
     }
-    RSG_FN bool next(int& t) {
+    // This lane's triangle of the round, or -1; mode 0 after the last round.
+    RSG_FN int next(int lane, int lanes) {
         if (mode == 1) {
-            while (!mask) {
-                if (at >= end) return false;
-                MeshLeaf leaf[4];
-                mask = leaf_list_mask(m->box_grid, at, end, lo, hi, leaf);
-                for (int r = 0; r < 4; r++) tri[r] = leaf[r].tri;
-                at += 4;
+            int tri = -1;
+            if (at + (uint32_t)lane < end) {
+                const MeshLeaf leaf = m->box_grid.leaves[m->box_grid.items[at + (uint32_t)lane]];
+                if (boxes_touch(leaf.lo, leaf.hi, lo, hi)) tri = leaf.tri;
             }
-            t = pick(__builtin_ctz(mask), tri[0], tri[1], tri[2], tri[3]);
-            mask &= mask - 1u;
-            return true;
+            at += (uint32_t)lanes;
+            if (at >= end) mode = 0;
+            return tri;
         }
-        if (mode == 0) return false;
+        if (mode == 0) return -1;
         while (true) {
             while (cur >= cur_end) {
-                if (++sub >= m->n_subtrees) return false;
+                if (++sub >= m->n_subtrees) { mode = 0; return -1; }
                 const QSubtree& st = m->subtrees[sub];
                 if (!q_overlap(qmin, qmax, st.qmin, st.qmax)) continue;
                 cur = st.root;
@@ -183,9 +188,19 @@ struct MeshBoxIter {
             const QNode& n = m->nodes[cur];
             const bool ov = q_overlap(qmin, qmax, n.qmin, n.qmax), leaf = n.esc_or_tri >= 0;
             cur += ov || leaf ? 1 : -n.esc_or_tri;
-            if (leaf && ov) { t = n.esc_or_tri; return true; }
+            if (leaf && ov) return lane == 0 ? n.esc_or_tri : -1;
         }
     }
+};
+
+// Body 0's side of a manifold, and what the contacts of the pair need.
+struct TeamPair {
+    int b0;
+    float thr, ball_r;
+    bool respond;
+    Xf x0, cx;        // the body's, its box's frame
+    V3 he;            // half extents of the box with its margin
+    V3 amin, amax;
 };
 
 struct Team {
@@ -447,7 +462,7 @@ struct Team {
         const TeamBody& t = body[p];
         const int mine = pop(t.statics_kept) + pop(t.dyn_kept);
         if (p == nb - 1) h->n_mf = n + mine < MAX_MANIFOLDS ? n + mine : MAX_MANIFOLDS;
-        if (p == 0) h->any_redo = h->any_locked = 0;
+        if (p == 0) h->any_locked = 0;
         if (n + mine < MAX_MANIFOLDS) {
             for (uint32_t m = t.statics_kept; m; m &= m - 1u) {
                 h->mf_b0[n] = (int8_t)p;
@@ -523,7 +538,8 @@ struct Team {
     // when the pair runs again in order.
     RSG_FN void effect(TeamManifold& m, int mi, int& n_eff, bool direct, int kind, int a, int b, V3 v0, V3 v1) {
         const int code = kind | (a << 8) | (b << 16);
-        if (direct) { team_apply_effect(A, code, v0, v1); return; }
+        // (the ball's against meshes come first in the pair order and are found in order)
+        if (direct || (kind == EFF_BALL_WORLD && mesh_of(mi))) { team_apply_effect(A, code, v0, v1); return; }
         if (kind == EFF_CAR_WORLD && n_eff > 0) { m.eff_v = v0; return; }  // the flag is set either way, the last normal stays
         if (n_eff >= PAIR_EFFECTS) { m.redo = 1; return; }
         if (n_eff == 0 && kind != EFF_CAR_CAR) {
@@ -538,160 +554,206 @@ struct Team {
         n_eff++;
     }
 
-    // Manifold mi's narrowphase: the pair's contacts come out of one loop (a
-    // plane or the ball gives at most one, a mesh one per triangle, two cars
-    // up to four), so that each algorithm, and adding a point, is in the code
-    // once.  Without work spaces a query that needs the penetration pass marks
-    // the manifold for a second run.
-    RSG_FN void pair(int mi, const EpaWork* first, const EpaWork* second, bool direct) {
-        const int b0 = h->mf_b0[mi], b1 = h->mf_b1[mi];
-        TeamManifold& m = manifold(mi);
-        const float thr = rs_min(w.threshold_of(b0), w.threshold_of(b1));
-        const bool respond = w.has_response(b0) && w.has_response(b1);
-        const int s = -1 - b1;
-        const MeshView* mesh = b1 < 0 && static_is_mesh(*geo, s) ? &geo->meshes[s] : nullptr;
-        {
-            float fa, ra, fb, rb;
-            w.body_material(b0, fa, ra);
-            w.body_material(b1, fb, rb);
-            // combined friction / restitution (btManifoldResult.cpp:56-77), then
-            // the contact callback's own
-            float fr = b1 < 0 ? (fa < fb ? fa : fb) : fa * fb;
-            float re = b1 < 0 ? (ra > rb ? ra : rb) : ra * rb;
-            if (respond && b0 > 0) {
-                if (b1 < 0) { fr = A.mut.car_world_friction; re = A.mut.car_world_restitution; }
-                else if (b1 == 0) { fr = CARBALL_COLLISION_FRICTION; re = CARBALL_COLLISION_RESTITUTION; }
-                else { fr = CARCAR_COLLISION_FRICTION; re = CARCAR_COLLISION_RESTITUTION; }
-            }
-            m.threshold = thr;
-            m.friction = fr;
-            m.restitution = re;
-            m.special = respond && b0 == 0 && b1 < 0;
-            m.redo = 0;
-        }
-        int n_pts = 0, n_eff = 0;
-        const Xf x0 = w.xf_of(b0), x1 = w.xf_of(b1);
-        const float ball_r = make_ball_phys(A.ball.radius_uu, A.ball.mass).radius;
-        // body0's shape and its box
-        Xf cx = x0;
-        V3 he = v3zero();
-        float margin0 = ball_r;
-        V3 amin, amax;
-        if (b0 > 0) {
-            const CarPhys& cp = *A.cars[b0 - 1].phys;
-            cx = w.car_child_xf(b0);
-            margin0 = cp.box_margin;
-            he = cp.box_implicit + v3(margin0, margin0, margin0);
-            const M3 ab = abs_m3(cx.R);
-            const V3 e = v3(dot(ab.r[0], he), dot(ab.r[1], he), dot(ab.r[2], he));
-            amin = cx.t - e;
-            amax = cx.t + e;
+    RSG_FN const MeshView* mesh_of(int mi) {
+        const int b1 = h->mf_b1[mi], s = -1 - b1;
+        return b1 < 0 && static_is_mesh(*geo, s) ? &geo->meshes[s] : nullptr;
+    }
+    // The first mesh manifold from mi on, or -1.
+    RSG_FN int next_mesh(int mi) {
+        for (; mi < h->n_mf; mi++)
+            if (mesh_of(mi)) return mi;
+        return -1;
+    }
+    RSG_FN TeamPair pair_of(int mi) {
+        TeamPair q;
+        q.b0 = h->mf_b0[mi];
+        const int b1 = h->mf_b1[mi];
+        q.thr = rs_min(w.threshold_of(q.b0), w.threshold_of(b1));
+        q.respond = w.has_response(q.b0) && w.has_response(b1);
+        q.x0 = q.cx = w.xf_of(q.b0);
+        q.ball_r = make_ball_phys(A.ball.radius_uu, A.ball.mass).radius;
+        q.he = v3zero();
+        if (q.b0 > 0) {
+            const CarPhys& cp = *A.cars[q.b0 - 1].phys;
+            q.cx = w.car_child_xf(q.b0);
+            q.he = cp.box_implicit + v3(cp.box_margin, cp.box_margin, cp.box_margin);
+            const M3 ab = abs_m3(q.cx.R);
+            const V3 e = v3(dot(ab.r[0], q.he), dot(ab.r[1], q.he), dot(ab.r[2], q.he));
+            q.amin = q.cx.t - e;
+            q.amax = q.cx.t + e;
         } else {
-            const float r = ball_r + 0.08f;
-            amin = x0.t - v3(r, r, r);
-            amax = x0.t + v3(r, r, r);
+            const float r = q.ball_r + 0.08f;
+            q.amin = q.x0.t - v3(r, r, r);
+            q.amax = q.x0.t + v3(r, r, r);
         }
-        MeshBoxIter it;
-        it.mode = 0;
-        if (mesh) it.start(mesh, amin, amax);
+        return q;
+    }
+    // The manifold, empty.
+    RSG_FN void open(int mi, const TeamPair& q) {
+        const int b0 = q.b0, b1 = h->mf_b1[mi];
+        TeamManifold& m = manifold(mi);
+        float fa, ra, fb, rb;
+        w.body_material(b0, fa, ra);
+        w.body_material(b1, fb, rb);
+        // combined friction / restitution (btManifoldResult.cpp:56-77), then
+        // the contact callback's own
+        float fr = b1 < 0 ? (fa < fb ? fa : fb) : fa * fb;
+        float re = b1 < 0 ? (ra > rb ? ra : rb) : ra * rb;
+        if (q.respond && b0 > 0) {
+            if (b1 < 0) { fr = A.mut.car_world_friction; re = A.mut.car_world_restitution; }
+            else if (b1 == 0) { fr = CARBALL_COLLISION_FRICTION; re = CARBALL_COLLISION_RESTITUTION; }
+            else { fr = CARCAR_COLLISION_FRICTION; re = CARCAR_COLLISION_RESTITUTION; }
+        }
+        m.threshold = q.thr;
+        m.friction = fr;
+        m.restitution = re;
+        m.special = q.respond && b0 == 0 && b1 < 0;
+        m.redo = 0;
+        m.n = 0;
+        m.n_effects = 0;
+    }
+    // btManifoldResult::addContactPoint and the contact-added callback: body 1's
+    // point pb, the normal on it and the distance; `tri` of a mesh's contact.
+    RSG_FN void add_point(int mi, const TeamPair& q, V3 n, V3 pb, float dist, bool direct, const MeshView* mesh, int tri) {
+        TeamManifold& m = manifold(mi);
+        const int b0 = q.b0, b1 = h->mf_b1[mi];
+        CPoint p;
+        p.pos_a = pb + n * dist;
+        p.pos_b = pb;
+        p.local_a = xf_inv_apply(q.x0, p.pos_a);
+        p.local_b = xf_inv_apply(w.xf_of(b1), pb);
+        p.normal = n;
+        p.dist = dist;
+        int n_pts = m.n, n_eff = m.n_effects;
+        const int idx = n_pts == MAX_POINTS_PER_MANIFOLD ? replace_point(m, p.local_a, dist) : n_pts++;
+        if (q.respond) {
+            if (b1 < 0) {
+                if (b0 > 0) effect(m, mi, n_eff, direct, EFF_CAR_WORLD, b0 - 1, 0, p.normal, v3zero());
+                else if (A.mode == RSG_MODE_HEATSEEKER) effect(m, mi, n_eff, direct, EFF_BALL_WORLD, 0, 0, p.normal, v3zero());
+            } else if (b1 == 0) {
+                effect(m, mi, n_eff, direct, EFF_CAR_BALL, b0 - 1, 0, p.local_b, v3zero());
+            } else {
+                effect(m, mi, n_eff, direct, EFF_CAR_CAR, b0 - 1, b1 - 1, p.local_a, p.local_b);
+            }
+            if (mesh) adjust_internal_edge(p, *mesh, tri);
+        }
+        TeamPoint& o = m.p[idx];
+        o.la = p.local_a;
+        o.lb = p.local_b;
+        o.n = p.normal;
+        o.dist = p.dist;
+        m.n = (uint8_t)n_pts;
+        m.n_effects = (uint8_t)n_eff;
+    }
+    // Manifold mi opened, with the contacts that need no search: a plane's, at
+    // most one, or two cars' boxes', up to four.  (A mesh's and the ball's
+    // against a car come in the rounds of contact().)
+    RSG_FN void pair(int mi, bool direct) {
+        const int b0 = h->mf_b0[mi], b1 = h->mf_b1[mi];
+        const TeamPair q = pair_of(mi);
+        open(mi, q);
+        if (b1 == 0 || mesh_of(mi)) return;
         BoxBoxContacts bc;
-        bc.n = 0;
+        bc.n = 1;
         if (b1 > 0) {
             // copies for the call out of line: what it takes by reference
             // lives in memory
             const CarPhys& p1 = *A.cars[b1 - 1].phys;
-            const Xf xa = cx, xb = w.car_child_xf(b1);
+            const Xf xa = q.cx, xb = w.car_child_xf(b1);
+            const V3 half = q.he;
             BoxBoxContacts out;
-            box_box(xa, he, xb, p1.box_implicit + v3(p1.box_margin, p1.box_margin, p1.box_margin), out);
+            box_box(xa, half, xb, p1.box_implicit + v3(p1.box_margin, p1.box_margin, p1.box_margin), out);
             bc = out;
         }
-        const int n_items = b1 > 0 ? bc.n : 1;
         RSG_UNROLL_1
-        for (int item = 0;; item++) {
-            V3 n, pb;
-            float dist = 0.f;
-            bool have = false, convex = false;
-            int tri = -1;
-            CShape other;
-            if (mesh) {
-                if (!it.next(tri)) break;
-                V3 v[3];
-                mesh_triangle(*mesh, tri, v);
-                if (!triangle_aabb_overlap(v, amin, amax)) continue;
-                // early out on the triangle's plane, from both sides
-                // (btConvexConcaveCollisionAlgorithm.cpp:86-125)
-                const V3 tn = normalized(cross(v[1] - v[0], v[2] - v[0]));
-                const M3 inv = inverse(cx.R);
-                bool out = false;
-                RSG_UNROLL_1
-                for (int side = 0; side < 2; side++) {
-                    const V3 sn = side ? tn * -1.f : tn;
-                    const V3 d = inv * sn;
-                    V3 lp;
-                    if (b0 > 0) lp = v3(fsel(d.x, he.x, -he.x), fsel(d.y, he.y, -he.y), fsel(d.z, he.z, -he.z));
-                    else lp = (len2(d) < FLT_EPS * FLT_EPS) ? normalized(v3(-1, -1, -1)) * ball_r : ball_r * normalized(d);
-                    const V3 wp = xf_apply(cx, lp);
-                    const float gap = dot(sn, v[0]) - dot(sn, wp);
-                    if (gap > thr) { out = true; break; }
-                }
-                if (out) continue;
-                if (b0 == 0) {
-                    have = World::sphere_triangle_contact(x0.t, ball_r, thr, v, n, pb, dist);
-                } else {
-                    convex = true;
-                    other = shape_triangle(v);
-                }
-            } else {
-                if (item >= n_items) break;
-                if (b1 < 0) {
-                    have = plane_contact(b0, s, cx, he, ball_r, thr, n, pb, dist);
-                } else if (b1 == 0) {
-                    convex = true;
-                    other = shape_sphere(ball_r);
-                } else {
-                    n = bc.normal;
-                    pb = pick(item, bc.point[0], bc.point[1], bc.point[2], bc.point[3]);
-                    dist = pick(item, bc.depth[0], bc.depth[1], bc.depth[2], bc.depth[3]);
-                    have = true;
-                }
-            }
-            if (convex) {
-                const CarPhys& cp = *A.cars[b0 - 1].phys;
-                const CShape box = shape_box(cp.box_implicit, cp.box_margin);
-                float md = box.margin + other.margin + thr;
-                md *= md;
-                const int r = gjk_closest(box, other, cx, x1, md, n, pb, dist, first, second);
-                if (r < 0) { m.redo = 1; break; }
-                have = r > 0;
-            }
-            if (!have || dist > thr) continue;
-            // btManifoldResult::addContactPoint and the contact-added callback
-            CPoint p;
-            p.pos_a = pb + n * dist;
-            p.pos_b = pb;
-            p.local_a = xf_inv_apply(x0, p.pos_a);
-            p.local_b = xf_inv_apply(x1, pb);
-            p.normal = n;
-            p.dist = dist;
-            const int idx = n_pts == MAX_POINTS_PER_MANIFOLD ? replace_point(m, p.local_a, dist) : n_pts++;
-            if (respond) {
-                if (b1 < 0) {
-                    if (b0 > 0) effect(m, mi, n_eff, direct, EFF_CAR_WORLD, b0 - 1, 0, p.normal, v3zero());
-                    else if (A.mode == RSG_MODE_HEATSEEKER) effect(m, mi, n_eff, direct, EFF_BALL_WORLD, 0, 0, p.normal, v3zero());
-                } else if (b1 == 0) {
-                    effect(m, mi, n_eff, direct, EFF_CAR_BALL, b0 - 1, 0, p.local_b, v3zero());
-                } else {
-                    effect(m, mi, n_eff, direct, EFF_CAR_CAR, b0 - 1, b1 - 1, p.local_a, p.local_b);
-                }
-                if (mesh) adjust_internal_edge(p, *mesh, tri);
-            }
-            TeamPoint& q = m.p[idx];
-            q.la = p.local_a;
-            q.lb = p.local_b;
-            q.n = p.normal;
-            q.dist = p.dist;
+        for (int item = 0; item < bc.n; item++) {
+            V3 n = bc.normal, pb = pick(item, bc.point[0], bc.point[1], bc.point[2], bc.point[3]);
+            float dist = pick(item, bc.depth[0], bc.depth[1], bc.depth[2], bc.depth[3]);
+            if (b1 < 0 && !plane_contact(b0, -1 - b1, q.cx, q.he, q.ball_r, q.thr, n, pb, dist)) continue;
+            if (dist > q.thr) continue;
+            add_point(mi, q, n, pb, dist, direct, nullptr, -1);
         }
-        // btPersistentManifold::refreshContactPoints (manifold_refresh)
+    }
+
+    // The rounds in which a team's lanes search contacts.  The first: the lane-th
+    // manifold of a car and the ball, one a lane.  Then a mesh manifold after
+    // the other, its triangles over the lanes.
+    struct Search {
+        int mi;        // the mesh manifold under way; before the first, -1
+        bool more;     // rounds left
+        TeamPair q;    // its pair (in the first round the lane's own)
+        MeshBoxIter it;
+    };
+    // This lane's part of the next round: its manifold, or -1, and triangle
+    // (-1: the ball).
+    RSG_FN int next_search(Search& s, bool first, int& tri) {
+        tri = -1;
+        if (first) {
+            s.mi = -1;
+            s.it.mode = 0;
+            int k = lane;
+            int mine = -1;
+            for (int m = 0; m < h->n_mf; m++)
+                if (h->mf_b1[m] == 0 && k-- == 0) mine = m;
+            s.more = next_mesh(0) >= 0;
+            if (mine >= 0) s.q = pair_of(mine);
+            return mine;
+        }
+        if (s.it.mode == 0) {
+            s.mi = next_mesh(s.mi + 1);
+            s.q = pair_of(s.mi);
+            s.it.start(mesh_of(s.mi), s.q.amin, s.q.amax);
+        }
+        tri = s.it.next(lane, lanes);
+        s.more = s.it.mode != 0 || next_mesh(s.mi + 1) >= 0;
+        return tri >= 0 ? s.mi : -1;
+    }
+    // The lane's contact of the round: the closest points of body 0 (a car's
+    // box, the ball's sphere) and its triangle or the ball.  1: there is one, 0:
+    // none, -1: that takes the penetration pass, and there is no work space.
+    RSG_FN int contact(const TeamPair& q, int mi, int tri, const EpaWork* first, const EpaWork* second, V3& n, V3& pb,
+                       float& dist) {
+        CShape other = shape_sphere(q.ball_r);
+        Xf x1 = xf_ident();
+        if (tri >= 0) {
+            V3 v[3];
+            mesh_triangle(*mesh_of(mi), tri, v);
+            if (!triangle_aabb_overlap(v, q.amin, q.amax)) return 0;
+            // early out on the triangle's plane, from both sides
+            // (btConvexConcaveCollisionAlgorithm.cpp:86-125)
+            const V3 tn = normalized(cross(v[1] - v[0], v[2] - v[0]));
+            const M3 inv = inverse(q.cx.R);
+            RSG_UNROLL_1
+            for (int side = 0; side < 2; side++) {
+                const V3 sn = side ? tn * -1.f : tn;
+                const V3 d = inv * sn;
+                V3 lp;
+                if (q.b0 > 0) lp = v3(fsel(d.x, q.he.x, -q.he.x), fsel(d.y, q.he.y, -q.he.y), fsel(d.z, q.he.z, -q.he.z));
+                else lp = (len2(d) < FLT_EPS * FLT_EPS) ? normalized(v3(-1, -1, -1)) * q.ball_r : q.ball_r * normalized(d);
+                const V3 wp = xf_apply(q.cx, lp);
+                const float gap = dot(sn, v[0]) - dot(sn, wp);
+                if (gap > q.thr) return 0;
+            }
+            if (q.b0 == 0)
+                return World::sphere_triangle_contact(q.x0.t, q.ball_r, q.thr, v, n, pb, dist) && !(dist > q.thr) ? 1 : 0;
+            other = shape_triangle(v);
+        } else {
+            x1 = w.xf_of(0);
+        }
+        const CarPhys& cp = *A.cars[q.b0 - 1].phys;
+        const CShape box = shape_box(cp.box_implicit, cp.box_margin);
+        float md = box.margin + other.margin + q.thr;
+        md *= md;
+        const int r = gjk_closest(box, other, q.cx, x1, md, n, pb, dist, first, second);
+        return r > 0 && dist > q.thr ? 0 : r;
+    }
+
+    // btPersistentManifold::refreshContactPoints (manifold_refresh).
+    RSG_FN void refresh(int mi) {
+        TeamManifold& m = manifold(mi);
+        const float thr = m.threshold;
+        const Xf x0 = w.xf_of(h->mf_b0[mi]), x1 = w.xf_of(h->mf_b1[mi]);
+        int n_pts = m.n;
         RSG_UNROLL_1
         for (int i = n_pts - 1; i >= 0; i--) {
             const TeamPoint p = m.p[i];
@@ -707,8 +769,10 @@ struct Team {
             if (i != n_pts) m.p[i] = m.p[n_pts];
         }
         m.n = (uint8_t)n_pts;
-        m.n_effects = (uint8_t)n_eff;
-        if (m.redo) h->any_redo = 1;
+    }
+    RSG_FN void refresh_all() {
+        RSG_UNROLL_1
+        for (int mi = lane; mi < h->n_mf; mi += lanes) refresh(mi);
     }
 
     // btConvexPlaneCollisionAlgorithm::processCollision for the ball or a
@@ -732,17 +796,16 @@ struct Team {
         return true;
     }
 
-    // Narrowphase pass 0: each lane its share; pass 1 (lane 0): the effects in
-    // pair order, with the marked manifolds run again, their penetration
-    // queries in `small` (or in the arena's global block where that is too
-    // small).
-    RSG_FN void narrow(int pass, EpaSmall* small) {
+    // Pass 0: each lane its share of the manifolds; pass 1 (lane 0): the effects
+    // in pair order, with the manifolds run again that had more than fit the
+    // record.
+    RSG_FN void narrow(int pass) {
         const int n = pass == 0 || lane == 0 ? h->n_mf : 0;
         RSG_UNROLL_1
         for (int mi = pass == 0 ? lane : 0; mi < n; mi += pass == 0 ? lanes : 1) {
             if (pass == 0 || manifold(mi).redo) {
-                const EpaWork first = epa_work(*small), second = epa_work(g->epa);
-                pair(mi, pass == 0 ? nullptr : &first, &second, pass != 0);
+                pair(mi, pass != 0);
+                if (pass != 0) refresh(mi);
                 continue;
             }
             const TeamManifold& m = manifold(mi);

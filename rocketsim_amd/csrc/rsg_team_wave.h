@@ -7,6 +7,62 @@
 
 namespace rsg {
 
+// Narrowphase of every arena of the wave: `team()` gives this lane's team, `on`
+// whether it takes part.  The rounds run for all teams together; a search that
+// needs the penetration pass gets the wave's one work space `small` in turn.
+//
+// What bounds it: the searches, each a chain of dependent loads and
+// arithmetic.  One lane went through a manifold's triangles before, 2 to 10 us
+// each, and ran the whole pair again for a penetration (2v2 x 4096 arenas 0.272
+// ms a tick against 0.194, as a wave waits for its slowest; a ball rolling on
+// the mesh 30 us a tick against 12).
+template <class MakeTeam>
+__device__ __forceinline__ void team_narrow(MakeTeam&& team, bool on, EpaSmall* small, uint64_t team_mask) {
+    if (on) team().narrow(0);
+    __syncthreads();
+    {
+        Team t = team();
+        const int self = (int)threadIdx.x;
+        Team::Search search;
+        search.more = on;
+        bool first = true;
+        RSG_UNROLL_1
+        while (__any(search.more)) {
+            int tri = -1, mi = -1;
+            if (search.more) mi = t.next_search(search, first, tri);
+            first = false;
+            V3 n, pb;
+            float dist = 0.f;
+            int found = 0;
+            uint64_t waiting = 0;
+            // once without the penetration pass, then those that need it in turn
+            RSG_UNROLL_1
+            for (int turn = 0; turn == 0 || waiting; turn++) {
+                if (turn == 0 ? mi >= 0 : self == __builtin_ctzll(waiting)) {
+                    const EpaWork w0 = epa_work(*small), w1 = epa_work(t.g->epa);
+                    found = t.contact(search.q, mi, tri, turn ? &w0 : nullptr, &w1, n, pb, dist);
+                }
+                __syncthreads();
+                waiting = turn == 0 ? __ballot(found < 0) : waiting & (waiting - 1u);
+            }
+            // into the manifolds, each team's lanes in order
+            uint64_t left = __ballot(found > 0) & team_mask;
+            RSG_UNROLL_1
+            while (__any(left != 0)) {
+                if (left && self == __builtin_ctzll(left))
+                    t.add_point(mi, search.q, n, pb, dist, false, tri >= 0 ? t.mesh_of(mi) : nullptr, tri);
+                __syncthreads();
+                left &= left - 1u;
+            }
+        }
+    }
+    __syncthreads();
+    if (on) team().refresh_all();
+    __syncthreads();
+    if (on) team().narrow(1);
+    __syncthreads();
+}
+
 // The levels (rows() in rsg_team.h) on which any of the wave's lanes with `in`
 // has its row, one bit each; bit 63 stands for all from there on.
 __device__ __forceinline__ uint64_t wave_levels(bool in, int level) {

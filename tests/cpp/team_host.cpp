@@ -40,9 +40,33 @@ void team_tick(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, unsigne
     each([&](Team& t) { t.trim(); });
     each([&](Team& t) { t.drop_pairs(); });
     each([&](Team& t) { t.plan(); });
+    each([&](Team& t) { t.narrow(0); });
     EpaSmall small;
-    each([&](Team& t) { t.narrow(0, &small); });
-    each([&](Team& t) { t.narrow(1, &small); });
+    struct Found { int mi, tri, found; V3 n, pb; float dist; };
+    std::vector<Team::Search> search((size_t)lanes);
+    std::vector<Found> f((size_t)lanes);
+    bool first = true, more = true;
+    while (more) {
+        more = false;
+        each([&](Team& t) {
+            Found& o = f[(size_t)t.lane];
+            o.mi = t.next_search(search[(size_t)t.lane], first, o.tri);
+            more |= search[(size_t)t.lane].more;
+            o.found = 0;
+            const EpaWork w0 = epa_work(small), w1 = epa_work(t.g->epa);
+            for (int turn = 0; turn < 2 && o.mi >= 0 && (turn == 0 || o.found < 0); turn++)
+                o.found = t.contact(search[(size_t)t.lane].q, o.mi, o.tri, turn ? &w0 : nullptr, &w1, o.n, o.pb, o.dist);
+        });
+        first = false;
+        for (int k = 0; k < lanes; k++) {
+            if (f[(size_t)k].found <= 0) continue;
+            Team t(A, geo, local, max_cars, g, k, lanes);
+            const Found& o = f[(size_t)k];
+            t.add_point(o.mi, search[(size_t)k].q, o.n, o.pb, o.dist, false, o.tri >= 0 ? t.mesh_of(o.mi) : nullptr, o.tri);
+        }
+    }
+    each([&](Team& t) { t.refresh_all(); });
+    each([&](Team& t) { t.narrow(1); });
     each([&](Team& t) { t.rows(); });
     const int n = h->n_rows;
     std::vector<TeamRow> rows((size_t)n);

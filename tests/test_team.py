@@ -11,9 +11,9 @@ import numpy as np
 import pytest
 
 import tick_host
-from rocketsim_amd import arena_mesh
+from rocketsim_amd import arena_mesh, native
 from rocketsim_amd.state import (ARENA_MODES, BallState, CarState, Controls, MODE_HEATSEEKER, MODE_HOOPS, MODE_SOCCAR,
-                                 MODE_THE_VOID, NUM_PADS, PadState)
+                                 MODE_THE_VOID, MutatorConfig, NUM_PADS, PadState)
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -47,7 +47,7 @@ def _rotations(rng, n):
                      2 * (x * z - y * w), 2 * (y * z + x * w), 1 - 2 * (x * x + y * y)], -1)
 
 
-def _rollout(L, mode, per_team, ticks, seed, rotate_ball=False):
+def _rollout(L, mode, per_team, ticks, seed, rotate_ball=False, ball_radius=None):
     """Every tick's records of one arena per entry of per_team: cars about the
     ball and anywhere, upright and tumbling, under random controls."""
     rng = np.random.default_rng(seed)
@@ -57,8 +57,14 @@ def _rollout(L, mode, per_team, ticks, seed, rotate_ball=False):
     presets = [int(p) for p in rng.integers(0, 7, total)]
     cmfs = [] if mode not in ARENA_MODES else (
         arena_mesh.hoops_cmfs() if mode == MODE_HOOPS else [arena_mesh.soccar_cmf()])
+    mut = None
+    if ball_radius:
+        mut = MutatorConfig()
+        native.check(native.lib().rsg_mutator_config_default(mode, C.byref(mut)))
+        mut.ball_radius = ball_radius
     h = L.th_create(mode, n, (C.c_int * n)(*[2 * k for k in per_team]), (C.c_uint8 * max(total, 1))(*teams),
-                    (C.c_uint8 * max(total, 1))(*presets), *tick_host.mesh_args(cmfs), 120.0, None, None)
+                    (C.c_uint8 * max(total, 1))(*presets), *tick_host.mesh_args(cmfs), 120.0,
+                    C.byref(mut) if mut is not None else None, None)
     if rotate_ball:
         L.th_set_ball_rotation(h, 1)
     cars, balls, ctl = (CarState * max(total, 1))(), (BallState * n)(), (Controls * max(total, 1))()
@@ -116,6 +122,12 @@ def _compare(libs, *args, **kw):
 ])
 def test_phases_match_the_serial_tick(build, mode, per_team, ticks, rotate_ball):
     assert not _compare(build(), mode, per_team, ticks, 1, rotate_ball=rotate_ball).any()
+
+
+@pytest.mark.parametrize("mode", [MODE_SOCCAR, MODE_HOOPS])
+def test_phases_match_where_the_tree_serves_the_ball(build, mode):
+    # a ball whose box the leaf lists do not serve, beside cars that they serve
+    assert not _compare(build(), mode, [0, 1, 2] * 5, 240, 5, ball_radius=240.0).any()
 
 
 @pytest.mark.parametrize("limit", ["RSG_TEST_MAX_MANIFOLDS=1", "RSG_TEST_MAX_MANIFOLDS=2",

@@ -227,6 +227,15 @@ int rsg_air_rollout(int n, int ticks, int ckpt_every, float tick_rate, const flo
 int rsg_air_rollout_backward(int n, int ticks, int ckpt_every, float tick_rate, const float* controls,
                              const float* target, const float* checkpoints, const float* dloss, float* dcontrols,
                              float* dstate0, void* stream);
+/* The same over arrays by car: state [n][13], controls [ticks][n][4], target
+ * [n][7] and their gradients (checkpoints as above).  The rollout also writes,
+ * where not NULL, copies of the controls and the target for the backward pass. */
+int rsg_air_rollout_rows(int n, int ticks, int ckpt_every, float tick_rate, const float* state0, const float* controls,
+                         const float* target, float* state_out, float* loss, float* checkpoints, float* kept_controls,
+                         float* kept_target, void* stream);
+int rsg_air_rollout_rows_backward(int n, int ticks, int ckpt_every, float tick_rate, const float* controls,
+                                  const float* target, const float* checkpoints, const float* dloss, float* dcontrols,
+                                  float* dstate0, void* stream);
 
 /* Differentiable aerial shot: one airborne car and the ball per pair, through
  * the car-ball hit (no counterpart in the reference; the forward model is the

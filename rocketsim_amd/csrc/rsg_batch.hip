@@ -865,30 +865,61 @@ int rsg_batch_graph_launch(rsg_batch* b, void* stream) {
 
 int rsg_batch_graph_ticks(rsg_batch* b) { return b ? b->graph_ticks : fail("null batch"); }
 
+namespace {
+int air_forward(const char* who, bool rows, int n, int ticks, int ckpt_every, float tick_rate, const float* state0,
+                const float* controls, const float* target, float* state_out, float* loss, float* checkpoints,
+                float* kept_controls, float* kept_target, void* stream) {
+    const std::string w(who);
+    if (n < 0 || ticks <= 0) return fail(w + ": need n >= 0 and ticks > 0");
+    if (ckpt_every < 1 || ckpt_every > AIR_MAX_K) return fail(w + ": ckpt_every must be 1..32");
+    if (tick_rate <= 0.f) return fail(w + ": tick_rate must be > 0");
+    if (!state0 || !controls || ((loss || kept_target) && !target)) return fail(w + ": null argument");
+    if (n == 0) return 0;
+    HIP_OK(launch_air_forward(rows, n, ticks, ckpt_every, 1.f / tick_rate, state0, controls, target, state_out, loss,
+                              checkpoints, kept_controls, kept_target, (hipStream_t)stream));
+    return 0;
+}
+
+int air_backward(const char* who, bool rows, int n, int ticks, int ckpt_every, float tick_rate, const float* controls,
+                 const float* target, const float* checkpoints, const float* dloss, float* dcontrols, float* dstate0,
+                 void* stream) {
+    const std::string w(who);
+    if (n < 0 || ticks <= 0) return fail(w + ": need n >= 0 and ticks > 0");
+    if (ckpt_every < 1 || ckpt_every > AIR_MAX_K) return fail(w + ": ckpt_every must be 1..32");
+    if (tick_rate <= 0.f) return fail(w + ": tick_rate must be > 0");
+    if (!controls || !target || !checkpoints || !dloss || !dcontrols) return fail(w + ": null argument");
+    if (n == 0) return 0;
+    HIP_OK(launch_air_backward(rows, n, ticks, ckpt_every, 1.f / tick_rate, controls, target, checkpoints, dloss,
+                               dcontrols, dstate0, (hipStream_t)stream));
+    return 0;
+}
+}  // namespace
+
 int rsg_air_rollout(int n, int ticks, int ckpt_every, float tick_rate, const float* state0, const float* controls,
                     const float* target, float* state_out, float* loss, float* checkpoints, void* stream) {
-    if (n < 0 || ticks <= 0) return fail("rsg_air_rollout: need n >= 0 and ticks > 0");
-    if (ckpt_every < 1 || ckpt_every > AIR_MAX_K) return fail("rsg_air_rollout: ckpt_every must be 1..32");
-    if (tick_rate <= 0.f) return fail("rsg_air_rollout: tick_rate must be > 0");
-    if (!state0 || !controls || (loss && !target)) return fail("rsg_air_rollout: null argument");
-    if (n == 0) return 0;
-    HIP_OK(launch_air_forward(n, ticks, ckpt_every, 1.f / tick_rate, state0, controls, target, state_out, loss,
-                              checkpoints, (hipStream_t)stream));
-    return 0;
+    return air_forward("rsg_air_rollout", false, n, ticks, ckpt_every, tick_rate, state0, controls, target, state_out,
+                       loss, checkpoints, nullptr, nullptr, stream);
+}
+
+int rsg_air_rollout_rows(int n, int ticks, int ckpt_every, float tick_rate, const float* state0, const float* controls,
+                         const float* target, float* state_out, float* loss, float* checkpoints, float* kept_controls,
+                         float* kept_target, void* stream) {
+    return air_forward("rsg_air_rollout_rows", true, n, ticks, ckpt_every, tick_rate, state0, controls, target,
+                       state_out, loss, checkpoints, kept_controls, kept_target, stream);
 }
 
 int rsg_air_rollout_backward(int n, int ticks, int ckpt_every, float tick_rate, const float* controls,
                              const float* target, const float* checkpoints, const float* dloss, float* dcontrols,
                              float* dstate0, void* stream) {
-    if (n < 0 || ticks <= 0) return fail("rsg_air_rollout_backward: need n >= 0 and ticks > 0");
-    if (ckpt_every < 1 || ckpt_every > AIR_MAX_K) return fail("rsg_air_rollout_backward: ckpt_every must be 1..32");
-    if (tick_rate <= 0.f) return fail("rsg_air_rollout_backward: tick_rate must be > 0");
-    if (!controls || !target || !checkpoints || !dloss || !dcontrols)
-        return fail("rsg_air_rollout_backward: null argument");
-    if (n == 0) return 0;
-    HIP_OK(launch_air_backward(n, ticks, ckpt_every, 1.f / tick_rate, controls, target, checkpoints, dloss,
-                               dcontrols, dstate0, (hipStream_t)stream));
-    return 0;
+    return air_backward("rsg_air_rollout_backward", false, n, ticks, ckpt_every, tick_rate, controls, target,
+                        checkpoints, dloss, dcontrols, dstate0, stream);
+}
+
+int rsg_air_rollout_rows_backward(int n, int ticks, int ckpt_every, float tick_rate, const float* controls,
+                                  const float* target, const float* checkpoints, const float* dloss, float* dcontrols,
+                                  float* dstate0, void* stream) {
+    return air_backward("rsg_air_rollout_rows_backward", true, n, ticks, ckpt_every, tick_rate, controls, target,
+                        checkpoints, dloss, dcontrols, dstate0, stream);
 }
 
 int rsg_shot_rollout(int n, int ticks, int ckpt_every, float tick_rate, const float* state0, const float* controls,

@@ -47,9 +47,10 @@ hipError_t launch_controls_write(const BatchDev& d, const int32_t* car_at, const
 
 // Differentiable rollouts (rsg_k_diff.hip).
 constexpr int AIR_MAX_K = 32;
-hipError_t launch_air_forward(int n, int ticks, int K, float dt, const float* s0, const float* ctrl,
-                              const float* target, float* s_out, float* loss, float* ckpt, hipStream_t s);
-hipError_t launch_air_backward(int n, int ticks, int K, float dt, const float* ctrl, const float* target,
+hipError_t launch_air_forward(bool rows, int n, int ticks, int K, float dt, const float* s0, const float* ctrl,
+                              const float* target, float* s_out, float* loss, float* ckpt, float* kept,
+                              float* kept_target, hipStream_t s);
+hipError_t launch_air_backward(bool rows, int n, int ticks, int K, float dt, const float* ctrl, const float* target,
                                const float* ckpt, const float* dloss, float* dctrl, float* ds0, hipStream_t s);
 hipError_t launch_shot_forward(int n, int ticks, int K, float dt, const float* state0, const float* ctrl,
                                const float* target, float* state_out, float* loss, float* ckpt, uint32_t* flags,

@@ -8,9 +8,9 @@
 // state0 [n, 13] (position uu, quaternion x y z w, velocity uu/s, angular
 // velocity rad/s), controls [ticks, n, 4] (pitch, yaw, roll in [-1, 1], boost
 // in [0, 1]), target [n, 7] (quaternion, position uu); GPU tensors.  The
-// forward keeps a checkpoint of every car's state every ckpt_every ticks; the
-// backward recomputes each segment from its checkpoint and runs the
-// hand-written adjoint kernel.  Gradients flow to controls and state0.
+// forward keeps a checkpoint of every car's state every ckpt_every ticks (every
+// tick where that is small); the backward recomputes each segment from its
+// checkpoint and runs the hand-written adjoint kernel.  Gradients flow to controls and state0.
 // `stream` is the hipStream_t to run on (the caller's current stream); the
 // backward runs on the stream of its forward, as autograd does for every op.
 #include <torch/extension.h>
@@ -28,6 +28,10 @@ void check(int rc, const char* what) {
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
+// 65536 cars x 120 ticks (409 MB of states) is within it; a batch four times as
+// long goes by checkpoints, as the states would crowd out a caller's own memory.
+constexpr int64_t AIR_KEEP_BYTES = (int64_t)512 << 20;
+
 struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
     static variable_list forward(AutogradContext* ctx, torch::Tensor state0, torch::Tensor controls,
                                  torch::Tensor target, int64_t ckpt_every, double tick_rate, int64_t stream) {
@@ -39,27 +43,34 @@ struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
         TORCH_CHECK(target.dim() == 2 && target.size(1) == 7 && target.size(0) == state0.size(0),
                     "air_rollout: target must be [n, 7]");
         const int64_t n = state0.size(0), ticks = controls.size(0);
-        auto s0 = state0.to(torch::kFloat).t().contiguous();                  // [13][n]
-        auto ctrl = controls.to(torch::kFloat).permute({0, 2, 1}).contiguous();  // [ticks][4][n]
-        auto tgt = target.to(torch::kFloat).t().contiguous();                  // [7][n]
-        const int64_t nseg = (ticks + ckpt_every - 1) / ckpt_every;
+        auto s0 = state0.to(torch::kFloat).contiguous();
+        auto ctrl = controls.to(torch::kFloat).contiguous();
+        auto tgt = target.to(torch::kFloat).contiguous();
+        // Every tick's state is kept where that takes up to AIR_KEEP_BYTES, and
+        // the backward pass then computes none of them again; past it, one every
+        // ckpt_every ticks.
+        const int64_t state_bytes = n * ticks * 13 * (int64_t)sizeof(float);
+        const int64_t every = state_bytes <= AIR_KEEP_BYTES ? 1 : ckpt_every;
+        const int64_t nseg = (ticks + every - 1) / every;
         auto opts = s0.options();
         auto ckpt = torch::empty({nseg * 13 * n}, opts);
-        auto out = torch::empty({13, n}, opts);
+        auto out = torch::empty({n, 13}, opts);
         auto loss = torch::empty({n}, opts);
-        check(rsg_air_rollout((int)n, (int)ticks, (int)ckpt_every, (float)tick_rate, s0.data_ptr<float>(),
-                              ctrl.data_ptr<float>(), tgt.data_ptr<float>(), out.data_ptr<float>(),
-                              loss.data_ptr<float>(), ckpt.data_ptr<float>(), (void*)stream),
+        // the backward pass's own copies: the caller may change its tensors
+        auto kept = torch::empty_like(ctrl), kept_target = torch::empty_like(tgt);
+        check(rsg_air_rollout_rows((int)n, (int)ticks, (int)every, (float)tick_rate, s0.data_ptr<float>(),
+                                   ctrl.data_ptr<float>(), tgt.data_ptr<float>(), out.data_ptr<float>(),
+                                   loss.data_ptr<float>(), ckpt.data_ptr<float>(), kept.data_ptr<float>(),
+                                   kept_target.data_ptr<float>(), (void*)stream),
               "rsg_air_rollout");
-        ctx->save_for_backward({ctrl, tgt, ckpt});
+        ctx->save_for_backward({kept, kept_target, ckpt});
         ctx->saved_data["n"] = n;
         ctx->saved_data["ticks"] = ticks;
-        ctx->saved_data["ckpt_every"] = ckpt_every;
+        ctx->saved_data["ckpt_every"] = every;
         ctx->saved_data["tick_rate"] = tick_rate;
         ctx->saved_data["stream"] = stream;
-        auto final_state = out.t().contiguous();
-        ctx->mark_non_differentiable({final_state});
-        return {loss, final_state};
+        ctx->mark_non_differentiable({out});
+        return {loss, out};
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -71,13 +82,13 @@ struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
         const int64_t stream = ctx->saved_data["stream"].toInt();
         auto dl = grads[0].defined() ? grads[0].to(torch::kFloat).contiguous() : torch::zeros({n}, ctrl.options());
         auto dctrl = torch::empty_like(ctrl);
-        auto ds0 = torch::empty({13, n}, ctrl.options());
-        check(rsg_air_rollout_backward((int)n, (int)ticks, (int)ckpt_every, (float)tick_rate, ctrl.data_ptr<float>(),
-                                       tgt.data_ptr<float>(), ckpt.data_ptr<float>(), dl.data_ptr<float>(),
-                                       dctrl.data_ptr<float>(), ds0.data_ptr<float>(), (void*)stream),
+        auto ds0 = torch::empty({n, 13}, ctrl.options());
+        check(rsg_air_rollout_rows_backward((int)n, (int)ticks, (int)ckpt_every, (float)tick_rate,
+                                            ctrl.data_ptr<float>(), tgt.data_ptr<float>(), ckpt.data_ptr<float>(),
+                                            dl.data_ptr<float>(), dctrl.data_ptr<float>(), ds0.data_ptr<float>(),
+                                            (void*)stream),
               "rsg_air_rollout_backward");
-        return {ds0.t().contiguous(), dctrl.permute({0, 2, 1}).contiguous(), torch::Tensor(), torch::Tensor(),
-                torch::Tensor(), torch::Tensor()};
+        return {ds0, dctrl, torch::Tensor(), torch::Tensor(), torch::Tensor(), torch::Tensor()};
     }
 };
 

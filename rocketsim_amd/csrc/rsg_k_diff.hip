@@ -279,6 +279,80 @@ __global__ void __launch_bounds__(256) rsg_shot_backward_kernel(int n, int ticks
     if (ds0 && lane < SHOT_STATE_WORDS) ds0[(size_t)lane * n + i] = mine * shot_unit(lane);
 }
 
+// Backward with every tick's state at hand (K = 1): `per` pairs a wave, a lane
+// each, take the ticks without a contact by the hand-written adjoint; where a
+// pair has a contact, which is some ticks of a shot, 32 lanes take its 26
+// tangents, two pairs at a time.
+//
+// What bounds it: the chain of ticks, 2.5 us each.  One group of lanes a pair
+// ran all 26 tangents on every tick: 16384 pairs x 90 ticks 3210 us against 614,
+// 101 x 60 298 against 186.
+__global__ void __launch_bounds__(64) rsg_shot_backward_kept_kernel(int n, int ticks, int per, float dt,
+                                                                    const float* ctrl, const float* target,
+                                                                    const float* ckpt, const float* dloss,
+                                                                    float* dctrl, float* ds0) {
+    const int lane = threadIdx.x, first = blockIdx.x * per;
+    const bool on = lane < per && first + lane < n;
+    const int i = on ? first + lane : first;   // a lane without a pair reads the wave's first
+    const ShotConsts k = shot_consts(dt);
+    auto load = [&](int t, int at, ShotState<float>& s, int& le) {
+        shot_ckpt_load(ckpt + (size_t)t * SHOT_CKPT_WORDS * n, n, at, s, le);
+    };
+    ShotState<float> x;
+    int le;
+    load(ticks - 1, i, x, le);
+    ShotCtrl<float> c = shot_ctrl(ctrl, n, i, ticks - 1);
+    float g[SHOT_STATE_WORDS];
+    {
+        ShotState<float> s = x;
+        int last_extra = le;
+        uint32_t fl = 0;
+        shot_step(s, c, ticks - 1, last_extra, fl, k);
+        shot_loss_grad(s, v3(target[i], target[n + i], target[2 * n + i]), dloss[i], g);
+    }
+    RSG_UNROLL_1
+    for (int t = ticks - 1; t >= 0; t--) {
+        const int before = t > 0 ? t - 1 : 0;
+        ShotState<float> xb;
+        int leb;
+        load(before, i, xb, leb);
+        const ShotCtrl<float> cb = shot_ctrl(ctrl, n, i, before);
+        const bool touch = shot_touches(x, k);
+        uint64_t touching = __ballot(on && touch);
+        RSG_UNROLL_1
+        while (touching) {
+            const int a = __builtin_ctzll(touching);
+            touching &= touching - 1u;
+            const int b = touching ? __builtin_ctzll(touching) : a;
+            touching &= touching - 1u;
+            const int from = lane < SHOT_GROUP ? a : b, j = lane & (SHOT_GROUP - 1);
+            ShotState<float> s;
+            int last_extra;
+            load(t, first + from, s, last_extra);
+            float gs[SHOT_STATE_WORDS];
+            for (int w = 0; w < SHOT_STATE_WORDS; w++) gs[w] = __shfl(g[w], from);
+            const float mine = shot_vjp_entry(s, shot_ctrl(ctrl, n, first + from, t), t, last_extra, k, gs, j);
+            if (j >= SHOT_STATE_WORDS && j < SHOT_INPUTS)
+                dctrl[(size_t)t * 4 * n + (size_t)(j - SHOT_STATE_WORDS) * n + first + from] = mine;
+            for (int w = 0; w < SHOT_STATE_WORDS; w++) {
+                const float v = __shfl(mine, w + (lane == a ? 0 : SHOT_GROUP));
+                g[w] = lane == a || lane == b ? v : g[w];
+            }
+        }
+        if (on && !touch) {
+            AirCtrl gc;
+            shot_flight_vjp(x, c, k, g, gc);
+            float* o = dctrl + (size_t)t * 4 * n;
+            o[i] = gc.pitch; o[n + i] = gc.yaw; o[2 * n + i] = gc.roll; o[3 * n + i] = gc.boost;
+        }
+        x = xb;
+        le = leb;
+        c = cb;
+    }
+    if (ds0 && on)
+        for (int w = 0; w < SHOT_STATE_WORDS; w++) ds0[(size_t)w * n + i] = g[w] * shot_unit(w);
+}
+
 namespace rsg {
 
 // 64-lane workgroups spread the cars over every CU.
@@ -303,11 +377,20 @@ hipError_t launch_air_backward(bool rows, int n, int ticks, int K, float dt, con
     return hipGetLastError();
 }
 
+// Pairs per wave: spread over the SIMDs first, as a wave takes the contact path
+// on every tick on which one of its pairs has a contact (forward, 16384 pairs x
+// 90 ticks: 301 us at 16 a wave against 375 at 64; 101 x 60: 117 at 1 against
+// 291).
+static int shot_per_wave(int n) {
+    constexpr int SIMDS = 1024;
+    const int per = (n + SIMDS - 1) / SIMDS;
+    return per > 64 ? 64 : per;
+}
+
 hipError_t launch_shot_forward(int n, int ticks, int K, float dt, const float* state0, const float* ctrl,
                                const float* target, float* state_out, float* loss, float* ckpt, uint32_t* flags,
                                hipStream_t s) {
-    // 64-lane workgroups spread the pairs over every CU
-    const int block = 64, grid = (n + block - 1) / block;
+    const int block = shot_per_wave(n), grid = (n + block - 1) / block;
     hipLaunchKernelGGL(rsg_shot_forward_kernel, dim3(grid), dim3(block), 0, s, n, ticks, K, dt, state0, ctrl, target,
                        state_out, loss, ckpt, flags);
     return hipGetLastError();
@@ -315,6 +398,12 @@ hipError_t launch_shot_forward(int n, int ticks, int K, float dt, const float* s
 
 hipError_t launch_shot_backward(int n, int ticks, int K, float dt, const float* ctrl, const float* target,
                                 const float* ckpt, const float* dloss, float* dctrl, float* ds0, hipStream_t s) {
+    if (K == 1) {
+        const int per = shot_per_wave(n);
+        hipLaunchKernelGGL(rsg_shot_backward_kept_kernel, dim3((n + per - 1) / per), dim3(64), 0, s, n, ticks, per, dt, ctrl,
+                           target, ckpt, dloss, dctrl, ds0);
+        return hipGetLastError();
+    }
     const int block = 256, per_block = block / SHOT_GROUP, grid = (n + per_block - 1) / per_block;
     const size_t lds = (size_t)per_block * K * SHOT_LDS_WORDS * sizeof(float);
     hipLaunchKernelGGL(rsg_shot_backward_kernel, dim3(grid), dim3(block), lds, s, n, ticks, K, dt, ctrl, target, ckpt,

@@ -229,6 +229,30 @@ RSG_FN void shot_apply(const ShotRow<S>& c, ShotBody<S>& A, ShotBody<S>& B, S de
     B.dw = B.dw + c.ang_b * delta;
 }
 
+// The car's hitbox and the ball: the closest point of the box's core to the
+// ball's centre, from there.
+template <class S>
+struct ShotGap {
+    Vt<S> to_box;
+    S dist_core, depth;
+    bool inside, contact;
+};
+template <class S>
+RSG_FN ShotGap<S> shot_gap(const ShotState<S>& s, Vt<S> f, Vt<S> r, Vt<S> u, const ShotConsts& k) {
+    ShotGap<S> o;
+    Vt<S> box_c = s.cp + f * k.box_offset.x + r * k.box_offset.y + u * k.box_offset.z;
+    Vt<S> d = s.bp - box_c;
+    S lx = vdot(f, d), ly = vdot(r, d), lz = vdot(u, d);
+    o.inside = fabsf(sval(lx)) < k.box_he.x && fabsf(sval(ly)) < k.box_he.y && fabsf(sval(lz)) < k.box_he.z;
+    S qx = s_clamp(lx, -k.box_he.x, k.box_he.x), qy = s_clamp(ly, -k.box_he.y, k.box_he.y),
+      qz = s_clamp(lz, -k.box_he.z, k.box_he.z);
+    o.to_box = (box_c + f * qx + r * qy + u * qz) - s.bp;
+    o.dist_core = s_sqrt(vlen2(o.to_box));
+    o.depth = o.dist_core - (k.box_margin + k.radius);
+    o.contact = !o.inside && sval(o.depth) < k.threshold && sval(o.dist_core) > 0.f;
+    return o;
+}
+
 // One tick.  `tick` counts from 0; last_extra is the tick of the last extra
 // hit impulse (start below -1); flags collect SHOT_*.
 template <class S>
@@ -248,18 +272,11 @@ RSG_FN void shot_step(ShotState<S>& s, const ShotCtrl<S>& c, int tick, int& last
     s.bv = s.bv * k.drag;
     Vt<S> ext_fb = grav * dt;
 
-    // car hitbox vs ball: closest point of the box core to the ball centre
-    Vt<S> box_c = s.cp + f * k.box_offset.x + r * k.box_offset.y + u * k.box_offset.z;
-    Vt<S> d = s.bp - box_c;
-    S lx = vdot(f, d), ly = vdot(r, d), lz = vdot(u, d);
-    const bool inside = fabsf(sval(lx)) < k.box_he.x && fabsf(sval(ly)) < k.box_he.y && fabsf(sval(lz)) < k.box_he.z;
-    S qx = s_clamp(lx, -k.box_he.x, k.box_he.x), qy = s_clamp(ly, -k.box_he.y, k.box_he.y),
-      qz = s_clamp(lz, -k.box_he.z, k.box_he.z);
-    Vt<S> to_box = (box_c + f * qx + r * qy + u * qz) - s.bp;
-    S dist_core = s_sqrt(vlen2(to_box));
-    S depth = dist_core - (k.box_margin + k.radius);
-    if (inside) flags |= SHOT_DEEP;
-    const bool contact = !inside && sval(depth) < k.threshold && sval(dist_core) > 0.f;
+    const ShotGap<S> gap = shot_gap(s, f, r, u, k);
+    const Vt<S> to_box = gap.to_box;
+    const S dist_core = gap.dist_core, depth = gap.depth;
+    const bool contact = gap.contact;
+    if (gap.inside) flags |= SHOT_DEEP;
 
     Vt<S> cache = vt(s_const<S>(0.f), s_const<S>(0.f), s_const<S>(0.f));
     Vt<S> car_v = s.cv, car_w = s.cw, ball_v = s.bv, ball_w = s.bw;
@@ -524,6 +541,43 @@ RSG_FN float shot_vjp_entry(const ShotState<float>& s, const ShotCtrl<float>& c,
     float acc = 0.f;
     for (int w = 0; w < SHOT_STATE_WORDS; w++) acc += g[w] * shot_word(sd, w).d;
     return acc;
+}
+
+// Whether the tick at s has a contact.
+RSG_FN bool shot_touches(const ShotState<float>& s, const ShotConsts& k) {
+    Vt<float> f, r, u;
+    qt_basis(s.cq, f, r, u);
+    return shot_gap(s, f, r, u, k).contact;
+}
+
+// The product of a tick without a contact, by hand: the car is rsg_adjoint.h's,
+// and the ball flies by itself.
+RSG_FN void shot_flight_vjp(const ShotState<float>& s, const ShotCtrl<float>& c, const ShotConsts& k,
+                            float g[SHOT_STATE_WORDS], AirCtrl& gc) {
+    AirState a, ga;
+    a.p = v3(s.cp.x, s.cp.y, s.cp.z);
+    a.q = q4(s.cq.x, s.cq.y, s.cq.z, s.cq.w);
+    a.v = v3(s.cv.x, s.cv.y, s.cv.z);
+    a.w = v3(s.cw.x, s.cw.y, s.cw.z);
+    ga.p = v3(g[0], g[1], g[2]);
+    ga.q = q4(g[3], g[4], g[5], g[6]);
+    ga.v = v3(g[7], g[8], g[9]);
+    ga.w = v3(g[10], g[11], g[12]);
+    AirCtrl ac;
+    ac.pitch = c.pitch; ac.yaw = c.yaw; ac.roll = c.roll; ac.boost = c.boost;
+    gc.pitch = gc.yaw = gc.roll = gc.boost = 0.f;
+    air_step_adjoint(a, ac, k.dt, ga, gc);
+    g[0] = ga.p.x; g[1] = ga.p.y; g[2] = ga.p.z;
+    g[3] = ga.q.x; g[4] = ga.q.y; g[5] = ga.q.z; g[6] = ga.q.w;
+    g[7] = ga.v.x; g[8] = ga.v.y; g[9] = ga.v.z;
+    g[10] = ga.w.x; g[11] = ga.w.y; g[12] = ga.w.z;
+    // bv1 = bv drag + gravity dt; bp' = bp + bv1 dt; bv' and bw' capped
+    const V3 gp = v3(g[13], g[14], g[15]);
+    const V3 bv1 = v3(s.bv.x, s.bv.y, s.bv.z) * k.drag + v3(0.f, 0.f, GRAVITY_Z * UU_TO_BT) * k.dt;
+    const V3 gv = (air_cap_adjoint(bv1, BALL_MAX_SPEED * UU_TO_BT, v3(g[16], g[17], g[18])) + gp * k.dt) * k.drag;
+    const V3 gw = air_cap_adjoint(v3(s.bw.x, s.bw.y, s.bw.z), BALL_MAX_ANG_SPEED, v3(g[19], g[20], g[21]));
+    g[16] = gv.x; g[17] = gv.y; g[18] = gv.z;
+    g[19] = gw.x; g[20] = gw.y; g[21] = gw.z;
 }
 
 // Vector-Jacobian product of tick t at (s, c): g (adjoint of the output

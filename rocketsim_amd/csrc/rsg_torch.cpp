@@ -28,9 +28,15 @@ void check(int rc, const char* what) {
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-// 65536 cars x 120 ticks (409 MB of states) is within it; a batch four times as
-// long goes by checkpoints, as the states would crowd out a caller's own memory.
-constexpr int64_t AIR_KEEP_BYTES = (int64_t)512 << 20;
+// Ticks per checkpoint.  Where all ticks' states take up to KEEP_BYTES they are
+// all kept, and the backward pass computes none of them again (65536 cars x 120
+// ticks, 409 MB: 455 us in all against 548; 16384 shots x 90 ticks, 136 MB:
+// 950 us against 3540); past it one every ckpt_every ticks, as the states would crowd out a
+// caller's own memory.
+constexpr int64_t KEEP_BYTES = (int64_t)512 << 20;
+int64_t kept_every(int64_t words, int64_t ckpt_every) {
+    return words * (int64_t)sizeof(float) <= KEEP_BYTES ? 1 : ckpt_every;
+}
 
 struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
     static variable_list forward(AutogradContext* ctx, torch::Tensor state0, torch::Tensor controls,
@@ -46,11 +52,7 @@ struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
         auto s0 = state0.to(torch::kFloat).contiguous();
         auto ctrl = controls.to(torch::kFloat).contiguous();
         auto tgt = target.to(torch::kFloat).contiguous();
-        // Every tick's state is kept where that takes up to AIR_KEEP_BYTES, and
-        // the backward pass then computes none of them again; past it, one every
-        // ckpt_every ticks.
-        const int64_t state_bytes = n * ticks * 13 * (int64_t)sizeof(float);
-        const int64_t every = state_bytes <= AIR_KEEP_BYTES ? 1 : ckpt_every;
+        const int64_t every = kept_every(n * ticks * 13, ckpt_every);
         const int64_t nseg = (ticks + every - 1) / every;
         auto opts = s0.options();
         auto ckpt = torch::empty({nseg * 13 * n}, opts);
@@ -109,13 +111,14 @@ struct ShotRolloutFn : public torch::autograd::Function<ShotRolloutFn> {
         auto s0 = state0.to(torch::kFloat).t().contiguous();
         auto ctrl = controls.to(torch::kFloat).permute({0, 2, 1}).contiguous();
         auto tgt = target.to(torch::kFloat).t().contiguous();
-        const int64_t nseg = (ticks + ckpt_every - 1) / ckpt_every;
+        const int64_t every = kept_every(n * ticks * 23, ckpt_every);
+        const int64_t nseg = (ticks + every - 1) / every;
         auto opts = s0.options();
         auto ckpt = torch::empty({nseg * 23 * n}, opts);
         auto out = torch::empty({22, n}, opts);
         auto loss = torch::empty({n}, opts);
         auto flags = torch::empty({n}, opts.dtype(torch::kInt32));
-        check(rsg_shot_rollout((int)n, (int)ticks, (int)ckpt_every, (float)tick_rate, s0.data_ptr<float>(),
+        check(rsg_shot_rollout((int)n, (int)ticks, (int)every, (float)tick_rate, s0.data_ptr<float>(),
                                ctrl.data_ptr<float>(), tgt.data_ptr<float>(), out.data_ptr<float>(),
                                loss.data_ptr<float>(), ckpt.data_ptr<float>(),
                                reinterpret_cast<uint32_t*>(flags.data_ptr<int32_t>()), (void*)stream),
@@ -123,7 +126,7 @@ struct ShotRolloutFn : public torch::autograd::Function<ShotRolloutFn> {
         ctx->save_for_backward({ctrl, tgt, ckpt});
         ctx->saved_data["n"] = n;
         ctx->saved_data["ticks"] = ticks;
-        ctx->saved_data["ckpt_every"] = ckpt_every;
+        ctx->saved_data["ckpt_every"] = every;
         ctx->saved_data["tick_rate"] = tick_rate;
         ctx->saved_data["stream"] = stream;
         auto final_state = out.t().contiguous();

@@ -624,11 +624,12 @@ struct Launch {
 
 // Kernel and arenas per workgroup.  The cooperative kernel is the fastest
 // wherever its per-arena block fits (ms per tick, cooperative / LDS / plain:
-// one 1v1 arena 0.030 / 0.100 / 0.128, 2v2 x 4096 0.303 / 0.609 / 0.771,
-// 2v2 x 16384 0.515 / 0.953 / 1.080, 32768 arenas of 1v1 to 3v3 0.81 / 2.07 /
-// 1.48), so it is the default; arenas are spread one per workgroup until every
+// one 1v1 arena 0.031 / 0.100 / 0.127, 2v2 x 4096 0.192 / 0.573 / 0.762,
+// 2v2 x 16384 0.350 / 0.931 / 1.072, 32768 arenas of 1v1 to 3v3 0.587 / 2.03 /
+// 1.45), so it is the default; arenas are spread one per workgroup until every
 // SIMD has a wave, then packed up to the most a workgroup holds (2v2 x 16384
-// at 1, 2, 3 and 4 arenas a workgroup: 0.723, 0.583, 0.533 and 0.515).
+// at 1, 2, 3 and 4 arenas a workgroup: 0.522, 0.410, 0.363 and 0.350; x 4096:
+// 0.223, 0.185, 0.196 and 0.192).
 Launch choose_launch(const rsg_batch* b) {
     const int simds = device_simds();
     int spread = (b->dev.n + simds - 1) / simds;  // arenas per wave at one wave per SIMD

@@ -12,9 +12,9 @@ namespace rsg {
 // plain and LDS kernels run fastest with the whole register file (1).  The
 // cooperative kernel waits on memory and on its slowest lane half of the time
 // and gains from a second wave per SIMD where there are waves to fill it
-// (2v2 x 16384 arenas: 0.515 ms a tick at 2, 0.561 at 1; 32768 arenas of 1v1
-// to 3v3: 0.81 and 1.14), and loses a little to its spills where there are
-// not (2v2 x 4096: 0.303 and 0.271).
+// (2v2 x 16384 arenas: 0.350 ms a tick at 2, 0.415 at 1; 32768 arenas of 1v1
+// to 3v3: 0.587 and 0.940), and loses a little to its spills where there are
+// not (2v2 x 4096: 0.192 and 0.183).
 #ifndef RSG_STEP_WAVES_PER_EU
 #define RSG_STEP_WAVES_PER_EU 1
 #endif

@@ -31,11 +31,11 @@
 // kernel whose serial lane did most of this through global work space: 839 KB
 // of code against an instruction cache of 64 KB, 3.4 KB of private memory per
 // lane and 1600 vector memory operations a wave-tick.  Here every algorithm
-// has one inlined instance (136 KB of code), the working set of an ordinary
-// tick is in LDS and registers (330 vector reads a wave-tick), and what is
-// rare (penetration, box-box, kickoff) is out of line.  2v2 x 16384 arenas:
-// 0.515 ms a tick against 0.863; one 1v1 arena: 0.030 against 0.059.  A
-// wave-tick takes 93 us: narrow 26, solve 16, rays 11, pads 7, car 7.
+// has one inlined instance, the working set of an ordinary tick is in LDS and
+// registers (185 vector reads a wave-tick), and what is rare (penetration,
+// box-box, kickoff) is out of line.  2v2 x 16384 arenas: 0.350 ms a tick against
+// 0.863; one 1v1 arena: 0.031 against 0.059.  Waves still wait 47 % of their
+// time, and a launch ends with its slowest wave.
 #pragma once
 
 #include "rsg_tick.h"

@@ -160,7 +160,8 @@ struct rsg_batch {
     int32_t* car_at = nullptr;          // arena << 4 | slot of each car (launch_records_read)
     unsigned char* records = nullptr;   // pinned: what the records kernel writes
     size_t records_bytes = 0;
-    bool records_fresh = false;         // they hold every record of the device's state (small batches)
+    bool records_fresh = false;         // they hold every record of the device's state (small batches); whatever
+                                        // writes to the device's planes clears it
     rsg_controls* controls = nullptr;   // pinned: the controls set last
     bool controls_pending = false;      // they are newer than the mirror's and the device's
     bool synced = false;                // no device work of this batch since the device was waited for
@@ -218,6 +219,7 @@ int flush_controls(rsg_batch* b, hipStream_t s) {
     HIP_OK(launch_controls_write(b->dev, b->car_at, b->controls, b->total_cars, s));
     b->controls_pending = false;
     b->dev_newer = true;
+    b->records_fresh = false;
     b->synced = false;
     return 0;
 }
@@ -231,6 +233,7 @@ int upload(rsg_batch* b) {
         HIP_OK(hipMemcpy(const_cast<rsg_mutator_config*>(b->dev.mut), b->h_mut.data(),
                          b->h_mut.size() * sizeof(rsg_mutator_config), hipMemcpyHostToDevice));
         b->host_dirty = false;
+        b->records_fresh = false;
     }
     if (b->controls_pending) {
         if (flush_controls(b, nullptr) != 0) return -1;

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from rocketsim_amd.batch import ArenaBatch
+from rocketsim_amd.game_events import GameEventTracker
 from rocketsim_amd.state import Controls, MODE_HEATSEEKER, MODE_HOOPS, MODE_SOCCAR, MODE_THE_VOID
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +76,34 @@ def test_controls_on_either_way(arenas):
         return out
 
     assert play(False) == play(True)
+
+
+@pytest.mark.parametrize("arenas", [1, 33, 1500])
+def test_what_was_set_is_read_back_after_uploads_without_a_step(arenas):
+    """A state set after a read goes to the device by one call that does not
+    step, controls set then by another; the getters give what was set."""
+    b = _batch([2] * arenas)
+    tracker = GameEventTracker(b)
+    b.step(30)
+    before = _records(b)
+    cars, balls, pads = b.get_cars(), b.get_balls(), b.get_pads()
+    for c in cars:
+        c.boost = 77.0
+    for x in balls:
+        x.pos[0], x.vel[2] = 123.0, 456.0
+    for p in pads:
+        p.cooldown, p.is_active = 3.0, 0
+    b.set_cars(cars)
+    b.set_balls(balls)
+    b.set_pads(pads)
+    tracker.update(b)               # the set state to the device
+    b.set_controls((Controls * b.n_cars)(*[Controls(throttle=1.0)] * b.n_cars))
+    tracker.update(b)               # the controls to the device
+    got = _records(b)               # the device's are the newer
+    b.get_goals()
+    want = _records(b)              # the mirror's
+    tracker.close()
+    b.close()
+    for what, x, y, z in zip(("cars", "balls", "pads"), got, want, before):
+        assert x == y, what
+        assert x != z, what + " as before the set"

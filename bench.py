@@ -169,11 +169,11 @@ def run_timed(batch, steps, warmup, preroll, chunk, use_graph, stream):
 
 
 def bench_adjoint(n_cars=65536, ticks=120, reps=5, seed=7):
-    """Differentiable air control (65536 airborne cars, 120 ticks, checkpoints
-    every 16 ticks): rollouts/s of forward + hand-written adjoint through the
+    """Differentiable air control (65536 airborne cars, 120 ticks, every
+    tick's state kept): rollouts/s of forward + hand-written adjoint through the
     torch autograd Function."""
     import torch
-    from rocketsim_amd.adjoint import air_rollout
+    from rocketsim_amd.adjoint import air_ckpt_every, air_rollout
     g = torch.Generator(device="cuda").manual_seed(seed)
     pos = torch.stack([torch.rand(n_cars, device="cuda", generator=g) * 4000 - 2000,
                        torch.rand(n_cars, device="cuda", generator=g) * 4000 - 2000,
@@ -200,18 +200,19 @@ def bench_adjoint(n_cars=65536, ticks=120, reps=5, seed=7):
         one()
     torch.cuda.synchronize()
     wall = (time.perf_counter() - t0) / reps
-    return {"value": n_cars / wall, "unit": "rollouts/s", "cars": n_cars, "ticks": ticks, "ckpt_every": 16,
+    return {"value": n_cars / wall, "unit": "rollouts/s", "cars": n_cars, "ticks": ticks,
+            "ckpt_every": air_ckpt_every(n_cars, ticks),
             "ms_per_batch": wall * 1e3,
             "workload": "airborne cars, z U[800,1800], random orientation, v N(0,500), w N(0,2); "
                         "controls tanh/sigmoid of parameters; loss geodesic angle + 1e-4 |dp|^2; fwd + adjoint"}
 
 
 def bench_shot(n=16384, ticks=90, reps=5, seed=13):
-    """Differentiable aerial shot (16384 car+ball pairs, 90 ticks, checkpoints
-    every 16 ticks): rollouts/s of forward + adjoint through the car-ball hit,
+    """Differentiable aerial shot (16384 car+ball pairs, 90 ticks, every
+    tick's state kept): rollouts/s of forward + adjoint through the car-ball hit,
     through the LibTorch autograd Function."""
     import torch
-    from rocketsim_amd.adjoint import shot_rollout
+    from rocketsim_amd.adjoint import shot_ckpt_every, shot_rollout
     from rocketsim_amd.workloads import shot_problem
     s0, ctrl, tgt = shot_problem(n, ticks, seed)
     state0, target = s0.float().cuda(), tgt.float().cuda()
@@ -233,7 +234,8 @@ def bench_shot(n=16384, ticks=90, reps=5, seed=13):
     torch.cuda.synchronize()
     wall = (time.perf_counter() - t0) / reps
     fl = flags.cpu()
-    return {"value": n / wall, "unit": "rollouts/s", "pairs": n, "ticks": ticks, "ckpt_every": 16,
+    return {"value": n / wall, "unit": "rollouts/s", "pairs": n, "ticks": ticks,
+            "ckpt_every": shot_ckpt_every(n, ticks),
             "ms_per_batch": wall * 1e3, "touched": int(((fl & 1) != 0).sum()),
             "outside_model": int(((fl & 6) != 0).sum()),
             "workload": "ball x U[-3000,3000], y U[-4000,4000], z U[300,1500] uu, v N(0,800); car airborne "

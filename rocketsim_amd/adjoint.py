@@ -11,8 +11,13 @@ state0 [n, 13] (position uu, quaternion x y z w, velocity uu/s, angular
 velocity rad/s), controls [ticks, n, 4] (pitch, yaw, roll in [-1, 1], boost
 in [0, 1]), target [n, 7] (quaternion, position uu); float32 CUDA tensors.
 The forward pass keeps a checkpoint of every car's state every `ckpt_every`
-ticks; the backward pass recomputes each segment from its checkpoint and runs
-the hand-written adjoint kernel.  Gradients flow to controls and state0.
+ticks (1 to 32); the backward pass recomputes each segment from its checkpoint
+and runs the hand-written adjoint kernel.  Gradients flow to controls and
+state0.  Without a `ckpt_every`, `air_rollout` and `shot_rollout` keep every
+tick's state, which is the fastest, where all states take up to 512 MB, and
+else one every CKPT_EVERY ticks; name one to bound the memory that a graph
+holds until its backward pass (ceil(ticks / ckpt_every) * n * 52 bytes, for the
+shot 92).
 """
 import importlib.util
 import os
@@ -85,7 +90,7 @@ def torch_ext():
     return _ext
 
 
-def air_rollout(state0, controls, target, ckpt_every=CKPT_EVERY, tick_rate=120.0):
+def air_rollout(state0, controls, target, ckpt_every=None, tick_rate=120.0):
     """(loss [n], final state [n, 13]) through the LibTorch C++ Function, on
     the current stream."""
     stream = torch.cuda.current_stream().cuda_stream
@@ -93,7 +98,7 @@ def air_rollout(state0, controls, target, ckpt_every=CKPT_EVERY, tick_rate=120.0
     return loss, final
 
 
-def shot_rollout(state0, controls, target, ckpt_every=CKPT_EVERY, tick_rate=120.0):
+def shot_rollout(state0, controls, target, ckpt_every=None, tick_rate=120.0):
     """Differentiable aerial shot through the LibTorch C++ Function:
     state0 [n, 22] (car position uu, quaternion, velocity uu/s, angular
     velocity; ball position uu, velocity uu/s, angular velocity), controls
@@ -104,6 +109,16 @@ def shot_rollout(state0, controls, target, ckpt_every=CKPT_EVERY, tick_rate=120.
     stream = torch.cuda.current_stream().cuda_stream
     loss, final, flags = torch_ext().shot_rollout(state0, controls, target, ckpt_every, tick_rate, stream)
     return loss, final, flags
+
+
+def air_ckpt_every(n, ticks):
+    """The ckpt_every that air_rollout takes by itself for n cars."""
+    return torch_ext().air_ckpt_every(n, ticks)
+
+
+def shot_ckpt_every(n, ticks):
+    """The ckpt_every that shot_rollout takes by itself for n pairs."""
+    return torch_ext().shot_ckpt_every(n, ticks)
 
 
 def air_rollout_py(state0, controls, target, ckpt_every=CKPT_EVERY, tick_rate=120.0):

@@ -8,11 +8,14 @@
 // state0 [n, 13] (position uu, quaternion x y z w, velocity uu/s, angular
 // velocity rad/s), controls [ticks, n, 4] (pitch, yaw, roll in [-1, 1], boost
 // in [0, 1]), target [n, 7] (quaternion, position uu); GPU tensors.  The
-// forward keeps a checkpoint of every car's state every ckpt_every ticks (every
-// tick where that is small); the backward recomputes each segment from its
-// checkpoint and runs the hand-written adjoint kernel.  Gradients flow to controls and state0.
+// forward keeps a checkpoint of every car's state every ckpt_every ticks (None:
+// chosen by size, chosen_every below); the backward recomputes each segment
+// from its checkpoint and runs the hand-written adjoint kernel.  Gradients flow
+// to controls and state0.
 // `stream` is the hipStream_t to run on (the caller's current stream); the
 // backward runs on the stream of its forward, as autograd does for every op.
+#include <optional>
+
 #include <torch/extension.h>
 
 #include <string>
@@ -28,15 +31,19 @@ void check(int rc, const char* what) {
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-// Ticks per checkpoint.  Where all ticks' states take up to KEEP_BYTES they are
-// all kept, and the backward pass computes none of them again (65536 cars x 120
-// ticks, 409 MB: 455 us in all against 548; 16384 shots x 90 ticks, 136 MB:
-// 950 us against 3540); past it one every ckpt_every ticks, as the states would crowd out a
-// caller's own memory.
+// Ticks per checkpoint where the caller names none: every tick's state, which
+// the backward pass then need not compute again, up to KEEP_BYTES of them
+// (65536 cars x 120 ticks, 409 MB: 455 us in all against 548 at one every 16;
+// 16384 shots x 90 ticks, 136 MB: 950 us against 3540); past it one state every
+// CKPT_EVERY ticks, as the states would crowd out a caller's own memory.
 constexpr int64_t KEEP_BYTES = (int64_t)512 << 20;
-int64_t kept_every(int64_t words, int64_t ckpt_every) {
-    return words * (int64_t)sizeof(float) <= KEEP_BYTES ? 1 : ckpt_every;
+constexpr int64_t CKPT_EVERY = 16, MAX_CKPT_EVERY = 32;
+constexpr int64_t AIR_WORDS = 13, SHOT_WORDS = 23;   // of a checkpoint
+int64_t chosen_every(int64_t n, int64_t ticks, int64_t words) {
+    return n * ticks * words * (int64_t)sizeof(float) <= KEEP_BYTES ? 1 : CKPT_EVERY;
 }
+int64_t air_ckpt_every(int64_t n, int64_t ticks) { return chosen_every(n, ticks, AIR_WORDS); }
+int64_t shot_ckpt_every(int64_t n, int64_t ticks) { return chosen_every(n, ticks, SHOT_WORDS); }
 
 struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
     static variable_list forward(AutogradContext* ctx, torch::Tensor state0, torch::Tensor controls,
@@ -52,15 +59,14 @@ struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
         auto s0 = state0.to(torch::kFloat).contiguous();
         auto ctrl = controls.to(torch::kFloat).contiguous();
         auto tgt = target.to(torch::kFloat).contiguous();
-        const int64_t every = kept_every(n * ticks * 13, ckpt_every);
-        const int64_t nseg = (ticks + every - 1) / every;
+        const int64_t nseg = (ticks + ckpt_every - 1) / ckpt_every;
         auto opts = s0.options();
-        auto ckpt = torch::empty({nseg * 13 * n}, opts);
+        auto ckpt = torch::empty({nseg * AIR_WORDS * n}, opts);
         auto out = torch::empty({n, 13}, opts);
         auto loss = torch::empty({n}, opts);
         // the backward pass's own copies: the caller may change its tensors
         auto kept = torch::empty_like(ctrl), kept_target = torch::empty_like(tgt);
-        check(rsg_air_rollout_rows((int)n, (int)ticks, (int)every, (float)tick_rate, s0.data_ptr<float>(),
+        check(rsg_air_rollout_rows((int)n, (int)ticks, (int)ckpt_every, (float)tick_rate, s0.data_ptr<float>(),
                                    ctrl.data_ptr<float>(), tgt.data_ptr<float>(), out.data_ptr<float>(),
                                    loss.data_ptr<float>(), ckpt.data_ptr<float>(), kept.data_ptr<float>(),
                                    kept_target.data_ptr<float>(), (void*)stream),
@@ -68,7 +74,7 @@ struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
         ctx->save_for_backward({kept, kept_target, ckpt});
         ctx->saved_data["n"] = n;
         ctx->saved_data["ticks"] = ticks;
-        ctx->saved_data["ckpt_every"] = every;
+        ctx->saved_data["ckpt_every"] = ckpt_every;
         ctx->saved_data["tick_rate"] = tick_rate;
         ctx->saved_data["stream"] = stream;
         ctx->mark_non_differentiable({out});
@@ -111,14 +117,13 @@ struct ShotRolloutFn : public torch::autograd::Function<ShotRolloutFn> {
         auto s0 = state0.to(torch::kFloat).t().contiguous();
         auto ctrl = controls.to(torch::kFloat).permute({0, 2, 1}).contiguous();
         auto tgt = target.to(torch::kFloat).t().contiguous();
-        const int64_t every = kept_every(n * ticks * 23, ckpt_every);
-        const int64_t nseg = (ticks + every - 1) / every;
+        const int64_t nseg = (ticks + ckpt_every - 1) / ckpt_every;
         auto opts = s0.options();
-        auto ckpt = torch::empty({nseg * 23 * n}, opts);
+        auto ckpt = torch::empty({nseg * SHOT_WORDS * n}, opts);
         auto out = torch::empty({22, n}, opts);
         auto loss = torch::empty({n}, opts);
         auto flags = torch::empty({n}, opts.dtype(torch::kInt32));
-        check(rsg_shot_rollout((int)n, (int)ticks, (int)every, (float)tick_rate, s0.data_ptr<float>(),
+        check(rsg_shot_rollout((int)n, (int)ticks, (int)ckpt_every, (float)tick_rate, s0.data_ptr<float>(),
                                ctrl.data_ptr<float>(), tgt.data_ptr<float>(), out.data_ptr<float>(),
                                loss.data_ptr<float>(), ckpt.data_ptr<float>(),
                                reinterpret_cast<uint32_t*>(flags.data_ptr<int32_t>()), (void*)stream),
@@ -126,7 +131,7 @@ struct ShotRolloutFn : public torch::autograd::Function<ShotRolloutFn> {
         ctx->save_for_backward({ctrl, tgt, ckpt});
         ctx->saved_data["n"] = n;
         ctx->saved_data["ticks"] = ticks;
-        ctx->saved_data["ckpt_every"] = every;
+        ctx->saved_data["ckpt_every"] = ckpt_every;
         ctx->saved_data["tick_rate"] = tick_rate;
         ctx->saved_data["stream"] = stream;
         auto final_state = out.t().contiguous();
@@ -154,16 +159,24 @@ struct ShotRolloutFn : public torch::autograd::Function<ShotRolloutFn> {
 };
 
 std::vector<torch::Tensor> shot_rollout(torch::Tensor state0, torch::Tensor controls, torch::Tensor target,
-                                        int64_t ckpt_every, double tick_rate, int64_t stream) {
-    TORCH_CHECK(ckpt_every >= 1 && ckpt_every <= 32, "shot_rollout: ckpt_every must be within [1, 32]");
-    auto r = ShotRolloutFn::apply(state0, controls, target, ckpt_every, tick_rate, stream);
+                                        std::optional<int64_t> ckpt_every, double tick_rate, int64_t stream) {
+    TORCH_CHECK(!ckpt_every || (*ckpt_every >= 1 && *ckpt_every <= MAX_CKPT_EVERY),
+                "shot_rollout: ckpt_every must be within [1, 32]");
+    // (tensors of other shapes are refused by the Function)
+    const int64_t every = ckpt_every ? *ckpt_every
+                        : controls.dim() == 3 ? shot_ckpt_every(controls.size(1), controls.size(0)) : CKPT_EVERY;
+    auto r = ShotRolloutFn::apply(state0, controls, target, every, tick_rate, stream);
     return {r[0], r[1], r[2]};
 }
 
 std::vector<torch::Tensor> air_rollout(torch::Tensor state0, torch::Tensor controls, torch::Tensor target,
-                                       int64_t ckpt_every, double tick_rate, int64_t stream) {
-    TORCH_CHECK(ckpt_every >= 1 && ckpt_every <= 32, "air_rollout: ckpt_every must be within [1, 32]");
-    auto r = AirRolloutFn::apply(state0, controls, target, ckpt_every, tick_rate, stream);
+                                       std::optional<int64_t> ckpt_every, double tick_rate, int64_t stream) {
+    TORCH_CHECK(!ckpt_every || (*ckpt_every >= 1 && *ckpt_every <= MAX_CKPT_EVERY),
+                "air_rollout: ckpt_every must be within [1, 32]");
+    // (tensors of other shapes are refused by the Function)
+    const int64_t every = ckpt_every ? *ckpt_every
+                        : controls.dim() == 3 ? air_ckpt_every(controls.size(1), controls.size(0)) : CKPT_EVERY;
+    auto r = AirRolloutFn::apply(state0, controls, target, every, tick_rate, stream);
     return {r[0], r[1]};
 }
 
@@ -174,6 +187,10 @@ PYBIND11_MODULE(rsg_torch, m) {
     m.def("air_rollout", &air_rollout, "loss, final = air_rollout(state0, controls, target, ckpt_every, tick_rate, stream)",
           pybind11::arg("state0"), pybind11::arg("controls"), pybind11::arg("target"), pybind11::arg("ckpt_every"),
           pybind11::arg("tick_rate"), pybind11::arg("stream"));
+    m.def("air_ckpt_every", &air_ckpt_every, "Ticks per checkpoint of air_rollout with ckpt_every=None",
+          pybind11::arg("n"), pybind11::arg("ticks"));
+    m.def("shot_ckpt_every", &shot_ckpt_every, "Ticks per checkpoint of shot_rollout with ckpt_every=None",
+          pybind11::arg("n"), pybind11::arg("ticks"));
     m.def("shot_rollout", &shot_rollout,
           "loss, final, flags = shot_rollout(state0, controls, target, ckpt_every, tick_rate, stream)",
           pybind11::arg("state0"), pybind11::arg("controls"), pybind11::arg("target"), pybind11::arg("ckpt_every"),

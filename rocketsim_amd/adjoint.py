@@ -17,7 +17,7 @@ state0.  Without a `ckpt_every`, `air_rollout` and `shot_rollout` keep every
 tick's state, which is the fastest, where all states take up to 512 MB, and
 else one every CKPT_EVERY ticks; name one to bound the memory that a graph
 holds until its backward pass (ceil(ticks / ckpt_every) * n * 52 bytes, for the
-shot 92).
+shot 92).  A call that records no graph keeps none.
 """
 import importlib.util
 import os

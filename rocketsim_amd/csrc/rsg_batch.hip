@@ -164,6 +164,7 @@ struct rsg_batch {
                                         // writes to the device's planes clears it
     rsg_controls* controls = nullptr;   // pinned: the controls set last
     bool controls_pending = false;      // they are newer than the mirror's and the device's
+    bool captured = false;              // a caller's graph holds a step: replays, on any stream, go unseen
     bool synced = false;                // no device work of this batch since the device was waited for
     int arenas_per_block = 0;  // 0: derived from the device's SIMD count
     int kernel = RSG_KERNEL_AUTO;
@@ -202,6 +203,13 @@ void ran_on(rsg_batch* b, hipStream_t s) {
     b->dev_newer = true;
     b->records_fresh = false;
     b->synced = false;
+}
+
+// A step is about to go to `s`: whether into a graph that a caller records.
+void note_capture(rsg_batch* b, hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+    else if (cap != hipStreamCaptureStatusNone) b->captured = true;
 }
 
 void mirror_controls(rsg_batch* b, const rsg_controls* in) {
@@ -334,6 +342,8 @@ int read_records(rsg_batch* b, RecordKind kind, void* out) {
         HIP_OK(hipHostMalloc((void**)&b->records, bytes, hipHostMallocDefault));
         b->records_bytes = bytes;
     }
+    // a replay of the caller's may be under way on a stream that last_stream is not ordered with
+    if (b->captured) HIP_OK(hipDeviceSynchronize());
     auto launch = [&](RecordsOut o) -> int {
         HIP_OK(launch_records_read(b->dev, b->car_at, o, b->last_stream));
         HIP_OK(hipDeviceSynchronize());
@@ -349,7 +359,7 @@ int read_records(rsg_batch* b, RecordKind kind, void* out) {
             o.n_cars = b->total_cars;
             o.n_balls = o.n_pad_arenas = b->dev.n;
             if (launch(o) != 0) return -1;
-            b->records_fresh = true;
+            b->records_fresh = !b->captured;
         }
         std::memcpy(out, b->records + at[kind], one * n);
         return 0;
@@ -742,6 +752,7 @@ int rsg_batch_step(rsg_batch* b, int ticks, void* stream) {
     if (ticks == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     if (upload_for_step(b, s) != 0) return -1;
+    note_capture(b, s);
     if (launch_step(b, b->dev, choose_launch(b), ticks, s) != 0) return -1;
     ran_on(b, s);
     return check_strict(b, "rsg_batch_step");
@@ -862,6 +873,7 @@ int rsg_batch_graph_launch(rsg_batch* b, void* stream) {
     if (!b->graph_exec) return fail("rsg_batch_graph_launch: no graph (call rsg_batch_graph_create)");
     hipStream_t s = (hipStream_t)stream;
     if (upload_for_step(b, s) != 0) return -1;
+    note_capture(b, s);
     HIP_OK(hipGraphLaunch(b->graph_exec, s));
     ran_on(b, s);
     return check_strict(b, "rsg_batch_graph_launch");

@@ -107,3 +107,27 @@ def test_what_was_set_is_read_back_after_uploads_without_a_step(arenas):
     for what, x, y, z in zip(("cars", "balls", "pads"), got, want, before):
         assert x == y, what
         assert x != z, what + " as before the set"
+
+
+@pytest.mark.parametrize("arenas", [3, 1500])
+def test_reads_wait_for_replays_of_a_captured_step(arenas):
+    """A step that the caller records into a graph of its own and replays on
+    another stream: each read gives the state after the replay before it."""
+    torch = pytest.importorskip("torch")
+    a, b = (_batch([2] * arenas, synth_controls=True, auto_reset=True) for _ in range(2))
+    a.step(1)
+    b.step(1)
+    torch.cuda.synchronize()
+    record, replay = torch.cuda.Stream(), torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(record):
+        graph.capture_begin()
+        b.step(100, stream=record.cuda_stream)      # some 10 ms
+        graph.capture_end()
+    for _ in range(3):
+        a.step(100)
+        with torch.cuda.stream(replay):
+            graph.replay()
+        assert _records(b) == _records(a)
+    a.close()
+    b.close()

@@ -2,7 +2,10 @@
 the one over arrays by word with checkpoints: the same bits, at tick counts
 around the group of loads and the checkpoint distance, for one car, a ragged
 wave and several, for inputs that are views at odd offsets or transposed, and
-when the caller's tensors change between forward and backward."""
+when the caller's tensors change between forward and backward.  And the entry
+points by car against those by word at every kind of checkpoint distance (every
+tick kept; segments of one group of loads, ragged and whole), with and without
+the optional outputs."""
 import pytest
 import torch
 
@@ -46,4 +49,41 @@ def test_by_car_equals_by_word(n, ticks):
         for got, w in zip(_grads(air_rollout, make(s0), make(ctrl), make(tgt)), want):
             assert torch.equal(got, w)
     for got, w in zip(_grads(air_rollout, s0.clone(), ctrl.clone(), tgt.clone(), change=True), want):
+        assert torch.equal(got, w)
+
+
+@pytest.mark.parametrize("every", [1, 3, 16, 32])
+@pytest.mark.parametrize("n,ticks", [(1, 1), (65, 31), (130, 32), (64, 33), (257, 96)])
+def test_entry_points_by_car_equal_those_by_word(n, ticks, every):
+    from rocketsim_amd import native
+    L = native.lib()
+    s0, ctrl, tgt = _problem(n, ticks, 7 * n + ticks)
+    by_word = [s0.t().contiguous(), ctrl.permute(0, 2, 1).contiguous(), tgt.t().contiguous()]
+    dl = torch.linspace(-1, 2, n, device="cuda")
+    new = lambda *shape: torch.full(shape, float("nan"), device="cuda")     # noqa: E731
+    words = ((ticks + every - 1) // every) * 13 * n
+    check, p = native.check, lambda x: x.data_ptr()                         # noqa: E731
+
+    final, loss, ckpt, dc, ds = new(13, n), new(n), new(words), new(ticks, 4, n), new(13, n)
+    check(L.rsg_air_rollout(n, ticks, every, 120.0, *map(p, by_word), p(final), p(loss), p(ckpt), None))
+    check(L.rsg_air_rollout_backward(n, ticks, every, 120.0, p(by_word[1]), p(by_word[2]), p(ckpt), p(dl), p(dc), p(ds),
+                                     None))
+    want = [final.t(), loss, ckpt, dc.permute(0, 2, 1), ds.t()]
+
+    final, loss, ckpt, dc, ds = new(n, 13), new(n), new(words), new(ticks, n, 4), new(n, 13)
+    kept, kept_target = new(ticks, n, 4), new(n, 7)
+    check(L.rsg_air_rollout_rows(n, ticks, every, 120.0, p(s0), p(ctrl), p(tgt), p(final), p(loss), p(ckpt), p(kept),
+                                 p(kept_target), None))
+    check(L.rsg_air_rollout_rows_backward(n, ticks, every, 120.0, p(kept), p(kept_target), p(ckpt), p(dl), p(dc), p(ds),
+                                          None))
+    torch.cuda.synchronize()
+    for got, w in zip([final, loss, ckpt, dc, ds, kept, kept_target], want + [ctrl, tgt]):
+        assert torch.equal(got, w)
+    # outputs left out
+    final2, loss2, dc2 = new(n, 13), new(n), new(ticks, n, 4)
+    check(L.rsg_air_rollout_rows(n, ticks, every, 120.0, p(s0), p(ctrl), p(tgt), p(final2), p(loss2), None, None, None,
+                                 None))
+    check(L.rsg_air_rollout_rows_backward(n, ticks, every, 120.0, p(ctrl), p(tgt), p(ckpt), p(dl), p(dc2), None, None))
+    torch.cuda.synchronize()
+    for got, w in ((final2, final), (loss2, loss), (dc2, dc)):
         assert torch.equal(got, w)

@@ -386,8 +386,11 @@ int rsg_ball_pred_get_all(rsg_ball_pred* p, rsg_ball_state* out);
  * prediction is empty. */
 int rsg_ball_pred_state_for_time(rsg_ball_pred* p, int tracker, float pred_time, rsg_ball_state* out);
 
-/* Launch shape of the updates: trackers per 64-lane wave (1..64), or 0 for
- * the default, ceil(n / SIMDs) so that every SIMD holds a wave. */
+/* Launch shape of the updates: trackers per wave (1..64), or 0 for the
+ * default, ceil(n / SIMDs) so that every SIMD holds a wave.  A wave holds as
+ * many as its share of the LDS does, 15, and runs that many where more are
+ * asked for; a tracker gets min(64 / trackers, 16) lanes.  The predictions do
+ * not depend on it. */
 int rsg_ball_pred_set_launch(rsg_ball_pred* p, int trackers_per_wave);
 
 /* Device view of the predictions for consumers on the GPU (no copy). */

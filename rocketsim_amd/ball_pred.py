@@ -72,7 +72,8 @@ class BallPredTracker:
         return out
 
     def set_launch(self, trackers_per_wave):
-        """Trackers per 64-lane wave (0 = one wave per SIMD)."""
+        """Trackers per 64-lane wave, 15 at most whatever is asked for (0 = one
+        wave per SIMD)."""
         native.check(self.L.rsg_ball_pred_set_launch(self.h, trackers_per_wave))
 
     def view(self):

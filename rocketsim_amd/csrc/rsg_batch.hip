@@ -1614,8 +1614,10 @@ int pred_stride() { return (int)((pred_arena_bytes() + team_local_bytes(1) + 15)
 constexpr int PRED_LANES = 16;
 
 // Trackers per wave: as few as give every SIMD one wave, as a wave waits for
-// its slowest tracker (4096 trackers of 720 ticks at 1, 2 and 4 a wave: 23.3,
-// 18.3 and 18.9 ms; the longest chain of contacts alone takes 17).
+// its slowest tracker and more waves than SIMDs wait for each other (4096
+// trackers of 720 ticks at 1, 2 and 4 a wave: 23.3, 18.3 and 18.9 ms, so that
+// the rule's 4 lies 3 % off the best there; the longest chain of contacts alone
+// takes 17).
 int pred_per_wave(int n) {
     int per = (n + device_simds() - 1) / device_simds();
     return per < 1 ? 1 : per;

@@ -1,8 +1,9 @@
 """The ball-prediction kernel's teams (csrc/rsg_k_pred.hip) against a batch of
 arenas without cars stepped one tick at a time by the plain kernel: the same
-bits in every predicted record, whatever the trackers per wave (one lane a
-tracker to a whole wave each), for balls in flight, rolling along curved walls
-and resting, at odd counts, in every mode, fresh and carried on."""
+bits in every predicted record, whatever the trackers per wave (one of 16 lanes
+to fifteen of 4, the most a wave's LDS holds; more are run as fifteen), for balls
+in flight, rolling along curved walls and resting, at odd counts, in every mode,
+fresh and carried on."""
 import ctypes as C
 
 import numpy as np
@@ -52,7 +53,7 @@ def test_predictions_are_the_plain_kernels_ticks(mode):
         want.append(_key(b.get_balls()))
         b.step(1)
     b.close()
-    for per_wave in (0, 1, 3, 16, 64):
+    for per_wave in (0, 1, 3, 5, 7, 12, 15, 64):     # 16, 16, 16, 12, 9, 5, 4 and 4 lanes
         tr = BallPredTracker(mode=mode, n=n, num_pred_ticks=T)
         tr.set_launch(per_wave)
         tr.force_update_all_pred(balls)

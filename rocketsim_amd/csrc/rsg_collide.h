@@ -81,9 +81,9 @@ struct IslandTables {
 };
 
 // What the contact-added callbacks do to the arena (Arena.cpp:244-414),
-// recorded while the pairs' narrowphase runs and applied afterwards in pair
-// order, which is the order the reference's dispatcher meets the contacts
-// in.  The narrowphase reads only poses, shapes and the pre-tick contact
+// by a team of lanes recorded while the pairs' narrowphase runs and applied
+// afterwards in pair order, which is the order the reference's dispatcher meets
+// the contacts in.  The narrowphase reads only poses, shapes and the pre-tick contact
 // response flags, none of which these effects change, so recording them
 // changes no result.
 enum EffectKind { EFF_CAR_WORLD = 1, EFF_BALL_WORLD = 2, EFF_CAR_BALL = 3, EFF_CAR_CAR = 4 };
@@ -98,11 +98,9 @@ constexpr int PAIR_EFFECTS = RSG_TEST_PAIR_EFFECTS;
 constexpr int PAIR_EFFECTS = 4;
 #endif
 struct PairEffects {
-    int n;
-    int redo;  // more effects than fit, or the pair needs the penetration pass: run it again in order
     Effect e[PAIR_EFFECTS];
 };
-// One arena's record of a shared narrowphase, one entry per manifold.
+// One arena's record of a team's narrowphase, one entry per manifold.
 struct PairLog {
     PairEffects eff[MAX_MANIFOLDS];
 };
@@ -132,10 +130,9 @@ static_assert(sizeof(StepSpace) + sizeof(ArenaLocal) <= 62 * 1024, "the plain ke
 #endif
 
 // An arena's block of a batch's global work space: the world step's work
-// space and the record of a shared narrowphase.
+// space, or a team's (rsg_team.h).
 struct ArenaSpace {
     StepSpace step;
-    PairLog log;
 };
 
 // predictUnconstraintMotion (damping on every dynamic body; the ball's linear
@@ -156,16 +153,9 @@ struct World {
 
     WorldTables* T;  // ws->wt
     Manifold* mf;   // ws->mf
-    // Narrowphase of one planned pair: where its callbacks' effects go (null:
-    // applied at once) and the penetration work space (null: a query that
-    // needs it marks the pair for a second, in-order run).
-    PairEffects* rec;
-    EpaSpace* epa;
-    bool aborted;
 
     RSG_FN World(ArenaLocal& a, const ArenaGeom* g, bool s, StepSpace* w = nullptr)
-        : A(a), geo(g), soccar(s), mesh(nullptr), ws(w), T(w ? &w->wt : nullptr), mf(w ? w->mf : nullptr),
-          rec(nullptr), epa(w ? &w->epa : nullptr), aborted(false) {}
+        : A(a), geo(g), soccar(s), mesh(nullptr), ws(w), T(w ? &w->wt : nullptr), mf(w ? w->mf : nullptr) {}
 
     // Whether the subsimplex ray cast against a convex of bounding radius
     // `radius` about `center` can report a hit with fraction below 1: only
@@ -393,42 +383,29 @@ struct World {
 
     // Arena::_BulletContactAddedCallback (src/Sim/Arena/Arena.cpp:244-314):
     // the point's combined material and flags here, the arena's side through
-    // effect().
+    // apply_effect().
     RSG_FN void contact_added(CPoint& cp, int b0, int b1) {
         if (!has_response(b0) || !has_response(b1)) return;
         if (b0 > 0 && b1 < 0) {
             // car + world (Arena.cpp:407-414)
             cp.friction = A.mut.car_world_friction;
             cp.restitution = A.mut.car_world_restitution;
-            effect(EFF_CAR_WORLD, b0 - 1, 0, cp.normal, v3zero());
+            apply_effect(EFF_CAR_WORLD, b0 - 1, 0, cp.normal, v3zero());
         } else if (b0 == 0 && b1 < 0) {
             // ball + world: Ball::_OnWorldCollision, then the averaged
             // "special" row (Arena.cpp:296-304)
-            if (A.mode == RSG_MODE_HEATSEEKER) effect(EFF_BALL_WORLD, 0, 0, cp.normal, v3zero());
+            if (A.mode == RSG_MODE_HEATSEEKER) apply_effect(EFF_BALL_WORLD, 0, 0, cp.normal, v3zero());
             cp.special = true;
         } else if (b0 > 0 && b1 == 0) {
             cp.friction = CARBALL_COLLISION_FRICTION;
             cp.restitution = CARBALL_COLLISION_RESTITUTION;
-            effect(EFF_CAR_BALL, b0 - 1, 0, cp.local_b, v3zero());
+            apply_effect(EFF_CAR_BALL, b0 - 1, 0, cp.local_b, v3zero());
         } else if (b0 > 0 && b1 > 0) {
             cp.friction = CARCAR_COLLISION_FRICTION;
             cp.restitution = CARCAR_COLLISION_RESTITUTION;
-            effect(EFF_CAR_CAR, b0 - 1, b1 - 1, cp.local_a, cp.local_b);
+            apply_effect(EFF_CAR_CAR, b0 - 1, b1 - 1, cp.local_a, cp.local_b);
         }
         if (b1 < 0 && cp.tri >= 0 && static_is_mesh(*geo, -1 - b1)) adjust_internal_edge(cp, geo->meshes[-1 - b1], cp.tri);
-    }
-
-    RSG_FN void effect(int kind, int a, int b, V3 v0, V3 v1) {
-        if (!rec) { apply_effect(kind, a, b, v0, v1); return; }
-        if (kind == EFF_CAR_WORLD && rec->n > 0 && (rec->e[rec->n - 1].code & 0xff) == EFF_CAR_WORLD) {
-            rec->e[rec->n - 1].v0 = v0;  // the flag is set either way; the last normal stays
-            return;
-        }
-        if (rec->n >= PAIR_EFFECTS) { rec->redo = 1; return; }
-        Effect& e = rec->e[rec->n++];
-        e.code = kind | (a << 8) | (b << 16);
-        e.v0 = v0;
-        e.v1 = v1;
     }
 
     RSG_FN void apply_effect(int kind, int a, int b, V3 v0, V3 v1) {
@@ -719,11 +696,10 @@ struct World {
             RSG_FN void operator()(int t) { w->car_triangle(mi, code, t, amin, amax, cx, he); }
         } cb{this, mi, code, amin, amax, cx, he};
         mesh_query_aabb(*mesh, amin, amax, cb);
-        if (!aborted) refresh(mi);
+        refresh(mi);
     }
 
     RSG_FN void car_triangle(int mi, int code, int t, V3 amin, V3 amax, const Xf& cx, V3 he) {
-        if (aborted) return;
         V3 v[3];
         mesh_triangle(*mesh, t, v);
         if (!triangle_aabb_overlap(v, amin, amax)) return;
@@ -746,9 +722,7 @@ struct World {
         md *= md;
         V3 n, pb;
         float dist;
-        int r = gjk_closest(box, tri, cx, xf_ident(), md, n, pb, dist, epa);
-        if (r < 0) aborted = true;
-        else if (r) add_contact(mi, n, pb, dist, t);
+        if (gjk_closest(box, tri, cx, xf_ident(), md, n, pb, dist, &ws->epa)) add_contact(mi, n, pb, dist, t);
     }
 
     // Car hitbox vs the ball: btConvexConvexAlgorithm (GJK) on the box and the
@@ -761,9 +735,8 @@ struct World {
         md *= md;
         V3 n, pb;
         float dist;
-        int r = gjk_closest(box, sph, cx, xf_from(A.ball.b.pos, A.ball.b.rot), md, n, pb, dist, epa);
-        if (r < 0) { aborted = true; return; }
-        if (r) add_contact(mi, n, pb, dist, -1);
+        if (gjk_closest(box, sph, cx, xf_from(A.ball.b.pos, A.ball.b.rot), md, n, pb, dist, &ws->epa))
+            add_contact(mi, n, pb, dist, -1);
         refresh(mi);
     }
 
@@ -828,7 +801,7 @@ struct World {
     RSG_FN void step(float dt) {
         step_begin(dt);
         run_pairs();
-        step_end(dt, nullptr);
+        step_end(dt);
     }
 
     // Gravity, damping, bounds, broadphase and the manifold plan.
@@ -898,15 +871,10 @@ struct World {
         plan_pairs();
     }
 
-    // The narrowphase's recorded effects (when it was shared: `log`),
-    // islands and solver, integration.
-    RSG_FN void step_end(float dt, const PairLog* log) {
-        step_solve(dt, log);
-        for (int i = 0; i < num_bodies(); i++) body_integrate(i, dt);
-    }
-    RSG_FN void step_solve(float dt, const PairLog* log) {
-        if (log) apply_recorded(log);
+    // Islands and solver, integration.
+    RSG_FN void step_end(float dt) {
         solve_islands(dt);
+        for (int i = 0; i < num_bodies(); i++) body_integrate(i, dt);
     }
 
     // integrateTransforms for body i (active bodies only), then
@@ -1022,7 +990,6 @@ struct World {
     RSG_FN void run_pair(int mi) {
         const Pair pr = T->pairs[T->plan[mi]];
         const int a = pr.a, b = pr.b;
-        aborted = false;
         open_manifold(mi, b, a);
         if (a < 0) {
             const int s = -1 - a;
@@ -1042,46 +1009,9 @@ struct World {
         }
     }
 
-    // The narrowphase on one lane, pair by pair, effects applied as they come.
+    // The narrowphase, pair by pair.
     RSG_FN void run_pairs() {
-        rec = nullptr;
-        epa = &ws->epa;
         for (int mi = 0; mi < T->n_mf; mi++) run_pair(mi);
-    }
-
-    // One lane's share of the narrowphase when the lanes of an arena run the
-    // planned pairs side by side: effects recorded in `log`, no penetration
-    // pass (`space` null) or the lane's own.
-    RSG_FN void run_pairs_recorded(int first, int stride, EpaSpace* space, PairLog* log) {
-        epa = space;
-        for (int mi = first; mi < T->n_mf; mi += stride) {
-            PairEffects& pe = log->eff[mi];
-            pe.n = 0;
-            pe.redo = 0;
-            rec = &pe;
-            run_pair(mi);
-            if (aborted) pe.redo = 1;
-        }
-        rec = nullptr;
-        epa = &ws->epa;
-    }
-
-    // The recorded effects in pair order; a pair marked for it runs again,
-    // with its effects applied as they come.
-    RSG_FN void apply_recorded(const PairLog* log) {
-        rec = nullptr;
-        epa = &ws->epa;
-        for (int mi = 0; mi < T->n_mf; mi++) {
-            const PairEffects& pe = log->eff[mi];
-            if (pe.redo) {
-                run_pair(mi);
-                continue;
-            }
-            for (int j = 0; j < pe.n; j++) {
-                const Effect& e = pe.e[j];
-                apply_effect(e.code & 0xff, (e.code >> 8) & 0xff, e.code >> 16, e.v0, e.v1);
-            }
-        }
     }
 
     // -----------------------------------------------------------------------

@@ -784,57 +784,6 @@ RSG_FN void tick_world(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo,
     world.step(P.dt);
 }
 
-// The same world step in three parts for an arena whose lanes share the
-// narrowphase: the first and last on one lane, the pairs on every lane
-// (`lane` of `lanes`, effects recorded in `log`), with the arena unchanged
-// in between.  A pair whose contact needs the penetration pass is run again
-// by the last part, on the arena's own work space.
-RSG_FN void tick_world_begin(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws) {
-    ball_pre_tick(A.ball, P.mode, P.dt);
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr, ws);
-    world.step_begin(P.dt);
-}
-RSG_FN void tick_world_pairs(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws, PairLog* log,
-                             int lane, int lanes) {
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr, ws);
-    world.run_pairs_recorded(lane, lanes, nullptr, log);
-}
-RSG_FN void tick_world_end(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws,
-                           const PairLog* log) {
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr, ws);
-    world.step_end(P.dt, log);
-}
-
-// The begin and end parts in finer pieces, for lanes that share an arena:
-// the per-body work (proxy AABBs, integration) goes one body per lane
-// (`lane` of `lanes`), the rest stays on one lane, with the arena unchanged
-// by other lanes in between.  In order they equal tick_world_begin and
-// tick_world_end.
-RSG_FN void tick_world_prologue(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws) {
-    ball_pre_tick(A.ball, P.mode, P.dt);
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr, ws);
-    world.step_prologue(P.dt);
-}
-RSG_FN void tick_world_aabbs(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws, int lane,
-                             int lanes) {
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr, ws);
-    for (int i = lane; i < world.num_bodies(); i += lanes) world.body_aabb(i, P.dt);
-}
-RSG_FN void tick_world_broadphase(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws) {
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr, ws);
-    world.step_broadphase();
-}
-RSG_FN void tick_world_solve(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws,
-                             const PairLog* log) {
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr, ws);
-    world.step_solve(P.dt, log);
-}
-RSG_FN void tick_world_integrate(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws, int lane,
-                                 int lanes) {
-    World world(A, geo, mode_has_arena(P.mode) && geo != nullptr, ws);
-    for (int i = lane; i < world.num_bodies(); i += lanes) world.body_integrate(i, P.dt);
-}
-
 // The rest of Arena::Step after tick_begin, serially.  `pre` holds every
 // wheel's ray result (car-major, 4 per car) when cast ahead, else null.
 RSG_FN void tick_rest(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, const RayHit* pre, StepSpace* ws) {

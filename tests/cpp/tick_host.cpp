@@ -9,12 +9,8 @@
 //                            it, the GPU's (divide by the length);
 //   RSG_TEST_MAX_MANIFOLDS,  lower contact capacities, so that ordinary play
 //   RSG_TEST_MAX_SOLVER_ROWS reaches the overflow status bits;
-//   RSG_TEST_SPLIT_WORLD=n   the world step as the cooperative kernel runs
-//                            it: its narrowphase shared by n lanes (run here
-//                            one after another, last lane first) with no
-//                            penetration work space, the effects applied in
-//                            pair order afterwards;
-//   RSG_TEST_PAIR_EFFECTS=n  room for n recorded effects per pair.
+//   RSG_TEST_PAIR_EFFECTS=n  room for n recorded effects per pair (team_host.cpp,
+//                            which steps by the cooperative kernel's phases).
 #ifdef RSG_SSE_NORMALIZE
 #include <immintrin.h>
 
@@ -189,32 +185,6 @@ void th_get_status(void* p, uint32_t* out) {
     for (int a = 0; a < h.dev.n; a++) out[a] = arena_ref(h.dev, a).u(AW_STATUS);
 }
 
-#ifdef RSG_TEST_SPLIT_WORLD
-// One tick in the order of rsg_step_arena_coop_kernel's phases, with the
-// world step in its three parts.
-static void tick_split(ArenaLocal& A, const TickParams& P, const ArenaGeom* geo, StepSpace* ws, PairLog* log) {
-    tick_begin(A, P);
-    {
-        World world(A, geo, mode_has_arena(P.mode) && geo != nullptr);
-        for (int oi = 0; oi < A.n_cars; oi++) car_pre_tick(A, P, world, A.order[oi], nullptr);
-    }
-    pads_pre_tick(A, P);
-    tick_world_prologue(A, P, geo, ws);
-    for (int lane = RSG_TEST_SPLIT_WORLD - 1; lane >= 0; lane--)
-        tick_world_aabbs(A, P, geo, ws, lane, RSG_TEST_SPLIT_WORLD);
-    tick_world_broadphase(A, P, geo, ws);
-    for (int lane = RSG_TEST_SPLIT_WORLD - 1; lane >= 0; lane--)
-        tick_world_pairs(A, P, geo, ws, log, lane, RSG_TEST_SPLIT_WORLD);
-    tick_world_solve(A, P, geo, ws, log);
-    for (int lane = RSG_TEST_SPLIT_WORLD - 1; lane >= 0; lane--)
-        tick_world_integrate(A, P, geo, ws, lane, RSG_TEST_SPLIT_WORLD);
-    for (int oi = 0; oi < A.n_cars; oi++) car_post_tick(A, P, A.order[oi]);
-    if (mode_has_arena(P.mode))
-        for (int p = 0; p < PAD_NUM; p++) pad_check_cars(A, p);
-    tick_end(A, P);
-}
-#endif
-
 // ArenaConfig::customBoostPads for every arena (the batch's custom_pads).
 void th_set_custom_pads(void* p, const rsg_boost_pad_config* pads, int n) {
     HostBatch& h = *(HostBatch*)p;
@@ -226,31 +196,13 @@ void th_set_custom_pads(void* p, const rsg_boost_pad_config* pads, int n) {
 // ArenaConfig::noBallRot == false for every arena (the batch's ball_rotation).
 void th_set_ball_rotation(void* p, int on) { ((HostBatch*)p)->dev.ball_rot = on != 0; }
 
-// Steps every arena `ticks` ticks with the plain kernel's code path (or the
-// split world step, RSG_TEST_SPLIT_WORLD).
+// Steps every arena `ticks` ticks with the plain kernel's code path.
 void th_step(void* p, int ticks) {
     HostBatch& h = *(HostBatch*)p;
     const ArenaGeom mv = h.geo.geom();
     auto A = std::make_unique<ArenaLocal>();
     auto ws = std::make_unique<StepSpace>();
-#ifdef RSG_TEST_SPLIT_WORLD
-    auto log = std::make_unique<PairLog>();
-    for (int a = 0; a < h.dev.n; a++) {
-        load_arena(h.dev, a, *A);
-        TickParams P;
-        P.mode = h.dev.mode;
-        P.dt = h.dev.tick_time;
-        P.seed = h.dev.seed;
-        P.arena_id = (uint32_t)a;
-        P.synth_controls = h.dev.synth_controls != 0;
-        P.auto_reset = h.dev.auto_reset != 0;
-        const ArenaGeom* mp = mode_has_arena(h.dev.mode) ? &mv : nullptr;
-        for (int t = 0; t < ticks; t++) tick_split(*A, P, mp, ws.get(), log.get());
-        store_arena(h.dev, a, *A);
-    }
-#else
     for (int a = 0; a < h.dev.n; a++) step_arena(h.dev, mv, a, ticks, *A, ws.get());
-#endif
 }
 
 }  // extern "C"

@@ -131,7 +131,7 @@ def test_undefined_behaviour_sanitizer_on_every_arena_kind(tmp_path, variant):
     so = str(tmp_path / f"tick_host_ub_{variant}.so")
     tick_host.build(so, tick_host.VARIANTS[variant],
                     ["-fsanitize=address,undefined", "-fno-sanitize-recover=all", "-fno-omit-frame-pointer"],
-                    load_it=False)
+                    load_it=False, src=tick_host.source(variant))
     libs = [subprocess.run(["g++", f"-print-file-name={n}"], capture_output=True, text=True).stdout.strip()
             for n in ("libasan.so", "libubsan.so")]
     env = dict(os.environ, LD_PRELOAD=" ".join(libs), ASAN_OPTIONS="detect_leaks=0:abort_on_error=1",

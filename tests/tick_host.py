@@ -13,13 +13,14 @@ from rocketsim_amd.state import (ARENA_MODES, BallState, CarConfig, CarState, Co
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 SRC = os.path.join(HERE, "cpp", "tick_host.cpp")
+TEAM_SRC = os.path.join(HERE, "cpp", "team_host.cpp")   # the same, stepped by a team of lanes
 
 
-def build(out_path, defines=(), extra=(), load_it=True):
+def build(out_path, defines=(), extra=(), load_it=True, src=SRC):
     """Compile the host tick library with the given -D switches (and load it,
     unless load_it is False: a sanitizer build loads only under its runtime)."""
     cmd = ["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", *["-D" + d for d in defines],
-           *extra, "-I" + os.path.join(ROOT, "include"), SRC, "-o", out_path]
+           *extra, "-I" + os.path.join(ROOT, "include"), src, "-o", out_path]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(r.stderr[-4000:])
@@ -28,13 +29,16 @@ def build(out_path, defines=(), extra=(), load_it=True):
 
 _cache = {}
 VARIANTS = {"sse": ["RSG_SSE_NORMALIZE"], "plain": [],
-            # the world step as the cooperative kernel runs it (narrowphase
-            # over 16 lanes, effects applied afterwards in pair order)
-            "sse_split": ["RSG_SSE_NORMALIZE", "RSG_TEST_SPLIT_WORLD=16"],
+            # the tick by the phases that the cooperative kernel's teams run
+            "sse_split": ["RSG_SSE_NORMALIZE"],
             # ... keeping one effect per pair, so pairs with more run again in order
-            "sse_split_1eff": ["RSG_SSE_NORMALIZE", "RSG_TEST_SPLIT_WORLD=16", "RSG_TEST_PAIR_EFFECTS=1"],
+            "sse_split_1eff": ["RSG_SSE_NORMALIZE", "RSG_TEST_PAIR_EFFECTS=1"],
             # contact capacities low enough for ordinary play to reach them
             "small_manifolds": ["RSG_TEST_MAX_MANIFOLDS=1"], "small_rows": ["RSG_TEST_MAX_SOLVER_ROWS=4"]}
+
+
+def source(variant):
+    return TEAM_SRC if variant.startswith("sse_split") else SRC
 
 
 def get(variant):
@@ -42,7 +46,8 @@ def get(variant):
     if variant not in _cache:
         import tempfile
         d = tempfile.mkdtemp(prefix="tick_host_")
-        _cache[variant] = build(os.path.join(d, f"tick_host_{variant}.so"), VARIANTS[variant])
+        _cache[variant] = build(os.path.join(d, f"tick_host_{variant}.so"), VARIANTS[variant],
+                                src=source(variant))
     return _cache[variant]
 
 

@@ -57,7 +57,7 @@ struct TeamManifold {
     uint8_t n;
     uint8_t special;   // ball against the world: solved through the averaged row
     uint8_t n_effects;
-    uint8_t redo;      // run again in order (effects past the record)
+    uint8_t redo;      // run again in order (two cars, effects past the record)
     TeamPoint p[MAX_POINTS_PER_MANIFOLD];
     int eff_code;      // the first effect (kind | car a << 8), unless car-car
     V3 eff_v;
@@ -535,13 +535,19 @@ struct Team {
     }
 
     // A contact callback's effect on the arena: recorded, or applied at once
-    // when the pair runs again in order.
+    // when the pair runs again in order.  Only two cars' pair can have more than
+    // the record holds, and only it may run again: pair() finds all its
+    // contacts, while those of a mesh and of the ball and a car come from the
+    // rounds of search.  (These have one effect a pair at most: a car on the
+    // world keeps its last, a car meets the ball in one point, a plane the ball
+    // in one, and the ball's on a mesh are applied as they come.)
+    static_assert(PAIR_EFFECTS >= 1, "one effect of any pair fits its record");
     RSG_FN void effect(TeamManifold& m, int mi, int& n_eff, bool direct, int kind, int a, int b, V3 v0, V3 v1) {
         const int code = kind | (a << 8) | (b << 16);
         // (the ball's against meshes come first in the pair order and are found in order)
         if (direct || (kind == EFF_BALL_WORLD && mesh_of(mi))) { team_apply_effect(A, code, v0, v1); return; }
         if (kind == EFF_CAR_WORLD && n_eff > 0) { m.eff_v = v0; return; }  // the flag is set either way, the last normal stays
-        if (n_eff >= PAIR_EFFECTS) { m.redo = 1; return; }
+        if (n_eff >= PAIR_EFFECTS) { m.redo = kind == EFF_CAR_CAR; return; }
         if (n_eff == 0 && kind != EFF_CAR_CAR) {
             m.eff_code = code;
             m.eff_v = v0;

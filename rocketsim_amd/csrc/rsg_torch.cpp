@@ -71,25 +71,21 @@ struct AirRolloutFn : public torch::autograd::Function<AirRolloutFn> {
         auto tgt = target.to(torch::kFloat).contiguous();
         const int64_t nseg = (ticks + ckpt_every - 1) / ckpt_every;
         auto opts = s0.options();
+        // the states, and the backward pass's own copies, as the caller may change its tensors
+        torch::Tensor ckpt, kept, kept_target;
+        if (graph) ckpt = torch::empty({nseg * AIR_WORDS * n}, opts);
         auto out = torch::empty({n, 13}, opts);
         auto loss = torch::empty({n}, opts);
-        if (!graph) {
-            check(rsg_air_rollout_rows((int)n, (int)ticks, (int)ckpt_every, (float)tick_rate, s0.data_ptr<float>(),
-                                       ctrl.data_ptr<float>(), tgt.data_ptr<float>(), out.data_ptr<float>(),
-                                       loss.data_ptr<float>(), nullptr, nullptr, nullptr, (void*)stream),
-                  "rsg_air_rollout");
-            ctx->mark_non_differentiable({out});
-            return {loss, out};
+        if (graph) {
+            kept = torch::empty_like(ctrl);
+            kept_target = torch::empty_like(tgt);
         }
-        auto ckpt = torch::empty({nseg * AIR_WORDS * n}, opts);
-        // the backward pass's own copies: the caller may change its tensors
-        auto kept = torch::empty_like(ctrl), kept_target = torch::empty_like(tgt);
+        auto data = [](const torch::Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; };
         check(rsg_air_rollout_rows((int)n, (int)ticks, (int)ckpt_every, (float)tick_rate, s0.data_ptr<float>(),
                                    ctrl.data_ptr<float>(), tgt.data_ptr<float>(), out.data_ptr<float>(),
-                                   loss.data_ptr<float>(), ckpt.data_ptr<float>(), kept.data_ptr<float>(),
-                                   kept_target.data_ptr<float>(), (void*)stream),
+                                   loss.data_ptr<float>(), data(ckpt), data(kept), data(kept_target), (void*)stream),
               "rsg_air_rollout");
-        ctx->save_for_backward({kept, kept_target, ckpt});
+        if (graph) ctx->save_for_backward({kept, kept_target, ckpt});
         ctx->saved_data["n"] = n;
         ctx->saved_data["ticks"] = ticks;
         ctx->saved_data["ckpt_every"] = ckpt_every;

@@ -583,15 +583,15 @@ int rsg_batch_car_offset(const rsg_batch* b, int arena) {
     return b->car_offset[arena];
 }
 
-// Launch geometry.  One lane simulates one arena and the kernel runs at one
-// wave per SIMD (its register and private-memory footprint), so a launch is
-// latency bound: spreading the arenas over every SIMD (partial waves) beats
-// packing 64 lanes into few waves.
+// Launch geometry.  A launch is latency bound, so spreading the arenas over
+// every SIMD (partial waves) beats packing few waves full.
 //
-// Two kernels: the arena's working copy in private scratch, or in LDS.  LDS
-// cuts the latency of every state access but holds only ~40 KB per wave at
-// one wave per SIMD (160 KB per CU), i.e. a few arenas per wave; the LDS
-// kernel is chosen when that still covers the batch in one round of waves.
+// Three kernels: a team of lanes per arena, the arena and its team's tables in
+// LDS (cooperative); one lane per arena with its working copy in LDS; one lane
+// per arena with all of it in private memory (plain).  LDS holds about 40 KB
+// per wave at one wave per SIMD (160 KB per CU), i.e. a few arenas per wave.
+// Where an arena's team does not fit, the LDS kernel is taken when it covers
+// the batch in one round of waves, else the plain one.
 namespace {
 constexpr size_t LDS_PER_WAVE = 40 * 1024;
 
@@ -642,7 +642,8 @@ struct Launch {
 // 1.45), so it is the default; arenas are spread one per workgroup until every
 // SIMD has a wave, then packed up to the most a workgroup holds (2v2 x 16384
 // at 1, 2, 3 and 4 arenas a workgroup: 0.522, 0.410, 0.363 and 0.350; x 4096:
-// 0.223, 0.185, 0.196 and 0.192).
+// 0.223, 0.185, 0.196 and 0.192, so that the rule's 4 lies 4 % off the best
+// there, the price of one wave per SIMD; rsg_batch_autotune takes the best).
 Launch choose_launch(const rsg_batch* b) {
     const int simds = device_simds();
     int spread = (b->dev.n + simds - 1) / simds;  // arenas per wave at one wave per SIMD

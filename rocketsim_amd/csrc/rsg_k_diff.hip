@@ -19,7 +19,9 @@ using namespace rsg;
 // in Bullet units either way.
 //
 // What bounds them: the chain of ticks, 1 us forward and 2 us for the adjoint,
-// at one wave per SIMD; and memory where whole arrays are passed over again.
+// at one wave per SIMD (65536 cars: 309 and 756 VALU instructions a tick, whose
+// issue takes 45 and 72 % of the wave's cycles; it waits 37 and 14 %); and
+// memory where whole arrays are passed over again.
 // By car, controls are read and their gradient written as 16 bytes a lane
 // where the caller has them, with no transposed copies (65536 cars x 120 ticks:
 // 130 us).  With K = 1 the adjoint reads each tick's state, a tick ahead of its
@@ -284,7 +286,8 @@ __global__ void __launch_bounds__(256) rsg_shot_backward_kernel(int n, int ticks
 // pair has a contact, which is some ticks of a shot, 32 lanes take its 26
 // tangents, two pairs at a time.
 //
-// What bounds it: the chain of ticks, 2.5 us each.  One group of lanes a pair
+// What bounds it: the chain of ticks, 2.5 us each (16384 pairs: 78 % of a
+// wave's cycles issue VALU instructions, it waits 14 %).  One group of lanes a pair
 // ran all 26 tangents on every tick: 16384 pairs x 90 ticks 3210 us against 614,
 // 101 x 60 298 against 186.
 __global__ void __launch_bounds__(64) rsg_shot_backward_kept_kernel(int n, int ticks, int per, float dt,
@@ -380,7 +383,7 @@ hipError_t launch_air_backward(bool rows, int n, int ticks, int K, float dt, con
 // Pairs per wave: spread over the SIMDs first, as a wave takes the contact path
 // on every tick on which one of its pairs has a contact (forward, 16384 pairs x
 // 90 ticks: 301 us at 16 a wave against 375 at 64; 101 x 60: 117 at 1 against
-// 291).
+// 291).  (A wave holds any number, so the count of an MI355X serves elsewhere.)
 static int shot_per_wave(int n) {
     constexpr int SIMDS = 1024;
     const int per = (n + SIMDS - 1) / SIMDS;
